@@ -437,22 +437,82 @@ __device__ inline uint64_t argmax_key(int32_t v, uint32_t idx) {
     return ((uint64_t)((uint32_t)v ^ 0x80000000u) << 32) | (uint64_t)(0xFFFFFFFFu - idx);
 }
 
-__global__ __launch_bounds__(kBlock) void argmax_kernel(const int32_t* __restrict__ v, int n, int ldv,
-                                                       int64_t* __restrict__ out) {
-    __shared__ uint64_t red[kBlock];
+// Four consecutive values of a row: rows start at any 4-byte address (odd
+// lengths and strides), which a 16-byte global load accepts.
+typedef int32_t RowQuad __attribute__((ext_vector_type(4), aligned(4)));
+
+// The passes over whole logit rows (argmax, sampling) run one block
+// of 16 waves per row and walk it in segments of kRowSeg values per wave, the
+// block's waves side by side: four 16-byte loads per lane and segment, two
+// segments in flight, 128 KB per block, which is what one CU needs to draw
+// its share of the memory rate with few rows in flight.
+constexpr int kRowThreads = 1024;
+constexpr int kRowWaves = kRowThreads / 64;
+constexpr int kRowSeg = 1024;
+
+// Calls f(i, v) for the values of row[0, n) that fall to this thread, i in
+// ascending order, and seg(s, full) after each of its segments s.
+template <class F, class Seg>
+__device__ inline void row_segments(const int32_t* __restrict__ row, int n, const F& f, const Seg& seg) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nfull = n / kRowSeg;
+    auto load = [&](RowQuad (&v)[4], int s) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            v[q] = *reinterpret_cast<const RowQuad*>(row + (size_t)s * kRowSeg + q * 256 + lane * 4);
+    };
+    auto use = [&](const RowQuad (&v)[4], int s) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f(s * kRowSeg + q * 256 + lane * 4 + e, v[q][e]);
+        seg(s);
+    };
+    int s = w;
+    for (; s + kRowWaves < nfull; s += 2 * kRowWaves) {
+        RowQuad a[4], b[4];
+        load(a, s);
+        load(b, s + kRowWaves);
+        use(a, s);
+        use(b, s + kRowWaves);
+    }
+    if (s < nfull) {
+        RowQuad a[4];
+        load(a, s);
+        use(a, s);
+        s += kRowWaves;
+    }
+    if (s == nfull && s * kRowSeg < n) {  // the partial last segment
+        for (int i = s * kRowSeg + lane; i < n; i += 64) f(i, row[i]);
+        seg(s);
+    }
+}
+
+// Bound by reading the row: 600 x 152064 values in 61 us (6.0 TB/s), 24 in 7.8
+// us; 256 threads with one load in flight each and 64-bit keys throughout took
+// 280 and 73 us.  A thread keeps its first maximum (ascending i, so strictly
+// greater wins); keys order the threads'.
+__global__ __launch_bounds__(kRowThreads) void argmax_kernel(const int32_t* __restrict__ v, int n, int ldv,
+                                                            int64_t* __restrict__ out) {
+    __shared__ uint64_t red[kRowWaves];
     const int32_t* row = v + (size_t)blockIdx.x * ldv;
-    uint64_t best = 0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const uint64_t key = argmax_key(row[i], (uint32_t)i);
-        best = key > best ? key : best;
-    }
-    red[threadIdx.x] = best;
+    int32_t best = INT32_MIN;
+    int at = -1;
+    row_segments(
+        row, n,
+        [&](int i, int32_t x) {
+            const bool up = x > best || at < 0;
+            best = up ? x : best;
+            at = up ? i : at;
+        },
+        [](int) {});
+    const uint64_t key = wave_max_u64(at < 0 ? 0 : argmax_key(best, (uint32_t)at));
+    const int lane = threadIdx.x & 63;
+    if (lane == 0) red[threadIdx.x >> 6] = key;
     __syncthreads();
-    for (int s = blockDim.x >> 1; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) red[threadIdx.x] = red[threadIdx.x] > red[threadIdx.x + s] ? red[threadIdx.x] : red[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[blockIdx.x] = (int64_t)(0xFFFFFFFFu - (uint32_t)(red[0] & 0xFFFFFFFFu));
+    if (threadIdx.x >= 64) return;
+    const uint64_t m = wave_max_u64(lane < kRowWaves ? red[lane] : 0);
+    if (lane == 0) out[blockIdx.x] = (int64_t)(0xFFFFFFFFu - (uint32_t)(m & 0xFFFFFFFFu));
 }
 
 // Integer log-softmax of one row at its target (build-defined, see fixed.h):
@@ -517,7 +577,7 @@ hipError_t logsoftmax(const int32_t* z, int M, int n, int ldz, const int16_t* lu
 }
 
 hipError_t argmax(const int32_t* v, int M, int n, int ldv, int64_t* out, hipStream_t st) {
-    argmax_kernel<<<M, kBlock, 0, st>>>(v, n, ldv, out);
+    argmax_kernel<<<M, kRowThreads, 0, st>>>(v, n, ldv, out);
     return hipGetLastError();
 }
 
@@ -534,10 +594,12 @@ __device__ inline uint64_t splitmix64_next(uint64_t& state) {
     return z ^ (z >> 31);
 }
 
-// n % d by binary long division (no hardware divide); d < 2^63.
+// n % d by binary long division (no hardware divide); 0 < d < 2^63.  The top
+// bits of n that are together below d are the first remainder.
 __device__ inline uint64_t umod64(uint64_t n, uint64_t d) {
-    uint64_t r = 0;
-    for (int i = 63; i >= 0; --i) {
+    const int k = 64 - __builtin_clzll(d) - 1;  // 2^k <= d
+    uint64_t r = k ? n >> (64 - k) : 0;
+    for (int i = 63 - k; i >= 0; --i) {
         r = (r << 1) | ((n >> i) & 1u);
         if (r >= d) r -= d;
     }
@@ -572,36 +634,132 @@ __device__ inline int64_t block_scan_i64(int64_t v, int64_t* wt, int64_t& total)
     return (int64_t)((uint64_t)before + (uint64_t)inc - (uint64_t)v);
 }
 
+// Inclusive prefix sum of one i64 per lane over the wave (wrapping).
+__device__ inline int64_t wave_scan_i64(int64_t v, int lane) {
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t o = shfl_up_i64(v, d);
+        if (lane >= d) v = (int64_t)((uint64_t)v + (uint64_t)o);
+    }
+    return v;
+}
+
 // sample_integer_cdf (sampling.rs:27-46) of row blockIdx.x at state
 // states[row]: weights w_i = z_i - min z + 1 (logits_to_weights,
 // sampling.rs:20-24; i32 arithmetic, wrapping as the reference's release
 // build does), total = sum w_i as i64; total <= 0 gives token 0 and the state
 // unchanged; otherwise (state', r) = splitmix64(state), threshold = r % total
 // and the token is the first i with threshold < w_0 + ... + w_i (the last
-// index when there is none).  The running sums are scanned over tiles of
-// 4 x kSampleThreads positions in order, so the first such i is exact also
-// when wrapped weights make the sums non-monotone.
-constexpr int kSampleThreads = 1024;
-__global__ __launch_bounds__(kSampleThreads) void sample_cdf_kernel(const int32_t* __restrict__ z, int n, int ldz,
-                                                                   const uint64_t* __restrict__ states,
-                                                                   int64_t* __restrict__ tokens,
-                                                                   uint64_t* __restrict__ new_states) {
-    __shared__ int32_t redm[kSampleThreads / 64];
-    __shared__ int32_t redc[kSampleThreads / 64];
-    __shared__ int64_t wt[kSampleThreads / 64];
+// index when there is none).
+//
+// Bound by reading the row, and with few rows by one block's loads in
+// flight, so the row is read once: the pass keeps its minimum, its maximum
+// and the sum of z of every group of 2^lg segments in LDS.  When no
+// weight wraps (max - min + 1 < 2^31, as any logits of a model) the weights
+// are positive, so the group's weight sums follow from those sums and the
+// minimum, the running sum only rises, and the token lies in the first group
+// whose running sum passes the threshold: only that group is read again, by
+// one wave.  Rows with wrapped weights scan every value in order over tiles
+// of 4 x kRowThreads positions, so the first such i is exact also when the
+// running sums are not monotone.  24 x 152064: 17 us; three passes over the
+// row with one load in flight per thread took 130 us.
+constexpr int kSampleGroups = 1024;
+__global__ __launch_bounds__(kRowThreads) void sample_cdf_kernel(const int32_t* __restrict__ z, int n, int ldz, int lg,
+                                                                const uint64_t* __restrict__ states,
+                                                                int64_t* __restrict__ tokens,
+                                                                uint64_t* __restrict__ new_states) {
+    __shared__ int32_t redm[kRowWaves], redx[kRowWaves];
+    __shared__ int32_t redc[kRowWaves];
+    __shared__ int64_t wt[kRowWaves];
     __shared__ int64_t s_thr;
+    __shared__ unsigned long long gsum[kSampleGroups];
     const int32_t* row = z + (size_t)blockIdx.x * ldz;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int gvals = kRowSeg << lg;                                     // values per group
+    const int ngroups = (int)(((int64_t)n + gvals - 1) / kRowSeg >> lg);  // <= kSampleGroups
+    gsum[tid] = 0;
+    __syncthreads();
     // the minimum as ~max(~z) (bitwise not reverses the signed order)
-    int32_t nm = INT32_MIN;
-    for (int i = tid; i < n; i += kSampleThreads) nm = max(nm, ~row[i]);
-    const int32_t m = ~block_max_i32_dpp(nm, redm);
-    auto weight = [&](int32_t zi) -> int64_t { return (int64_t)(int32_t)((uint32_t)zi - (uint32_t)m + 1u); };
+    int32_t nm = INT32_MIN, mx = INT32_MIN;
     int64_t part = 0;
-    for (int i = tid; i < n; i += kSampleThreads) part += weight(row[i]);
+    row_segments(
+        row, n,
+        [&](int, int32_t x) {
+            nm = max(nm, ~x);
+            mx = max(mx, x);
+            part += x;
+        },
+        [&](int s) {
+            const int64_t t = wave_sum_i64(part);
+            if (lane == 0) atomicAdd(&gsum[s >> lg], (unsigned long long)t);
+            part = 0;
+        });
+    const int32_t m = ~block_max_i32_dpp(nm, redm);
+    mx = block_max_i32_dpp(mx, redx);  // its barrier also publishes gsum
+    uint64_t state = states[blockIdx.x];
+    auto weight = [&](int32_t zi) -> int64_t { return (int64_t)(int32_t)((uint32_t)zi - (uint32_t)m + 1u); };
+    if ((int64_t)mx - (int64_t)m + 1 <= (int64_t)INT32_MAX) {
+        if (tid >= 64) return;
+        // lane l: groups [16 l, 16 l + 16), their running weight sums
+        constexpr int kPerLane = kSampleGroups / 64;
+        const int64_t shift = (int64_t)m - 1;  // w = z - shift
+        auto gw = [&](int g) -> int64_t {
+            if (g >= ngroups) return 0;
+            const int64_t len = min((int64_t)gvals, (int64_t)n - (int64_t)g * gvals);
+            return (int64_t)gsum[g] - len * shift;
+        };
+        int64_t mine = 0;
+#pragma unroll
+        for (int j = 0; j < kPerLane; ++j) mine += gw(lane * kPerLane + j);
+        const int64_t inc = wave_scan_i64(mine, lane);
+        const int64_t total = (int64_t)readlane_u64((uint64_t)inc, 63);  // >= n
+        const uint64_t r = splitmix64_next(state);
+        const int64_t thr = (int64_t)umod64(r, (uint64_t)total);  // total < 2^62: n < 2^31 weights below 2^31
+        const uint64_t past = __ballot(thr < inc);                // the last lane's always is
+        const int l0 = (int)__builtin_ctzll(past);
+        int64_t base = (int64_t)readlane_u64((uint64_t)(inc - mine), l0);
+        int g = l0 * kPerLane;
+        for (int j = 0; j + 1 < kPerLane; ++j, ++g) {
+            const int64_t wg = gw(g);
+            if (thr < base + wg) break;
+            base += wg;
+        }
+        int pick = n - 1;
+        const int g0 = g * gvals, g1 = (int)min((int64_t)n, (int64_t)g0 + gvals);
+        for (int i0 = g0; i0 < g1; i0 += 256) {
+            int64_t w[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = i0 + 4 * lane + e;
+                w[e] = i < g1 ? (int64_t)row[i] - shift : 0;
+            }
+            const int64_t loc = w[0] + w[1] + w[2] + w[3];
+            const int64_t sc = wave_scan_i64(loc, lane);
+            const uint64_t hit = __ballot(thr < base + sc);
+            if (hit) {  // uniform
+                const int l = (int)__builtin_ctzll(hit);
+                int64_t acc = base + sc - loc;
+                int at = 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    acc += w[e];
+                    at += thr < acc ? 0 : 1;
+                }
+                pick = i0 + 4 * l + readlane_i32(at, l);
+                break;
+            }
+            base += (int64_t)readlane_u64((uint64_t)sc, 63);
+        }
+        if (lane == 0) {
+            tokens[blockIdx.x] = pick;
+            new_states[blockIdx.x] = state;
+        }
+        return;
+    }
+    part = 0;
+    for (int i = tid; i < n; i += kRowThreads) part += weight(row[i]);
     int64_t total = 0;
     (void)block_scan_i64(part, wt, total);
-    uint64_t state = states[blockIdx.x];
     if (total <= 0) {  // uniform: an empty or non-positive total keeps the state
         if (tid == 0) {
             tokens[blockIdx.x] = 0;
@@ -618,8 +776,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_cdf_kernel(const int32_
     const int64_t thr = s_thr;
     int64_t base = 0;
     int pick = n - 1;
-    for (int t0 = 0; t0 < n; t0 += 4 * kSampleThreads) {
-        const int i0 = t0 + 4 * tid;
+    for (int64_t t0 = 0; t0 < n; t0 += 4 * kRowThreads) {
+        const int64_t i0 = t0 + 4 * tid;
         int64_t w[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[e] = i0 + e < n ? weight(row[i0 + e]) : 0;
@@ -630,7 +788,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_cdf_kernel(const int32_
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             acc += w[e];
-            if (i0 + e < n && thr < acc && cand == INT32_MAX) cand = i0 + e;
+            if (i0 + e < n && thr < acc && cand == INT32_MAX) cand = (int)(i0 + e);
         }
         // the first candidate of the tile: a block minimum as ~max(~x)
         const int first = ~block_max_i32_dpp(~cand, redc);
@@ -645,7 +803,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_cdf_kernel(const int32_
 
 hipError_t sample_cdf(const int32_t* z, int M, int n, int ldz, const uint64_t* states, int64_t* tokens,
                       uint64_t* new_states, hipStream_t st) {
-    sample_cdf_kernel<<<M, kSampleThreads, 0, st>>>(z, n, ldz, states, tokens, new_states);
+    // 2^lg segments per group, so that the row's groups fit the block's LDS sums
+    int lg = 0;
+    while (((int64_t)kSampleGroups * kRowSeg << lg) < n) ++lg;
+    sample_cdf_kernel<<<M, kRowThreads, 0, st>>>(z, n, ldz, lg, states, tokens, new_states);
     return hipGetLastError();
 }
 

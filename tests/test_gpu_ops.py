@@ -454,6 +454,33 @@ def test_sample_dev_rows(backend, oracle):
         assert (int(tok[m]), int(ns[m])) == oracle.sample_integer_cdf(z[m], int(states[m])), m
 
 
+@pytest.mark.parametrize("n", [1, 255, 1023, 1024, 1025, 16384, 16385, 33793, 1 << 20, (1 << 20) + 1, (1 << 21) + 4097])
+def test_row_choice_edges(backend, oracle, n):
+    """argmax and the sampler at the edges of their row walk (1024 values per
+    wave segment, 16 waves, two segments in flight; past 2^20 values the
+    sampler's groups hold several segments), rows at odd addresses and strides:
+    ties across segments, a first and a last token, wrapped weights."""
+    import torch
+    case(f"row choice n={n}")
+    r = rng(n)
+    M, ld = 4, n + 3
+    buf = r.integers(-500, 500, M * ld + 1).astype(np.int32)
+    z = np.lib.stride_tricks.as_strided(buf[1:], (M, n), (4 * ld, 4))
+    z[0, n // 2:] = 499                       # the first of a run of ties
+    z[1, n - 1] = 2**29                       # the last value the maximum, nearly all weight there
+    if n > 1:
+        z[3, 0], z[3, n - 1] = -2**31, 2**31 - 1  # wrapped weights
+    d = torch.from_numpy(buf).cuda()
+    zd = torch.as_strided(d, (M, n), (ld, 1), 1)
+    assert list(backend.argmax_dev(zd).cpu().numpy()) == [oracle.argmax_int(np.ascontiguousarray(v)) for v in z]
+    for state in (0, 7, 2**64 - 3):
+        st = torch.from_numpy(np.full(M, state, np.uint64).view(np.int64)).cuda()
+        tok, ns = (t.cpu().numpy() for t in backend.sample_dev(zd, st))
+        for m in range(M):
+            want = oracle.sample_integer_cdf(np.ascontiguousarray(z[m]), state)
+            assert (int(tok[m]), int(ns.view(np.uint64)[m])) == want, (n, m, state)
+
+
 def test_device_forms_batch_rows(backend, oracle, luts64):
     import torch
     case("rmsnorm/softmax/argmax dev batch")
