@@ -450,42 +450,53 @@ constexpr int kRowThreads = 1024;
 constexpr int kRowWaves = kRowThreads / 64;
 constexpr int kRowSeg = 1024;
 
-// Calls f(i, v) for the values of row[0, n) that fall to this thread, i in
-// ascending order, and seg(s, full) after each of its segments s.
-template <class F, class Seg>
-__device__ inline void row_segments(const int32_t* __restrict__ row, int n, const F& f, const Seg& seg) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+// Calls full(s, v) for each whole segment s of row[0, n) that falls to this
+// wave, in ascending order (v[q][e] is value i = row_index(s, q, e), ascending
+// in q and e), then tail(i0) on the wave whose turn the partial last segment
+// [i0, n) is.
+__device__ inline int row_index(int s, int q, int e) {
+    return s * kRowSeg + q * 256 + (int)(threadIdx.x & 63) * 4 + e;
+}
+template <class Full, class Tail>
+__device__ inline void row_segments(const int32_t* __restrict__ row, int n, const Full& full, const Tail& tail) {
     const int nfull = n / kRowSeg;
     auto load = [&](RowQuad (&v)[4], int s) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-            v[q] = *reinterpret_cast<const RowQuad*>(row + (size_t)s * kRowSeg + q * 256 + lane * 4);
+        for (int q = 0; q < 4; ++q) v[q] = *reinterpret_cast<const RowQuad*>(row + row_index(s, q, 0));
     };
-    auto use = [&](const RowQuad (&v)[4], int s) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) f(s * kRowSeg + q * 256 + lane * 4 + e, v[q][e]);
-        seg(s);
-    };
-    int s = w;
+    int s = threadIdx.x >> 6;
     for (; s + kRowWaves < nfull; s += 2 * kRowWaves) {
         RowQuad a[4], b[4];
         load(a, s);
         load(b, s + kRowWaves);
-        use(a, s);
-        use(b, s + kRowWaves);
+        full(s, a);
+        full(s + kRowWaves, b);
     }
     if (s < nfull) {
         RowQuad a[4];
         load(a, s);
-        use(a, s);
+        full(s, a);
         s += kRowWaves;
     }
-    if (s == nfull && s * kRowSeg < n) {  // the partial last segment
-        for (int i = s * kRowSeg + lane; i < n; i += 64) f(i, row[i]);
-        seg(s);
-    }
+    if (s == nfull && s * kRowSeg < n) tail(s * kRowSeg);
+}
+
+// The same with f(i, v) for every value and seg(s) after each segment.
+template <class F, class Seg>
+__device__ inline void row_values(const int32_t* __restrict__ row, int n, const F& f, const Seg& seg) {
+    row_segments(
+        row, n,
+        [&](int s, const RowQuad (&v)[4]) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f(row_index(s, q, e), v[q][e]);
+            seg(s);
+        },
+        [&](int i0) {
+            for (int i = i0 + (int)(threadIdx.x & 63); i < n; i += 64) f(i, row[i]);
+            seg(i0 / kRowSeg);
+        });
 }
 
 // Bound by reading the row: 600 x 152064 values in 61 us (6.0 TB/s), 24 in 7.8
@@ -498,7 +509,7 @@ __global__ __launch_bounds__(kRowThreads) void argmax_kernel(const int32_t* __re
     const int32_t* row = v + (size_t)blockIdx.x * ldv;
     int32_t best = INT32_MIN;
     int at = -1;
-    row_segments(
+    row_values(
         row, n,
         [&](int i, int32_t x) {
             const bool up = x > best || at < 0;
@@ -519,49 +530,110 @@ __global__ __launch_bounds__(kRowThreads) void argmax_kernel(const int32_t* __re
 //   m = max z;  S = sum_j lut[(m - z_j) << 2] (0 past the table; logits are
 //   Q6 and the exp LUT's input is Q8);  lp = (z_target - m) * 2^10 - ln_q16(S)
 // in Q16.  One block per row; targets < 0 give 0.
-constexpr int kLogsoftmaxLds = 4096;  // exp-table entries a block copies to LDS (8 KB)
-__global__ __launch_bounds__(kBlock) void logsoftmax_kernel(const int32_t* __restrict__ z, int n, int ldz,
-                                                           const int16_t* __restrict__ lut, uint32_t lut_len,
-                                                           const int64_t* __restrict__ targets,
-                                                           int64_t* __restrict__ out) {
-    __shared__ int32_t red32[kBlock / 64];
-    __shared__ uint64_t red64[kBlock / 64];
-    __shared__ int16_t elut[kLogsoftmaxLds];
+//
+// Bound by reading the row, and S needs the maximum first, which read it
+// twice.  The logits are whole numbers, so one pass counts them instead: a
+// ring of kLogBins LDS counters indexed by z mod kLogBins (an LDS add where the
+// second pass had an LDS table lookup), with the maximum and the least value
+// counted.  Values kLogBins (128 logit units) or more below the largest of
+// 1024 sampled ones are past the table whatever the maximum is and are not
+// counted (masked tokens, say), and a segment of equal values is one add.
+// When the counted values lie less than kLogBins apart every counter stands
+// for one value and S = sum over k of count[m - k] * lut[k << 2]; other rows,
+// and tables longer than the ring, sum the table over a second pass.
+// 600 x 152064 values in 80 us (4.6 TB/s); two passes of 256 threads took 385.
+// Constant rows, rows wider than the ring and half-masked rows take 76, 150 and
+// 83 us (186, 200 and 293 before).
+constexpr int kLogBins = 8192;
+__global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* __restrict__ z, int n, int ldz,
+                                                                const int16_t* __restrict__ lut, uint32_t lut_len,
+                                                                const int64_t* __restrict__ targets,
+                                                                int64_t* __restrict__ out) {
+    __shared__ int32_t reds[kRowWaves], redm[kRowWaves], redx[kRowWaves];
+    __shared__ int64_t red64[kRowWaves];
+    __shared__ uint32_t count[kLogBins];
     const int32_t* row = z + (size_t)blockIdx.x * ldz;
-    // the table's first entries in LDS (the exp table is zero past a short
-    // prefix, so nearly every lookup is served there); the rest from memory
-    const int nl = (int)min(lut_len, (uint32_t)kLogsoftmaxLds);
-    for (int i = threadIdx.x; i < nl; i += kBlock) elut[i] = lut[i];
-    // 16-byte loads over the aligned part of the row, four in flight per thread
-    const int n4 = ((uintptr_t)row & 15) == 0 ? n >> 2 : 0;
-    const int4* row4 = reinterpret_cast<const int4*>(row);
-    int32_t mx = INT32_MIN;
-#pragma unroll 4
-    for (int i = threadIdx.x; i < n4; i += kBlock) {
-        const int4 v = row4[i];
-        mx = max(mx, max(max(v.x, v.y), max(v.z, v.w)));
-    }
-    for (int i = 4 * n4 + threadIdx.x; i < n; i += kBlock) mx = max(mx, row[i]);
-    const int32_t m = block_max_i32(mx, red32);  // its barrier also publishes elut
+    const int tid = threadIdx.x;
+    for (int i = tid; i < kLogBins; i += kRowThreads) count[i] = 0;
+    static_assert(kRowThreads == 1024, "one sample per thread");
+    const int32_t top = block_max_i32_dpp(row[((int64_t)tid * n) >> 10], reds);  // its barrier also clears the counts
+    const int32_t least = (int32_t)max((int64_t)top - (kLogBins - 1), (int64_t)INT32_MIN);
+    int32_t nm = INT32_MIN, mx = INT32_MIN;
+    row_segments(
+        row, n,
+        [&](int, const RowQuad (&v)[4]) {
+            int32_t smin = v[0][0], smax = v[0][0];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    smin = min(smin, v[q][e]);
+                    smax = max(smax, v[q][e]);
+                }
+            mx = max(mx, smax);
+            const int32_t first = __builtin_amdgcn_readfirstlane(smin);
+            if (__all(smin == first && smax == first)) {
+                if (first < least) return;
+                nm = max(nm, ~first);
+                if ((tid & 63) == 0) atomicAdd(&count[(uint32_t)first % kLogBins], (uint32_t)kRowSeg);
+                return;
+            }
+            if (__all(smin >= least)) {
+                nm = max(nm, ~smin);
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) atomicAdd(&count[(uint32_t)v[q][e] % kLogBins], 1u);
+                return;
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (v[q][e] >= least) {
+                        nm = max(nm, ~v[q][e]);  // the minimum as ~max(~z)
+                        atomicAdd(&count[(uint32_t)v[q][e] % kLogBins], 1u);
+                    }
+        },
+        [&](int i0) {
+            for (int i = i0 + (tid & 63); i < n; i += 64) {
+                const int32_t x = row[i];
+                mx = max(mx, x);
+                if (x < least) continue;
+                nm = max(nm, ~x);
+                atomicAdd(&count[(uint32_t)x % kLogBins], 1u);
+            }
+        });
+    const int32_t lo = ~block_max_i32_dpp(nm, redm);
+    const int32_t m = block_max_i32_dpp(mx, redx);  // the barriers also publish the counts
     constexpr uint32_t sh = MYL_TV_EXP_INPUT_FRAC - MYL_TV_LOGIT_FRAC_BITS;
-    auto term = [&](int32_t zi) -> int64_t {
-        const uint64_t d = (uint64_t)((int64_t)m - (int64_t)zi) << sh;
-        if (d < (uint64_t)nl) return (int64_t)elut[d];
+    auto term = [&](uint64_t below) -> int64_t {
+        const uint64_t d = below << sh;
         return d < lut_len ? (int64_t)lut[d] : 0;
     };
     int64_t s = 0;
-#pragma unroll 4
-    for (int i = threadIdx.x; i < n4; i += kBlock) {
-        const int4 v = row4[i];
-        s += term(v.x) + term(v.y) + term(v.z) + term(v.w);
+    if ((int64_t)m - (int64_t)lo < kLogBins && lut_len <= ((uint32_t)kLogBins << sh)) {
+        for (uint32_t k = tid; k < (uint32_t)kLogBins && ((uint64_t)k << sh) < lut_len; k += kRowThreads)
+            s += (int64_t)count[((uint32_t)m - k) % kLogBins] * term(k);
+    } else {
+        // the table's every fourth entry in the counters' place
+        int16_t* tab = reinterpret_cast<int16_t*>(count);
+        for (uint32_t k = tid; k < (uint32_t)kLogBins; k += kRowThreads) tab[k] = (int16_t)term(k);
+        __syncthreads();
+        row_values(
+            row, n,
+            [&](int, int32_t x) {
+                const uint64_t below = (uint64_t)((int64_t)m - (int64_t)x);
+                s += below < (uint64_t)kLogBins ? (int64_t)tab[below] : term(below);
+            },
+            [](int) {});
     }
-    for (int i = 4 * n4 + threadIdx.x; i < n; i += kBlock) s += term(row[i]);
     s = wave_sum_i64(s);
-    if ((threadIdx.x & 63) == 0) red64[threadIdx.x >> 6] = (uint64_t)s;
+    if ((tid & 63) == 0) red64[tid >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int64_t S = 0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) S += (int64_t)red64[w];
+    if (tid >= 64) return;
+    const int64_t S = wave_sum_i64(tid < kRowWaves ? red64[tid] : 0);
+    if (tid == 0) {
         const int64_t t = targets[blockIdx.x];
         int64_t lp = 0;
         if (t >= 0 && t < n)
@@ -572,7 +644,7 @@ __global__ __launch_bounds__(kBlock) void logsoftmax_kernel(const int32_t* __res
 
 hipError_t logsoftmax(const int32_t* z, int M, int n, int ldz, const int16_t* lut, int lut_len, const int64_t* targets,
                       int64_t* out, hipStream_t st) {
-    logsoftmax_kernel<<<M, kBlock, 0, st>>>(z, n, ldz, lut, (uint32_t)lut_len, targets, out);
+    logsoftmax_kernel<<<M, kRowThreads, 0, st>>>(z, n, ldz, lut, (uint32_t)lut_len, targets, out);
     return hipGetLastError();
 }
 
@@ -682,7 +754,7 @@ __global__ __launch_bounds__(kRowThreads) void sample_cdf_kernel(const int32_t* 
     // the minimum as ~max(~z) (bitwise not reverses the signed order)
     int32_t nm = INT32_MIN, mx = INT32_MIN;
     int64_t part = 0;
-    row_segments(
+    row_values(
         row, n,
         [&](int, int32_t x) {
             nm = max(nm, ~x);

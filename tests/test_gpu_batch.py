@@ -370,6 +370,38 @@ def test_logsoftmax_dev(backend, oracle):
         assert np.array_equal(got, exp)
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1025, 16385, 40003])
+@pytest.mark.parametrize("spread", [0, 700, 8191, 8192, 2**31])
+def test_logsoftmax_row_spreads(backend, oracle, n, spread):
+    """The counted pass (maximum - minimum below 8192) up to its edge and the
+    second pass beyond it, at the edges of the row walk, rows at odd addresses;
+    the 16385-entry table, a short one, one with negative entries and one
+    longer than the counters."""
+    import torch
+    from myelith_amd.luts import exp_lut
+    case(f"logsoftmax n={n} spread={spread}")
+    r = np.random.default_rng(n + spread % 1000)
+    M, ld = 3, n + 1
+    buf = np.zeros(M * ld + 1, np.int32)
+    z = np.lib.stride_tricks.as_strided(buf[1:], (M, n), (4 * ld, 4))
+    lo, hi = -(spread // 2), min(spread - spread // 2, 2**31 - 1)
+    v = r.integers(lo, hi, (M, n), endpoint=True)
+    v[:, r.integers(n)] = hi
+    if n > 1:
+        v[:, n - 1] = lo
+    v[1] += 2**31 - 1 - v[1].max()      # up to the largest value (spread 2^31: already there)
+    if spread < 2**31:
+        v[2] -= v[2].min() + 2**31      # down to the smallest
+    z[:] = np.maximum(v, -2**31)
+    zd = torch.as_strided(torch.from_numpy(buf).cuda(), (M, n), (ld, 1), 1)
+    t = np.array([0, n - 1, n // 2], np.int64)
+    for lut in (exp_lut(), exp_lut()[:1001], r.integers(-300, 300, 16385).astype(np.int16),
+                r.integers(-300, 300, 40001).astype(np.int16)):
+        got = backend.logsoftmax_dev(zd, lut, t).cpu().numpy()
+        exp = np.array([oracle.logsoftmax_at(np.ascontiguousarray(z[i]), lut, int(t[i])) for i in range(M)], np.int64)
+        assert np.array_equal(got, exp)
+
+
 def test_qwen7b_teacher_forced_rows(backend):
     """Qwen2.5-7B architecture at full size (int16 LM head on the matrix
     cores): two sequences x 20 teacher-forced positions in one 40-row batch;
