@@ -804,7 +804,7 @@ hipError_t forward_rows(myl_model* m, BatchState* b, int R, int lmax, int h0, in
         }
         EpiResidRows eo{};
         eo.shifts = Ld.so; eo.act_frac = f.attn_out_frac; eo.acc_frac = Ld.acc_attn; eo.res_frac = Ld.res_in;
-        eo.out_frac = Ld.res_mid; eo.res = b->X; eo.ldr = H; eo.out = b->X2; eo.ldo = H;
+        eo.out_frac = Ld.res_mid; eo.res = b->X; eo.out = b->X2; eo.ldo = H;
         if (norm_in_finish)
             e = resid_then_norm(mm->planes, R, Ld.wo, H, nq, eo, mm, Ld.res_mid, Ld.ref_mid, Ld.post_gamma,
                                 Ld.post_gamma_s, m, f.norm_mlp_frac, fuse_silu ? xin : mm->planes, st);
@@ -839,7 +839,7 @@ hipError_t forward_rows(myl_model* m, BatchState* b, int R, int lmax, int h0, in
         if ((e = hipGetLastError()) != hipSuccess) return e;
         EpiResidRows ed{};
         ed.shifts = Ld.sd; ed.act_frac = f.down_in_frac; ed.acc_frac = Ld.acc_mlp; ed.res_frac = Ld.res_mid;
-        ed.out_frac = Ld.res_out; ed.res = b->X2; ed.ldr = H; ed.out = b->X; ed.ldo = H;
+        ed.out_frac = Ld.res_out; ed.res = b->X2; ed.out = b->X; ed.ldo = H;
         in_normed = norm_in_finish && l + 1 < (int)m->spec.layers;
         if (in_normed) {
             const LayerDev& Ln = m->layers[l + 1];

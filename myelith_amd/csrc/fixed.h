@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #define MYL_FN __host__ __device__ static inline
+#define MYL_MEM __host__ __device__ inline
 
 typedef __int128 myl_i128;
 typedef unsigned __int128 myl_u128;
@@ -73,6 +74,75 @@ MYL_FN int64_t rescale64(int64_t acc, uint8_t in_frac, uint8_t out_frac) {
     int8_t sh = (int8_t)(uint8_t)((int8_t)in_frac - (int8_t)out_frac);
     return sh >= 0 ? rshift_round64(acc, (uint8_t)sh) : shl64(acc, (uint8_t)(-(int32_t)sh));
 }
+
+// ---- requantization of a byte-plane sum in 32-bit steps ----------------------
+//
+// A byte-plane product yields 256 hi + low with low = lo' + 128 rs (fixed
+// activations x = 256 hi + lo' + 128).  For K < 2^16, |hi| <= 2^14 K and
+// |low| <= 2^15 K are 32-bit, so the sum is u * 256 + r with u = hi + (low >> 8)
+// (|u| < 2^30 + 2^23) and 0 <= r < 256: a rounding shift by s >= 9 is one of u
+// by t = s - 8 with r as the sticky bits, and the half-even carry is
+// min(bit t of u | r, 1).  Columns whose shift is outside the range take the
+// 64-bit forms (fast = 0).
+struct PlaneRescale {
+    uint32_t t, fast;
+    int32_t base;
+    MYL_FN PlaneRescale of(uint8_t in_frac, uint8_t out_frac) {
+        const int8_t sh = (int8_t)(uint8_t)((int8_t)in_frac - (int8_t)out_frac);
+        const bool ok = sh >= 9 && sh <= 38;
+        const uint32_t t = ok ? (uint32_t)sh - 8u : 1u;
+        return PlaneRescale{t, ok ? 1u : 0u, (int32_t)((1u << (t - 1)) - 1u)};
+    }
+    // rescale64(256 u + r, in_frac, out_frac)
+    MYL_MEM int32_t operator()(int32_t u, uint32_t r) const {
+        const uint32_t c = (((uint32_t)u >> t) & 1u) | r;
+        return (u + base + (int32_t)(c < 1u ? c : 1u)) >> t;
+    }
+};
+
+// rshift_round128((256 u + r) * mult, shift) for shifts 39..70: the product is
+// 256 V + (r mult & 255) with V = u mult + (r mult >> 8), |V| < 2^62, and the
+// result fits 32 bits.
+struct PlaneMult {
+    int32_t mult;
+    uint32_t t, fast;
+    int64_t base;
+    MYL_FN PlaneMult of(int32_t mult, uint8_t shift) {
+        const bool ok = shift >= 39 && shift <= 70;
+        const uint32_t t = ok ? (uint32_t)shift - 8u : 31u;
+        return PlaneMult{mult, t, ok ? 1u : 0u, (int64_t)((1ull << (t - 1)) - 1u)};
+    }
+    MYL_MEM int32_t operator()(int32_t u, uint32_t r) const {
+        const int64_t rm = (int64_t)(int32_t)r * mult;
+        const int64_t v = (int64_t)u * mult + (int64_t)(int32_t)(rm >> 8);
+        const uint32_t c = ((uint32_t)(v >> t) & 1u) | ((uint32_t)rm & 255u);
+        return (int32_t)((v + base + (int64_t)(c < 1u ? c : 1u)) >> t);
+    }
+};
+
+// rescale64 of a value |v| < 2^30 followed by a clamp to [-2^16, 2^16] or
+// narrower, for left shifts of up to 14 and right shifts of up to 30.
+struct SmallRescale {
+    uint32_t s, ls, fast;
+    int32_t base;
+    MYL_FN SmallRescale of(uint8_t in_frac, uint8_t out_frac) {
+        const int8_t sh = (int8_t)(uint8_t)((int8_t)in_frac - (int8_t)out_frac);
+        const bool ok = sh >= -14 && sh <= 30;
+        const uint32_t s = ok && sh > 0 ? (uint32_t)sh : 0u;
+        return SmallRescale{s, ok && sh < 0 ? (uint32_t)-sh : 0u, ok ? 1u : 0u, s ? (int32_t)((1u << (s - 1)) - 1u) : 0};
+    }
+    // of an int16 (exact: at most 29 bits)
+    MYL_MEM int32_t of16(int32_t v) const { return round(v << ls); }
+    // clamp_i16 of the rescaled value
+    MYL_MEM int16_t clamped(int32_t v) const {
+        v = ls ? (v < -65536 ? -65536 : (v > 65536 ? 65536 : v)) : v;
+        return clamp_i16(round((int32_t)((uint32_t)v << ls)));
+    }
+    MYL_MEM int32_t round(int32_t v) const {
+        const uint32_t q = ((uint32_t)v >> s) & (s ? 1u : 0u);
+        return (v + base + (int32_t)q) >> s;
+    }
+};
 
 // floor(2^32 / d) for d >= 1 (2^33 - 1 for d = 0), by restoring long
 // division (integer only).  The dividend 2^32 has its only set bit at

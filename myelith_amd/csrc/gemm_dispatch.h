@@ -111,7 +111,7 @@ inline int mm_group() {
 // Whether 256 x 256 tiles with 128-byte K stages fill the chip well enough
 // (mm_planes).
 inline bool mm_wide_tiles(int M, int N, int K, int cus) {
-    return K % 128 == 0 && mm2_tiles<2, 2, 4, 4, 2, 128>(M, N) >= cus + cus / 2;
+    return K % 128 == 0 && mm2_tiles<4, 2, 2, 4, 2, 128>(M, N) >= cus + cus / 2;
 }
 
 // The product on planes Ap [2M x K] (mm_planes_ok): few rows stream the
@@ -143,7 +143,7 @@ inline hipError_t mm_planes(const int8_t* Ap, int M, const int8_t* W, int N, int
     if (M <= 32 && K % 128 == 0) return mm2_launch_splitk<2, 1, 1, 4, 2, 128>(Ap, M, W, N, K, epi, mm, 2 * cus, st);
     if (M <= 32) return mm2_launch_splitk<2, 1, 1, 4, 4>(Ap, M, W, N, K, epi, mm, cus, st);
     if (M <= 64 && K % 128 == 0) return mm2_launch_splitk<1, 1, 4, 2, 3, 128>(Ap, M, W, N, K, epi, mm, cus, st);
-    if (M > 64 && mm_wide_tiles(M, N, K, cus)) return mm2_launch<2, 2, 4, 4, 2, 128>(Ap, M, W, N, K, epi, st, mm_group());
+    if (M > 64 && mm_wide_tiles(M, N, K, cus)) return mm2_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, mm_group());
     if (M > 64 && mm2_tiles<2, 2, 4, 2, 3>(M, N) >= cus) return mm2_launch<2, 2, 4, 2, 3>(Ap, M, W, N, K, epi, st);
     return mm2_launch_splitk<2, 1, 2, 4, 4>(Ap, M, W, N, K, epi, mm, cus / 2, st);
 }
@@ -184,7 +184,7 @@ inline hipError_t mm_planes_staged(const int8_t* Ap, int M, const int8_t* W, int
     if (M <= 16) return mm2_staged_launch<1, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 32) return mm2_staged_launch<2, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 64) return mm2_staged_launch<2, 1, 2, 2, 4, 128>(Ap, M, W, N, K, epi, st);
-    if (mm_wide_tiles(M, N, K, mm->cus)) return mm2_staged_launch<2, 2, 4, 4, 2, 128>(Ap, M, W, N, K, epi, st, mm_group());
+    if (mm_wide_tiles(M, N, K, mm->cus)) return mm2_staged_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, mm_group());
     return mm2_staged_launch<2, 2, 4, 2, 3, 64>(Ap, M, W, N, K, epi, st);
 }
 

@@ -387,12 +387,26 @@ template <class Epi>
 struct SinkEpi {
     const Epi& e;
     __device__ inline void operator()(int n, int m, int64_t v) const { e.one(n, m, v); }
+    using Col = typename Epi::Col;
+    using Elt = typename Epi::Elt;
+    __device__ inline Col col(int n) const { return e.col(n); }
+    __device__ inline Elt elt(size_t i, uint32_t lo) const { return e.elt(i, lo); }
+    __device__ inline size_t idx(int n, int m) const { return e.idx(n, m); }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt& x) const { e.put(i, lo, u, r, c, x); }
 };
 struct SinkAtomic {
     unsigned long long* acc;
     int ldn;
     __device__ inline void operator()(int n, int m, int64_t v) const {
         atomicAdd(acc + (size_t)m * ldn + n, (unsigned long long)v);
+    }
+    struct Col { uint32_t fast; };
+    struct Elt {};
+    __device__ inline Col col(int) const { return Col{1}; }
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldn + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col&, const Elt&) const {
+        atomicAdd(acc + i + lo, (unsigned long long)(256 * (int64_t)u + r));
     }
 };
 
@@ -466,6 +480,12 @@ struct SinkGrouped {
     const EpiG& epi;
     int e, row0;
     __device__ inline void operator()(int n, int m, int64_t v) const { epi.one(e, n, row0 + m, v); }
+    using Col = typename EpiG::Col;
+    using Elt = EpiNoElt;
+    __device__ inline Col col(int n) const { return epi.col(e, n); }
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return epi.idx(n, row0 + m); }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const { epi.put(i, lo, u, r, c); }
 };
 
 template <int WM, int WN, int WAVES_M, int WAVES_N, class EpiG>

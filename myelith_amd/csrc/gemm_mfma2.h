@@ -49,7 +49,11 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const int16_t* __rest
     *reinterpret_cast<uint2*>(Ap + (size_t)(2 * m + 1) * K + c * 8) = l;
 }
 
-__device__ inline constexpr int waitcnt_vm(int v) { return (v & 0xF) | (0x7 << 4) | (0xF << 8) | (((v >> 4) & 0x3) << 14); }
+// The wave's loads but the last N and its LDS reads done, then the block barrier.
+template <int N>
+__device__ inline void mm2_stage_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
 
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS = 64>
 struct Mm2 : Mm2Dims<MB, NB, WM_, WN_, STAGES, KS> {
@@ -89,11 +93,18 @@ struct TileOrder {
 // The pipelined main loop: acc[i][j] = A' tile i x W tile j over K in
 // [kb, ke) (multiples of KS); rs[j] = the lane's weight-row sum (summed over
 // the lane pair l, l + 32 only after the loop).
+// The fragments of the next 32 bytes of K are read from LDS while the current
+// ones multiply (two register sets).  The switch to the next stage falls
+// between the halves of a stage's last 32 bytes: by then the wave has read all
+// of its current stage, so one barrier both publishes the next stage and
+// frees the current buffer, and the second half of the multiplies covers the
+// barrier and the first reads.
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS = 64>
 __device__ inline void mm2_main(const int8_t* __restrict__ Ap, int R2, const int8_t* __restrict__ W, int N, int K,
                                 int kb, int ke, int r0, int n0, int8_t* lds, v16i32_t (&acc)[MB][NB],
                                 int32_t (&rs)[NB]) {
     using S = Mm2<MB, NB, WM_, WN_, STAGES, KS>;
+    constexpr int SUB = KS / 32, L = S::kLoads;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave % WM_, wn = wave / WM_;
@@ -101,68 +112,148 @@ __device__ inline void mm2_main(const int8_t* __restrict__ Ap, int R2, const int
     // Each wave-level load moves 1 KiB (64 lanes x 16 bytes) of 1024/KS rows:
     // lane l takes row l / (KS/16) of the group and the global chunk whose
     // swizzled slot is l % (KS/16) (the swizzle is its own inverse).
-    auto issue = [&](int kt, int buf) {
-        int8_t* st = lds + buf * S::kStageBytes;
+    auto group = [&](int i) { return min(wave + i * (S::kThreads / 64), S::kGroups - 1); };
+    const int8_t* src[L];
 #pragma unroll
-        for (int i = 0; i < S::kLoadsMax; ++i) {
-            const int grp = wave + i * (S::kThreads / 64);   // 1 KiB row-group index in the stage
-            if (i >= S::kLoadsMin && grp >= S::kGroups) break;  // wave-uniform
-            const int row = grp * S::kRowsPerLoad + lane / S::kCpr;  // stage row: A' rows first
-            const int chunk = S::slot(row, lane & (S::kCpr - 1));
-            const int8_t* src;
-            if (row < S::BR) {
-                const int gr = min(r0 + row, R2 - 1);
-                src = Ap + (size_t)gr * K + kb + kt * KS + chunk * 16;
-            } else {
-                const int gn = min(n0 + row - S::BR, N - 1);
-                src = W + (size_t)gn * K + kb + kt * KS + chunk * 16;
-            }
-            __builtin_amdgcn_global_load_lds((const void*)src, (lds_void*)(st + grp * 1024), 16, 0, 0);
+    for (int i = 0; i < L; ++i) {
+        const int row = group(i) * S::kRowsPerLoad + lane / S::kCpr;  // A' rows first
+        const int chunk = S::slot(row, lane & (S::kCpr - 1));
+        const int8_t* p = row < S::BR ? Ap + (size_t)min(r0 + row, R2 - 1) * K : W + (size_t)min(n0 + row - S::BR, N - 1) * K;
+        src[i] = p + kb + chunk * 16;
+    }
+    auto issue = [&](int kt) {
+        int8_t* st = lds + (kt % STAGES) * S::kStageBytes;
+#pragma unroll
+        for (int i = 0; i < L; ++i)
+            __builtin_amdgcn_global_load_lds((const void*)(src[i] + (size_t)kt * KS),
+                                             (lds_void*)(st + group(i) * 1024), 16, 0, 0);
+    };
+    // A wave's fragments of 32 bytes of K: 16 bytes per lane, rows 32 apart
+    // share a swizzle slot.
+    int ao[SUB], bo[SUB];
+#pragma unroll
+    for (int s = 0; s < SUB; ++s) {
+        const int chunk = 2 * s + (lane >> 5);
+        const int ra = wm * MB * 32 + (lane & 31), rb = S::BR + wn * NB * 32 + (lane & 31);
+        ao[s] = ra * KS + (S::slot(ra, chunk) << 4);
+        bo[s] = rb * KS + (S::slot(rb, chunk) << 4);
+    }
+    v4i32_t a[2][MB], b[2][NB];
+    auto read = [&](int kt, int s, v4i32_t (&fa)[MB], v4i32_t (&fb)[NB]) {
+        const int8_t* st = lds + (kt % STAGES) * S::kStageBytes;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) fb[j] = *reinterpret_cast<const v4i32_t*>(st + bo[s] + j * 32 * KS);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fa[i] = *reinterpret_cast<const v4i32_t*>(st + ao[s] + i * 32 * KS);
+    };
+    auto mul = [&](const v4i32_t (&fa)[MB], const v4i32_t (&fb)[NB], int j0, int j1) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            if (j < j0 || j >= j1) continue;
+#pragma unroll
+            for (int i = 0; i < MB; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) rs[j] = sdot4((uint32_t)fb[j][q], 0x01010101u, rs[j]);
         }
     };
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int j = 0; j < NB; ++j) {
+        rs[j] = 0;
 #pragma unroll
-        for (int j = 0; j < NB; ++j)
+        for (int i = 0; i < MB; ++i)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+    }
+    // Loads retire in order, so with n later stages in flight a stage has
+    // landed when at most n L loads of the wave are outstanding.  lgkmcnt(0):
+    // the wave's reads of the buffer that the barrier frees are done.
 #pragma unroll
-    for (int j = 0; j < NB; ++j) rs[j] = 0;
-
-#pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
-        if (s < nk) issue(s, s);
+    for (int s = 0; s < STAGES; ++s)
+        if (s < nk) issue(s);
+    if (nk >= STAGES) mm2_stage_barrier<L*(STAGES - 1)>();
+    else mm2_stage_barrier<0>();
+    read(0, 0, a[0], b[0]);
     for (int kt = 0; kt < nk; ++kt) {
-        // stage kt complete: later stages may still be in flight (loads
-        // retire in order; a wave with kLoadsMax loads per stage waits for
-        // a few of the next stage's too)
-        if (kt + STAGES - 2 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_vm(S::kLoadsMin * (STAGES - 2)));
-        else __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-        __syncthreads();
-        if (kt + STAGES - 1 < nk) issue(kt + STAGES - 1, (kt + STAGES - 1) % STAGES);
-        const int8_t* st = lds + (kt % STAGES) * S::kStageBytes;
 #pragma unroll
-        for (int s = 0; s < KS / 32; ++s) {
-            const int chunk = 2 * s + (lane >> 5);
-            v4i32_t a[MB], b[NB];
+        for (int s = 0; s < SUB - 1; ++s) {
+            read(kt, s + 1, a[(s + 1) & 1], b[(s + 1) & 1]);
+            mul(a[s & 1], b[s & 1], 0, NB);
+        }
+        constexpr int cur = (SUB - 1) & 1, nxt = cur ^ 1;
+        mul(a[cur], b[cur], 0, NB / 2);
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + 1 < nk) {
+            if (kt + STAGES - 1 < nk) mm2_stage_barrier<L*(STAGES - 2)>();
+            else mm2_stage_barrier<0>();
+            if (kt + STAGES < nk) issue(kt + STAGES);
+            read(kt + 1, 0, a[nxt], b[nxt]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        mul(a[cur], b[cur], NB / 2, NB);
+    }
+}
+
+// Accumulator register r (even: the hi row of a token, r + 1 its lo' row) of a
+// 32-row tile holds A' row mm2_row(r) + 4 (lane / 32) of the tile.
+__device__ inline constexpr int mm2_row(int r) { return 8 * (r >> 2) + (r & 3); }
+
+// 32-bit sums u * 256 + r need K < 2^16 (fixed.h, PlaneRescale).
+constexpr int kPlaneSumK = 65536;
+
+// One wave's part of a tile's epilogue.  Column operands are resolved once and
+// an accumulator tile's element operands are all loaded before its first
+// store: the stores may alias them, so loads left in the per-value code would
+// wait out the memory latency once per value, and did: with 64-bit (multiplier:
+// 128-bit) arithmetic under a branch per value the epilogue took 0.7 of the
+// main loop's time (multiplier requant, 4001 x 18944 x 3584: 954 us of which
+// 570 the loop).
+template <int MB, int NB, bool FULL, class Sink>
+__device__ inline void mm2_emit(const v16i32_t (&acc)[MB][NB], const int32_t (&rs)[NB], int R2, int N, int arow0,
+                                int nw0, int lane, const Sink& sink) {
+    // an element's place is a uniform offset plus the lane's own (32 bits)
+    const int n_l = lane & 31, m_l = 2 * (lane >> 5), m0 = arow0 >> 1;
+    uint32_t lo = (uint32_t)(sink.idx(n_l, m_l) - sink.idx(0, 0));
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
-                const int row = S::BR + (wn * NB + j) * 32 + (lane & 31);
-                b[j] = *reinterpret_cast<const v4i32_t*>(st + row * KS + (S::slot(row, chunk) << 4));
+    for (int j = 0; j < NB; ++j) {
+        const int nj = nw0 + j * 32, n = nj + n_l;
+        asm("" : "+v"(lo));  // no per-lane addresses kept from one j for the next: they cost two registers each
+        const typename Sink::Col col = sink.col(FULL ? n : min(n, N - 1));
+        const int32_t rs128 = (int32_t)((uint32_t)rs[j] << 7);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+            const int mi = m0 + i * 16;
+            typename Sink::Elt elt[8];
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const int d = mm2_row(r) >> 1;
+                if (FULL || (2 * (mi + d + m_l) < R2 && n < N)) elt[r >> 1] = sink.elt(sink.idx(nj, mi + d), lo);
             }
 #pragma unroll
-            for (int i = 0; i < MB; ++i) {
-                const int row = (wm * MB + i) * 32 + (lane & 31);
-                a[i] = *reinterpret_cast<const v4i32_t*>(st + row * KS + (S::slot(row, chunk) << 4));
+            for (int r = 0; r < 16; r += 2) {
+                const int d = mm2_row(r) >> 1;
+                if (!FULL && (2 * (mi + d + m_l) >= R2 || n >= N)) continue;
+                const int32_t low = acc[i][j][r + 1] + rs128;
+                sink.put(sink.idx(nj, mi + d), lo, acc[i][j][r] + (low >> 8), (uint32_t)low & 255u, col, elt[r >> 1]);
             }
+        }
+    }
+}
+
+// The same from 64-bit sums (a column's shift or K outside the 32-bit range),
+// one register pair at a time.
+template <int MB, int NB, class Sink>
+__device__ inline void mm2_emit64(const v16i32_t (&acc)[MB][NB], const int32_t (&rs)[NB], int R2, int N, int arow0,
+                                  int nw0, int lane, const Sink& sink) {
 #pragma unroll
-            for (int j = 0; j < NB; ++j) {
+    for (int j = 0; j < NB; ++j) {
+        const int n = nw0 + j * 32 + (lane & 31);
 #pragma unroll
-                for (int i = 0; i < MB; ++i) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a[i], b[j], acc[i][j], 0, 0, 0);
-                rs[j] = sdot4((uint32_t)b[j][0], 0x01010101u, rs[j]);
-                rs[j] = sdot4((uint32_t)b[j][1], 0x01010101u, rs[j]);
-                rs[j] = sdot4((uint32_t)b[j][2], 0x01010101u, rs[j]);
-                rs[j] = sdot4((uint32_t)b[j][3], 0x01010101u, rs[j]);
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll 1
+            for (int r = 0; r < 16; r += 2) {
+                const int64_t v = (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128;
+                const int m = ((arow0 + i * 32 + mm2_row(r)) >> 1) + 2 * (lane >> 5);
+                if (2 * m < R2 && n < N) sink(n, m, v);
             }
         }
     }
@@ -178,27 +269,21 @@ __device__ inline void mm2_tile(const int8_t* __restrict__ Ap, int R2, const int
     v16i32_t acc[MB][NB];
     int32_t rs[NB];
     mm2_main<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, kb, ke, r0, n0, lds, acc, rs);
+    const int arow0 = r0 + wm * MB * 32, nw0 = n0 + wn * NB * 32;
+    if (arow0 >= R2 || nw0 >= N) return;
+    bool fast = ke - kb < kPlaneSumK;
 #pragma unroll
-    for (int j = 0; j < NB; ++j) rs[j] += __shfl_xor(rs[j], 32);
-    // accumulator rows 8*(r/4) + 4*(lane/32) + r%4: registers (r, r+1), r even,
-    // hold the hi and lo' rows of one token.
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int n = n0 + (wn * NB + j) * 32 + (lane & 31);
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const int arow = r0 + (wm * MB + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const int m = arow >> 1;
-                if (arow < R2 && n < N)
-                    sink(n, m, (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128);
-            }
-        }
+    for (int j = 0; j < NB; ++j) {
+        rs[j] += __shfl_xor(rs[j], 32);
+        fast = fast && __all((int)sink.col(min(nw0 + j * 32 + (lane & 31), N - 1)).fast);
+    }
+    if (!fast) mm2_emit64<MB, NB>(acc, rs, R2, N, arow0, nw0, lane, sink);
+    else if (arow0 + MB * 32 <= R2 && nw0 + NB * 32 <= N) mm2_emit<MB, NB, true>(acc, rs, R2, N, arow0, nw0, lane, sink);
+    else mm2_emit<MB, NB, false>(acc, rs, R2, N, arow0, nw0, lane, sink);
 }
 
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Epi>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_kernel(const int8_t* __restrict__ Ap, int R2, const int8_t* __restrict__ W,
+__global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, KS>::kMinWaves)) void mm2_kernel(const int8_t* __restrict__ Ap, int R2, const int8_t* __restrict__ W,
                                                              int N, int K, TileOrder ord, int ntiles, Epi epi) {
     using S = Mm2<MB, NB, WM_, WN_, STAGES, KS>;
     extern __shared__ __align__(16) int8_t lds[];
@@ -209,50 +294,51 @@ __global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_kernel(const int8_t* __res
     mm2_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, 0, K, (int)tr * S::BR, (int)tn * S::BN, lds, SinkEpi<Epi>{epi});
 }
 
-// As mm2_kernel, with a staged epilogue for products whose output columns
-// pair up (2i, 2i+1 -> element i of an output row): every accumulator value
-// is first reduced to an int16 by Epi::stage(n, sum) and parked in LDS as a
-// [BR/2 x BN] tile (the K stages are free by then); the block then hands
-// Epi::emit(m, i0, v) the 16 staged values of columns 2 i0 .. 2 i0 + 15 of
-// row m, for 8-column chunks of N / 2 (N % 16 == 0), so the outputs leave in
-// whole 8-byte pieces.
-template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Epi>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_staged_kernel(const int8_t* __restrict__ Ap, int R2,
-                                                                    const int8_t* __restrict__ W, int N, int K,
-                                                                    TileOrder ord, int ntiles, Epi epi) {
+// A tile with a staged epilogue, for products whose output columns pair up
+// (2i, 2i+1 -> element i of an output row): every sum is first reduced to an
+// int16 by sink.stage and parked in LDS as a [BR/2 x BN] tile (the K
+// stages are free by then); the block then hands sink.emit(m, i0, v) the 16
+// staged values of columns 2 i0 .. 2 i0 + 15 of row m, for 8-column chunks of
+// N / 2 (N % 16 == 0), so the outputs leave in whole 8-byte pieces.
+template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Sink>
+__device__ inline void mm2_staged_tile(const int8_t* __restrict__ Ap, int R2, const int8_t* __restrict__ W, int N, int K,
+                                       int r0, int n0, int8_t* lds, const Sink& sink) {
     using S = Mm2<MB, NB, WM_, WN_, STAGES, KS>;
     static_assert((size_t)(S::BR / 2) * S::BN * 2 <= S::kLds, "staged tile fits the stage buffers");
-    extern __shared__ __align__(16) int8_t lds[];
-    const int t = mm_tile_index(ntiles);
-    if (t < 0) return;
-    uint32_t tn, tr;
-    if (!ord.decode((uint32_t)t, tn, tr)) return;
-    const int r0 = (int)tr * S::BR, n0 = (int)tn * S::BN;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave % WM_, wn = wave / WM_;
     v16i32_t acc[MB][NB];
     int32_t rs[NB];
     mm2_main<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, 0, K, r0, n0, lds, acc, rs);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) rs[j] += __shfl_xor(rs[j], 32);
     __syncthreads();  // every wave is past its last stage read
     int16_t* tile = reinterpret_cast<int16_t*>(lds);  // [BR / 2][BN]
+    // rows and columns past the matrix hold sums of clamped operands; they are
+    // staged like the others and never emitted
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int j = 0; j < NB; ++j) {
+        rs[j] += __shfl_xor(rs[j], 32);
+        const int nl = (wn * NB + j) * 32 + (lane & 31), n = min(n0 + nl, N - 1);
+        const typename Sink::Col col = sink.col(n);
+        const bool fast = K < kPlaneSumK && __all((int)col.fast);
+        const int32_t rs128 = (int32_t)((uint32_t)rs[j] << 7);
+        int16_t* tj = tile + (wm * MB * 16 + 2 * (lane >> 5)) * S::BN + nl;
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int nl = (wn * NB + j) * 32 + (lane & 31);
-            const int n = n0 + nl;
+        for (int i = 0; i < MB; ++i) {
+            if (fast) {
 #pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const int arl = (wm * MB + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                int16_t v = 0;
-                if (r0 + arl < R2 && n < N)
-                    v = epi.stage(n, (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128);
-                tile[(arl >> 1) * S::BN + nl] = v;
+                for (int r = 0; r < 16; r += 2) {
+                    const int32_t low = acc[i][j][r + 1] + rs128;
+                    tj[((i * 32 + mm2_row(r)) >> 1) * S::BN] = sink.stage(col, acc[i][j][r] + (low >> 8), (uint32_t)low & 255u);
+                }
+            } else {
+#pragma unroll 1
+                for (int r = 0; r < 16; r += 2)
+                    tj[((i * 32 + mm2_row(r)) >> 1) * S::BN] =
+                        sink.stage64(n, (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128);
             }
         }
+    }
     __syncthreads();
     constexpr int kChunks = S::BN / 16;  // 8-column output chunks per tile row
     const int m0 = r0 >> 1, i00 = n0 >> 1;
@@ -261,8 +347,21 @@ __global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_staged_kernel(const int8_t
         const int m = m0 + ml, i0 = i00 + ic * 8;
         if (2 * m >= R2 || 2 * i0 >= N) continue;
         const uint4* src = reinterpret_cast<const uint4*>(tile + ml * S::BN + ic * 16);
-        epi.emit(m, i0, src[0], src[1]);
+        sink.emit(m, i0, src[0], src[1]);
     }
+}
+
+template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Epi>
+__global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, KS>::kMinWaves)) void mm2_staged_kernel(const int8_t* __restrict__ Ap, int R2,
+                                                                    const int8_t* __restrict__ W, int N, int K,
+                                                                    TileOrder ord, int ntiles, Epi epi) {
+    using S = Mm2<MB, NB, WM_, WN_, STAGES, KS>;
+    extern __shared__ __align__(16) int8_t lds[];
+    const int t = mm_tile_index(ntiles);
+    if (t < 0) return;
+    uint32_t tn, tr;
+    if (!ord.decode((uint32_t)t, tn, tr)) return;
+    mm2_staged_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, (int)tr * S::BR, (int)tn * S::BN, lds, epi);
 }
 
 // group: row tiles per group of the tile order (TileOrder; 0: the plain order).
@@ -288,39 +387,45 @@ hipError_t mm2_staged_launch(const int8_t* Ap, int M, const int8_t* W, int N, in
 // 2m+1 sit in registers r, r+1 of one lane and columns 2n, 2n+1 in lanes
 // l, l^1, so a DPP swap of lane pairs assembles
 //   x.w = 65536*hh + 256*(h lo' + lo' h) + lo' lo' + 128*(xsum + wsum) - 16384*K.
-template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Sink>
+template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Epi>
 __device__ inline void mm2w16_tile(const int8_t* __restrict__ Ap, int R2, const int8_t* __restrict__ Wp, int N2,
                                    int K, const int32_t* __restrict__ xsum, const int32_t* __restrict__ wsum, int r0,
-                                   int n0, int8_t* lds, const Sink& sink) {
+                                   int n0, int8_t* lds, const Epi& epi) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave % WM_, wn = wave / WM_;
     v16i32_t acc[MB][NB];
     int32_t rs[NB];
     mm2_main<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, Wp, N2, K, 0, K, r0, n0, lds, acc, rs);
-    const int64_t kterm = 16384 * (int64_t)K;
     const bool even = (lane & 1) == 0;
 #pragma unroll
-    for (int i = 0; i < MB; ++i)
+    for (int j = 0; j < NB; ++j) {
+        const int np = n0 + (wn * NB + j) * 32 + (lane & 31);
+        const int n = np >> 1;
+        const int nc = min(n, (N2 >> 1) - 1);
+        const typename Epi::Ops o = epi.ops(nc);
+        const int64_t nterm = 128 * (int64_t)wsum[nc] - 16384 * (int64_t)K;
 #pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int np = n0 + (wn * NB + j) * 32 + (lane & 31);
-            const int n = np >> 1;
+        for (int i = 0; i < MB; ++i) {
+            const int arow0 = r0 + (wm * MB + i) * 32 + 4 * (lane >> 5);
+            int32_t xs[8];  // ahead of the stores, as in mm2_emit
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) xs[r >> 1] = xsum[min(arow0 + mm2_row(r), R2 - 2) >> 1];
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
                 const int32_t a0 = acc[i][j][r], a1 = acc[i][j][r + 1];
                 const int32_t b0 = dpp_mov<dpp::kXor1>(a0), b1 = dpp_mov<dpp::kXor1>(a1);
-                const int arow = r0 + (wm * MB + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                const int m = arow >> 1;
+                const int arow = arow0 + mm2_row(r);
                 if (even && arow < R2 && np < N2)
-                    sink(n, m, 65536 * (int64_t)a0 + 256 * ((int64_t)a1 + (int64_t)b0) + (int64_t)b1 +
-                                   128 * ((int64_t)xsum[m] + (int64_t)wsum[n]) - kterm);
+                    epi.one_ops(n, arow >> 1, 65536 * (int64_t)a0 + 256 * ((int64_t)a1 + (int64_t)b0) + (int64_t)b1 +
+                                                  128 * (int64_t)xs[r >> 1] + nterm, o);
             }
         }
+    }
 }
 
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Epi>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void mm2w16_kernel(const int8_t* __restrict__ Ap, int R2,
+__global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, KS>::kMinWaves)) void mm2w16_kernel(const int8_t* __restrict__ Ap, int R2,
                                                                 const int8_t* __restrict__ Wp, int N2, int K,
                                                                 const int32_t* __restrict__ xsum,
                                                                 const int32_t* __restrict__ wsum, TileOrder ord,
@@ -332,7 +437,7 @@ __global__ __launch_bounds__(WM_ * WN_ * 64) void mm2w16_kernel(const int8_t* __
     uint32_t tn, tr;
     if (!ord.decode((uint32_t)t, tn, tr)) return;
     mm2w16_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, Wp, N2, K, xsum, wsum, (int)tr * S::BR, (int)tn * S::BN, lds,
-                                          SinkEpi<Epi>{epi});
+                                          epi);
 }
 
 // x int16 [M x K] -> planes as split_planes_kernel, plus xsum[m] = sum_k x[m][k].
@@ -395,10 +500,10 @@ hipError_t mm2w16_launch(const int8_t* Ap, const int32_t* xsum, int M, const int
     if (M <= 32) return mm2w16_launch_cfg<2, 1, 1, 4, 4, 64>(Ap, xsum, M, Wp, wsum, N, K, epi, st);
     if (M <= 64 && K % 128 == 0) return mm2w16_launch_cfg<2, 1, 2, 2, 3, 128>(Ap, xsum, M, Wp, wsum, N, K, epi, st);
     if (M <= 64) return mm2w16_launch_cfg<2, 1, 2, 4, 4, 64>(Ap, xsum, M, Wp, wsum, N, K, epi, st);
-    using W = Mm2<2, 2, 4, 4, 2, 128>;
+    using W = Mm2<4, 2, 2, 4, 2, 128>;
     const int wide_tiles = ((2 * M + W::BR - 1) / W::BR) * ((2 * N + W::BN - 1) / W::BN);
     if (K % 128 == 0 && wide_tiles >= 4 * cus)
-        return mm2w16_launch_cfg<2, 2, 4, 4, 2, 128>(Ap, xsum, M, Wp, wsum, N, K, epi, st);
+        return mm2w16_launch_cfg<4, 2, 2, 4, 2, 128>(Ap, xsum, M, Wp, wsum, N, K, epi, st);
     return mm2w16_launch_cfg<2, 2, 4, 2, 3, 64>(Ap, xsum, M, Wp, wsum, N, K, epi, st);
 }
 
@@ -406,7 +511,7 @@ hipError_t mm2w16_launch(const int8_t* Ap, const int32_t* xsum, int M, const int
 // partial sums of each slice are added into acc [M x N] (i64, zero-kept; the
 // finish kernel applies the epilogue and clears it).
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS = 64>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_splitk_kernel(const int8_t* __restrict__ Ap, int R2,
+__global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, KS>::kMinWaves)) void mm2_splitk_kernel(const int8_t* __restrict__ Ap, int R2,
                                                                     const int8_t* __restrict__ W, int N, int K,
                                                                     Divider tiles_r, Divider ntiles, int nitems,
                                                                     int kslice, unsigned long long* __restrict__ acc) {
@@ -442,7 +547,7 @@ __device__ inline int mm_dyn_tile_index(const int* __restrict__ nwork) {
 // *nwork on the device (the work table is built there); the grid covers
 // maxwork items.  K % KS == 0.
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class EpiG>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_grouped_kernel(const int8_t* __restrict__ Ap,
+__global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, KS>::kMinWaves)) void mm2_grouped_kernel(const int8_t* __restrict__ Ap,
                                                                      const int8_t* __restrict__ W, size_t w_stride,
                                                                      int N, int K, const int* __restrict__ offsets,
                                                                      const MmWork* __restrict__ work,
@@ -457,61 +562,32 @@ __global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_grouped_kernel(const int8_
                                            2 * wk.m0, wk.n0, lds, SinkGrouped<EpiG>{epi, wk.e, row0});
 }
 
-// mm2_grouped_kernel with the staged epilogue of mm2_staged_kernel: every
-// sum is reduced by EpiG::stage(e, n, sum) to an int16 parked in LDS, then
-// EpiG::emit(e, row, i0, v) takes the 16 values of columns 2 i0 .. 2 i0 + 15
-// of activation row `row` (Ap's token order) for 8-column chunks of N / 2
-// (N % 16 == 0).
+// mm2_grouped_kernel with the staged epilogue (mm2_staged_tile): the sums of
+// expert e reduce by EpiG::stage, and EpiG::emit takes the
+// staged values with the activation row in Ap's token order.
+template <class EpiG>
+struct SinkGroupedStaged {
+    const EpiG& epi;
+    int e, row0;
+    using Col = typename EpiG::Col;
+    __device__ inline Col col(int n) const { return epi.col(e, n); }
+    __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return epi.stage(c, u, r); }
+    __device__ inline int16_t stage64(int n, int64_t v) const { return epi.stage64(e, n, v); }
+    __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b) const { epi.emit(e, row0 + m, i0, a, b); }
+};
+
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class EpiG>
-__global__ __launch_bounds__(WM_ * WN_ * 64) void mm2_grouped_staged_kernel(
+__global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, KS>::kMinWaves)) void mm2_grouped_staged_kernel(
     const int8_t* __restrict__ Ap, const int8_t* __restrict__ W, size_t w_stride, int N, int K,
     const int* __restrict__ offsets, const MmWork* __restrict__ work, const int* __restrict__ nwork, EpiG epi) {
-    using S = Mm2<MB, NB, WM_, WN_, STAGES, KS>;
-    static_assert((size_t)(S::BR / 2) * S::BN * 2 <= S::kLds, "staged tile fits the stage buffers");
     extern __shared__ __align__(16) int8_t lds[];
     const int t = mm_dyn_tile_index(nwork);
     if (t < 0) return;
     const MmWork wk = work[t];
     const int row0 = offsets[wk.e];
-    const int R2 = 2 * (offsets[wk.e + 1] - row0);
-    const int r0 = 2 * wk.m0, n0 = wk.n0;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wm = wave % WM_, wn = wave / WM_;
-    v16i32_t acc[MB][NB];
-    int32_t rs[NB];
-    mm2_main<MB, NB, WM_, WN_, STAGES, KS>(Ap + (size_t)row0 * 2 * K, R2, W + (size_t)wk.e * w_stride, N, K, 0, K, r0,
-                                           n0, lds, acc, rs);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) rs[j] += __shfl_xor(rs[j], 32);
-    __syncthreads();  // every wave is past its last stage read
-    int16_t* tile = reinterpret_cast<int16_t*>(lds);  // [BR / 2][BN]
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j) {
-            const int nl = (wn * NB + j) * 32 + (lane & 31);
-            const int n = n0 + nl;
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-                const int arl = (wm * MB + i) * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                int16_t v = 0;
-                if (r0 + arl < R2 && n < N)
-                    v = epi.stage(wk.e, n,
-                                  (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128);
-                tile[(arl >> 1) * S::BN + nl] = v;
-            }
-        }
-    __syncthreads();
-    constexpr int kChunks = S::BN / 16;  // 8-column output chunks per tile row
-    const int m0 = r0 >> 1, i00 = n0 >> 1;
-    for (int c = threadIdx.x; c < (S::BR / 2) * kChunks; c += S::kThreads) {
-        const int ml = c / kChunks, ic = c % kChunks;  // powers of two
-        const int m = m0 + ml, i0 = i00 + ic * 8;
-        if (2 * m >= R2 || 2 * i0 >= N) continue;
-        const uint4* src = reinterpret_cast<const uint4*>(tile + ml * S::BN + ic * 16);
-        epi.emit(wk.e, row0 + m, i0, src[0], src[1]);
-    }
+    mm2_staged_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap + (size_t)row0 * 2 * K, 2 * (offsets[wk.e + 1] - row0),
+                                                  W + (size_t)wk.e * w_stride, N, K, 2 * wk.m0, wk.n0, lds,
+                                                  SinkGroupedStaged<EpiG>{epi, wk.e, row0});
 }
 
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class EpiG>

@@ -315,6 +315,16 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const int16_t* __rest
 // ---- standard epilogues ------------------------------------------------------
 
 // linear.rs:61-68 / :110-117: clamp_i16(rescale_i64(acc, w_shift + act_frac, out_frac)).
+// The byte-plane products (gemm_mfma2.h) hand an epilogue whole columns:
+//   Col; col(n)        the column's operands, loaded and resolved once;
+//                      Col::fast: the 32-bit form below is exact for it
+//   idx(n, m)          an element's place, linear in n and m; elt and put take
+//                      it as a uniform part and the lane's own
+//   Elt; elt(i, lo)    operands of one element, loaded ahead of any store
+//   put(i, lo, u, r, col, elt)   from the sum 256 u + r (fixed.h,
+//                      PlaneRescale); columns that are not fast take one()
+struct EpiNoElt {};
+
 struct EpiShift {
     const uint8_t* w_shifts;
     const uint8_t* out_frac_pc;  // per channel (linear_w8a16_pc) or null
@@ -330,6 +340,17 @@ struct EpiShift {
         out[(size_t)m * ldo + r] = clamp_i16_i64(rescale64(acc, (uint8_t)(o.ws + act_frac), o.of));
     }
     __device__ inline void one(int r, int m, int64_t acc) const { one_ops(r, m, acc, ops(r)); }
+    using Col = PlaneRescale;
+    __device__ inline Col col(int n) const {
+        const Ops o = ops(n);
+        return Col::of((uint8_t)(o.ws + act_frac), o.of);
+    }
+    using Elt = EpiNoElt;
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const {
+        (out + i)[lo] = clamp_i16(c(u, r));
+    }
     template <int R, int MT>
     __device__ inline void apply(int row0, int N, int M, int lane, const int64_t (&tot)[R][MT]) const {
 #pragma unroll
@@ -357,6 +378,14 @@ struct EpiMult {
         out[(size_t)m * ldo + r] = y < -32768 ? (int16_t)-32768 : (y > 32767 ? (int16_t)32767 : (int16_t)y);
     }
     __device__ inline void one(int r, int m, int64_t acc) const { one_ops(r, m, acc, ops(r)); }
+    using Col = PlaneMult;
+    __device__ inline Col col(int n) const { return Col::of(mult[n], shift[n]); }
+    using Elt = EpiNoElt;
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const {
+        (out + i)[lo] = clamp_i16(c(u, r));
+    }
     template <int R, int MT>
     __device__ inline void apply(int row0, int N, int M, int lane, const int64_t (&tot)[R][MT]) const {
 #pragma unroll
@@ -373,9 +402,20 @@ struct EpiLogits {
     uint8_t norm_frac, logit_frac;
     int32_t* out; int ldo;
     EpiLogits offset_m(int m0) const { EpiLogits e = *this; e.out += (size_t)m0 * ldo; return e; }
-    __device__ inline void one(int r, int m, int64_t acc) const {
-        out[(size_t)m * ldo + r] = clamp_i32_i64(rescale64(acc, (uint8_t)(row_shifts[r] + norm_frac), logit_frac));
+    struct Ops {
+        uint8_t sh;
+    };
+    __device__ inline Ops ops(int r) const { return Ops{row_shifts[r]}; }
+    __device__ inline void one_ops(int r, int m, int64_t acc, const Ops& o) const {
+        out[(size_t)m * ldo + r] = clamp_i32_i64(rescale64(acc, (uint8_t)(o.sh + norm_frac), logit_frac));
     }
+    __device__ inline void one(int r, int m, int64_t acc) const { one_ops(r, m, acc, ops(r)); }
+    using Col = PlaneRescale;
+    __device__ inline Col col(int n) const { return Col::of((uint8_t)(row_shifts[n] + norm_frac), logit_frac); }
+    using Elt = EpiNoElt;
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const { (out + i)[lo] = c(u, r); }
     template <int R, int MT>
     __device__ inline void apply(int row0, int N, int M, int lane, const int64_t (&tot)[R][MT]) const {
 #pragma unroll
@@ -391,6 +431,14 @@ struct EpiRaw {
     int64_t* out; int ldo;
     EpiRaw offset_m(int m0) const { EpiRaw e = *this; e.out += (size_t)m0 * ldo; return e; }
     __device__ inline void one(int r, int m, int64_t acc) const { out[(size_t)m * ldo + r] = acc; }
+    struct Col { uint32_t fast; };
+    __device__ inline Col col(int) const { return Col{1}; }
+    using Elt = EpiNoElt;
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col&, const Elt&) const {
+        (out + i)[lo] = 256 * (int64_t)u + r;
+    }
     template <int R, int MT>
     __device__ inline void apply(int row0, int N, int M, int lane, const int64_t (&tot)[R][MT]) const {
 #pragma unroll

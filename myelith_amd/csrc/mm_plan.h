@@ -25,12 +25,15 @@ struct Mm2Dims {
     static constexpr int kSwzRows = 256 / KS;  // rows sharing one swizzle slot
     static constexpr int kStageBytes = (BR + BN) * KS;
     static constexpr size_t kLds = (size_t)STAGES * kStageBytes;
-    // 1 KiB wave loads per stage, dealt round-robin to the waves: every wave
-    // issues kLoadsMin or kLoadsMax of them
+    // 1 KiB wave loads per stage, dealt round-robin to the waves; every wave
+    // issues kLoads (past the last group: that group again, the same bytes)
     static constexpr int kGroups = (BR + BN) / kRowsPerLoad;
-    static constexpr int kLoadsMin = kGroups / (kThreads / 64);
-    static constexpr int kLoadsMax = (kGroups + kThreads / 64 - 1) / (kThreads / 64);
+    static constexpr int kLoads = (kGroups + kThreads / 64 - 1) / (kThreads / 64);
     static_assert((BR + BN) % kRowsPerLoad == 0, "whole 1 KiB loads");
+    static_assert((STAGES - 1) * kLoads < 64, "a wait can count the loads in flight");
+    // waves per SIMD the register budget must allow: two blocks per CU where
+    // the stages leave room for them
+    static constexpr int kMinWaves = std::max(1, (kLds <= 80 * 1024 ? 2 : 1) * (kThreads / 64) / 4);
 };
 
 // Grid of a launch over `items` work items: a multiple of 8 (the XCD count),

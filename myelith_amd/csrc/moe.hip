@@ -361,6 +361,7 @@ struct EpiExpertGU {
         out[(size_t)row * n2 + n] =
             clamp_i16_i64(rescale64(acc, (uint8_t)(shifts[(size_t)e * n2 + n] + MYL_MOE_X_FRAC), frac));
     }
+    using Col = PlaneRescale;
 };
 
 // The grouped gate/up fused with the SiLU gate (mlp.rs:46-65) and the byte-plane
@@ -374,7 +375,12 @@ struct EpiExpertGUSiluPlanes {
     const int16_t* silu;
     uint32_t silu_len;
     int8_t* planes;         // [2R x I]
-    __device__ inline int16_t stage(int e, int n, int64_t acc) const {
+    using Col = PlaneRescale;
+    __device__ inline Col col(int e, int n) const {
+        return Col::of((uint8_t)(shifts[(size_t)e * n2 + n] + MYL_MOE_X_FRAC), (n & 1) ? MYL_MOE_UP_FRAC : MYL_MOE_GATE_FRAC);
+    }
+    __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return clamp_i16(c(u, r)); }
+    __device__ inline int16_t stage64(int e, int n, int64_t acc) const {
         const uint8_t frac = (n & 1) ? MYL_MOE_UP_FRAC : MYL_MOE_GATE_FRAC;
         return clamp_i16_i64(rescale64(acc, (uint8_t)(shifts[(size_t)e * n2 + n] + MYL_MOE_X_FRAC), frac));
     }
@@ -402,6 +408,12 @@ struct EpiExpertDown {
         out[(size_t)row * H + n] = clamp_i16_i64(
             rescale64(acc, (uint8_t)(shifts[(size_t)e * H + n] + MYL_MOE_DOWN_IN_FRAC), out_frac[n]));
     }
+    using Col = PlaneRescale;
+    __device__ inline Col col(int e, int n) const {
+        return Col::of((uint8_t)(shifts[(size_t)e * H + n] + MYL_MOE_DOWN_IN_FRAC), out_frac[n]);
+    }
+    __device__ inline size_t idx(int n, int row) const { return (size_t)row * H + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c) const { (out + i)[lo] = clamp_i16(c(u, r)); }
 };
 
 // ---------------------------------------------------------------------------
@@ -526,18 +538,18 @@ int moe_planes_tile(int H, int I) {
     return k128 ? 0 : 1;
 }
 int moe_tile_tokens(int tile) {
-    return tile == 0 ? Mm2GroupedShape<2, 2, 4, 4, 2, 128>::kTokens
+    return tile == 0 ? Mm2GroupedShape<4, 2, 2, 4, 2, 128>::kTokens
                      : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kTokens : Mm2GroupedShape<2, 1, 2, 4, 4, 64>::kTokens;
 }
 int moe_tile_rows(int tile) {
-    return tile == 0 ? Mm2GroupedShape<2, 2, 4, 4, 2, 128>::kRows
+    return tile == 0 ? Mm2GroupedShape<4, 2, 2, 4, 2, 128>::kRows
                      : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kRows : Mm2GroupedShape<2, 1, 2, 4, 4, 64>::kRows;
 }
 template <class EpiG>
 hipError_t moe_grouped(int tile, const int8_t* Ap, const int8_t* W, size_t w_stride, int N, int K, const int* offsets,
                        const MmWork* work, const int* nwork, int maxwork, const EpiG& epi, hipStream_t st) {
     if (tile == 0)
-        return mm2_grouped_launch<2, 2, 4, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
+        return mm2_grouped_launch<4, 2, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
     if (tile == 1)
         return mm2_grouped_launch<2, 2, 4, 2, 3, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
     return mm2_grouped_launch<2, 1, 2, 4, 4, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
@@ -548,7 +560,7 @@ hipError_t moe_grouped_staged(int tile, const int8_t* Ap, const int8_t* W, size_
                               const int* offsets, const MmWork* work, const int* nwork, int maxwork, const EpiG& epi,
                               hipStream_t st) {
     if (tile == 0)
-        return mm2_grouped_staged_launch<2, 2, 4, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi,
+        return mm2_grouped_staged_launch<4, 2, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi,
                                                              st);
     if (tile == 1)
         return mm2_grouped_staged_launch<2, 2, 4, 2, 3, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi,

@@ -4,6 +4,7 @@
 #pragma once
 
 #include "fixed.h"
+#include "gemv.h"
 #include "wave.h"
 #include "../../include/myl_theta_v.h"
 
@@ -46,6 +47,22 @@ struct EpiQKVRows : EpiApply<EpiQKVRows> {
         return v;
     }
     __device__ inline void one(int n, int m, int64_t acc) const { out[(size_t)m * ldo + n] = value(n, acc); }
+    struct Col { PlaneRescale r; uint32_t fast; int32_t b; };
+    __device__ inline Col col(int n) const {
+        const ValOps o = val_ops(n);
+        const uint8_t frac = n < nq ? q_frac : (n < nq + nkv ? k_frac : v_frac);
+        const PlaneRescale r = PlaneRescale::of((uint8_t)(o.sh + act_frac), frac);
+        // a bias past +-2^17 saturates the sum whatever the projection; no
+        // bias is one of 0 (the second clamp then changes nothing)
+        const int32_t b = bias ? rescale32((int32_t)o.b, o.bs, frac) : 0;
+        return Col{r, r.fast, min(max(b, -131072), 131072)};
+    }
+    using Elt = EpiNoElt;
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const {
+        (out + i)[lo] = clamp_i16((int32_t)clamp_i16(c.r(u, r)) + c.b);
+    }
 };
 
 // o_proj / down_proj with the residual add (model.rs:576-593, 612-671):
@@ -57,11 +74,11 @@ struct EpiResidRows : EpiApply<EpiResidRows> {
     const uint8_t* acc_frac;
     const uint8_t* res_frac;
     const uint8_t* out_frac;
-    const int16_t* res; int ldr;
+    const int16_t* res;  // laid out as out
     int16_t* out; int ldo;
     EpiResidRows offset_m(int m0) const {
         EpiResidRows e = *this;
-        e.res += (size_t)m0 * ldr;
+        e.res += (size_t)m0 * ldo;
         e.out += (size_t)m0 * ldo;
         return e;
     }
@@ -77,7 +94,7 @@ struct EpiResidRows : EpiApply<EpiResidRows> {
     // previous element's stores: one memory round trip per element).
     struct FinOps { uint8_t af, sh, rf, of; int16_t r; };
     __device__ inline FinOps fin_ops(int n, int m) const {
-        return FinOps{acc_frac[n], shifts[n], res_frac[n], out_frac[n], res[(size_t)m * ldr + n]};
+        return FinOps{acc_frac[n], shifts[n], res_frac[n], out_frac[n], res[(size_t)m * ldo + n]};
     }
     __device__ inline int16_t value_of(int64_t acc, const FinOps& o) const {
         const int16_t v = clamp_i16_i64(rescale64(acc, (uint8_t)(o.sh + act_frac), o.af));
@@ -85,6 +102,19 @@ struct EpiResidRows : EpiApply<EpiResidRows> {
         return clamp_i16_i64(rescale64(wadd64(h, (int64_t)v), o.af, o.of));
     }
     __device__ inline void one(int n, int m, int64_t acc) const { (void)value(n, m, acc); }
+    struct Col { PlaneRescale o; SmallRescale h, y; uint32_t fast; };
+    __device__ inline Col col(int n) const {
+        const uint8_t af = acc_frac[n];
+        const PlaneRescale o = PlaneRescale::of((uint8_t)(shifts[n] + act_frac), af);
+        const SmallRescale h = SmallRescale::of(res_frac[n], af), y = SmallRescale::of(af, out_frac[n]);
+        return Col{o, h, y, o.fast & h.fast & y.fast};
+    }
+    struct Elt { int16_t r; };
+    __device__ inline Elt elt(size_t i, uint32_t lo) const { return Elt{(res + i)[lo]}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt& e) const {
+        (out + i)[lo] = c.y.clamped(c.h.of16((int32_t)e.r) + (int32_t)clamp_i16(c.o(u, r)));
+    }
 };
 
 // gate (even rows) and up (odd rows) requantized to their own fracs (mlp.rs:46-53).
@@ -96,6 +126,16 @@ struct EpiGURows : EpiApply<EpiGURows> {
     __device__ inline void one(int n, int m, int64_t acc) const {
         const uint8_t frac = (n & 1) ? up_frac : gate_frac;
         out[(size_t)m * ldo + n] = clamp_i16_i64(rescale64(acc, (uint8_t)(shifts[n] + act_frac), frac));
+    }
+    using Col = PlaneRescale;
+    __device__ inline Col col(int n) const {
+        return Col::of((uint8_t)(shifts[n] + act_frac), (n & 1) ? up_frac : gate_frac);
+    }
+    using Elt = EpiNoElt;
+    __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
+    __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const {
+        (out + i)[lo] = clamp_i16(c(u, r));
     }
 };
 
@@ -120,8 +160,14 @@ struct EpiGUSiluPlanes {
     uint8_t act_frac, gate_frac, up_frac, down_in_frac;
     const int16_t* silu; uint32_t silu_len;
     int8_t* planes; int I;
-    __device__ inline int16_t stage(int n, int64_t acc) const { return stage_with(op(n), n, acc); }
-    // the same in two steps: the row's operand, fetched ahead of the sum
+    // the column's requantization, resolved ahead of the sums; the same from the 64-bit sum
+    using Col = PlaneRescale;
+    __device__ inline Col col(int n) const {
+        return Col::of((uint8_t)(shifts[n] + act_frac), (n & 1) ? up_frac : gate_frac);
+    }
+    __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return clamp_i16(c(u, r)); }
+    __device__ inline int16_t stage64(int n, int64_t acc) const { return stage_with(op(n), n, acc); }
+    // in two steps: the row's operand, fetched ahead of the sum
     using Op = uint8_t;
     __device__ inline Op op(int n) const { return shifts[n]; }
     __device__ inline int16_t stage_with(Op sh, int n, int64_t acc) const {

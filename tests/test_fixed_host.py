@@ -299,3 +299,91 @@ def test_score_byte_plane_identity(hd):
         assert ksum == int(k.sum())
         dot = 65536 * hh + 256 * mid + ll + 128 * int(q.sum()) + 128 * ksum - 16384 * hd
         assert dot == int(q.astype(np.int64) @ k.astype(np.int64))
+
+
+SRC_COLS = r"""
+#include <hip/hip_runtime.h>
+#include <cstdio>
+#include <cstdint>
+#include "fixed.h"
+static uint64_t sm = 0x9E3779B97F4A7C15ull;
+static uint64_t next() {
+    uint64_t z = (sm += 0x9E3779B97F4A7C15ull);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+static int16_t mult_general(int64_t acc, int32_t mult, uint8_t shift) {
+    const myl_i128 y = rshift_round128((myl_i128)acc * (myl_i128)mult, shift);
+    return y < -32768 ? (int16_t)-32768 : (y > 32767 ? (int16_t)32767 : (int16_t)y);
+}
+// the extreme and random parts of a sum over K < 2^16: hi, low (fixed.h)
+static void parts(int k, int s, int64_t* hi, int64_t* low) {
+    const int64_t K = 65535, H = 128 * 128 * K, L = 2 * H;
+    switch (k % 6) {
+    case 0: *hi = (k & 8) ? H : -H; *low = (k & 16) ? L : -L; break;
+    case 1: *hi = (int64_t)(next() % 9) - 4; *low = (int64_t)(next() % 1025) - 512; break;
+    case 2:  // half of the last place, and one off it
+        *hi = s >= 10 && s < 38 ? ((int64_t)(next() % 5) - 2) << (s - 9) : 0;
+        *low = (s == 9 ? 256 : 0) + (int64_t)(next() % 3) - 1;
+        break;
+    case 3: *hi = ((int64_t)next() >> 34) >> (k % 30); *low = (int64_t)next() >> 34; break;
+    default: *hi = (int64_t)next() >> 34; *low = ((int64_t)next() >> 33) >> (k % 31); break;
+    }
+}
+int main() {
+    long bad = 0, n = 0, fast = 0;
+    for (int in = 0; in < 256; ++in)
+        for (int out = 0; out < 256; ++out) {
+            const int sh = (int)(int8_t)(in - out);
+            const PlaneRescale p = PlaneRescale::of((uint8_t)in, (uint8_t)out);
+            for (int k = 0; p.fast && k < 300; ++k) {
+                int64_t hi, low;
+                parts(k, sh, &hi, &low);
+                const int64_t want = rescale64(hi * 256 + low, (uint8_t)in, (uint8_t)out);
+                const int32_t l32 = (int32_t)low;
+                ++n, ++fast;
+                bad += (int64_t)p((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u) != want;
+            }
+            const SmallRescale m = SmallRescale::of((uint8_t)in, (uint8_t)out);
+            for (int k = 0; m.fast && k < 60; ++k) {
+                int32_t v = (int32_t)((int64_t)next() >> 34) >> (k % 30);  // |v| < 2^30
+                if (k % 4 == 1) v = (int32_t)(((int64_t)(next() % 9) - 4) << (sh > 0 && sh < 26 ? sh - 1 : 0));
+                const int32_t v16 = (int32_t)(int16_t)next();
+                n += 2;
+                bad += m.clamped(v) != clamp_i16_i64(rescale64(v, (uint8_t)in, (uint8_t)out));
+                bad += (int64_t)m.of16(v16) != rescale64(v16, (uint8_t)in, (uint8_t)out);
+            }
+        }
+    const int32_t ms[] = {0, 1, -1, 3, 1 << 29, 1 << 30, (1 << 30) - 1, INT32_MAX, INT32_MIN, INT32_MIN + 1};
+    for (int s = 0; s < 256; ++s)
+        for (int k = 0; k < 3000; ++k) {
+            const int32_t mult = k % 3 ? (int32_t)next() : ms[(k / 3) % 10];
+            const PlaneMult p = PlaneMult::of(mult, (uint8_t)s);
+            if (!p.fast) continue;
+            int64_t hi, low;
+            parts(k, s - (k % 7 ? 29 : 30), &hi, &low);
+            const int32_t l32 = (int32_t)low;
+            ++n, ++fast;
+            bad += clamp_i16(p((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u)) != mult_general(hi * 256 + low, mult, (uint8_t)s);
+        }
+    printf("checked %ld (plane sums %ld), mismatches %ld\n", n, fast, bad);
+    return bad != 0 || fast < 100000;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None and not Path("/opt/rocm/bin/hipcc").exists(), reason="needs hipcc")
+def test_column_rescales_match_the_general_forms(tmp_path):
+    """PlaneRescale / SmallRescale / PlaneMult against rescale64 and the 128-bit
+    multiplier requant, over every pair of shift bytes they take, ties, and the
+    extremes of the sums and of the multipliers."""
+    src = tmp_path / "cols.hip"
+    src.write_text(SRC_COLS)
+    exe = tmp_path / "cols"
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    r = subprocess.run([hipcc, "-O1", "-std=c++17", "-x", "hip", "--offload-arch=gfx950", "-I",
+                        str(ROOT / "myelith_amd" / "csrc"), str(src), "-o", str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0, out.stdout
