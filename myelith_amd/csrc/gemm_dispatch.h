@@ -97,33 +97,18 @@ inline bool mm_planes_ok(int M, int K, const MmCtx* mm) {
            mm_env("MYL_MM_TILE") < 0;
 }
 
-// Row tiles per group of the tile order of 256 x 256 tiles (TileOrder): the
-// 32 blocks an XCD runs at one time cover 4 row tiles x 8 weight tiles.
-// MYL_MM_GROUP overrides it for sweeps (0: the plain order).
-inline int mm_group() {
-    static const int g = [] {
-        const int v = mm_env("MYL_MM_GROUP");
-        return v >= 0 ? v : 4;
-    }();
-    return g;
-}
-
-// Whether 256 x 256 tiles with 128-byte K stages fill the chip well enough
-// (mm_planes).
-inline bool mm_wide_tiles(int M, int N, int K, int cus) {
-    return K % 128 == 0 && mm2_tiles<4, 2, 2, 4, 2, 128>(M, N) >= cus + cus / 2;
-}
+// Row tiles per group of the tile order (TileOrder): the 32 blocks an XCD runs
+// at one time cover 4 row tiles x 8 weight tiles.
+constexpr int kMmGroup = 4;
 
 // The product on planes Ap [2M x K] (mm_planes_ok): few rows stream the
 // weights once in 64 or 128 plane-row tiles (K split until the chip is
-// full, or half full past 32 rows).  More rows take 256 x 256 block tiles of
-// 16 waves with 128-byte K stages (128 KB of LDS, one block per CU) when the
-// grid holds at least 1.5 such tiles per CU: 12-25% faster than the
-// alternative on MI355X for 2048-4096 rows of the 7B projections.  Smaller
-// grids, where the last partial wave of big tiles costs more than the stage
-// width gains (about 15% slower at 1.2 tiles per CU), take 256 x 128 tiles
-// with 64-byte stages (72 KB of LDS, two blocks per CU) when those give
-// every CU a tile.
+// full, or half full past 32 rows).  More rows take the tile of mm2_wide_pick;
+// long sums with at most one 64 x 128 tile per CU split K (100 / 250 rows of the
+// 7B down projection: 40 / 63 us split, 74 / 80 whole; with K = 4864 the partial
+// sums cost what the split gains).  K not a multiple of 128: 256 x 128 tiles
+// with 64-byte stages (two blocks per CU) when those give every CU a tile,
+// else 128 x 128 split over K.
 template <class Epi>
 inline hipError_t mm_planes(const int8_t* Ap, int M, const int8_t* W, int N, int K, const Epi& epi, const MmCtx* mm,
                             hipStream_t st) {
@@ -143,8 +128,17 @@ inline hipError_t mm_planes(const int8_t* Ap, int M, const int8_t* W, int N, int
     if (M <= 32 && K % 128 == 0) return mm2_launch_splitk<2, 1, 1, 4, 2, 128>(Ap, M, W, N, K, epi, mm, 2 * cus, st);
     if (M <= 32) return mm2_launch_splitk<2, 1, 1, 4, 4>(Ap, M, W, N, K, epi, mm, cus, st);
     if (M <= 64 && K % 128 == 0) return mm2_launch_splitk<1, 1, 4, 2, 3, 128>(Ap, M, W, N, K, epi, mm, cus, st);
-    if (M > 64 && mm_wide_tiles(M, N, K, cus)) return mm2_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, mm_group());
-    if (M > 64 && mm2_tiles<2, 2, 4, 2, 3>(M, N) >= cus) return mm2_launch<2, 2, 4, 2, 3>(Ap, M, W, N, K, epi, st);
+    if (K % 128 == 0) {
+        switch (mm2_wide_pick(M, N, cus)) {
+        case kMm2Wide256: return mm2_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2Wide192: return mm2_launch<3, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2Wide128: return mm2_launch<2, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        default: break;
+        }
+        if (K >= 8192) return mm2_launch_splitk<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, mm, cus + 1, st);
+        return mm2_launch<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+    }
+    if (M > 64 && mm2_tiles<2, 2, 4, 2, 3>(M, N) >= cus) return mm2_launch<2, 2, 4, 2, 3>(Ap, M, W, N, K, epi, st, kMmGroup);
     return mm2_launch_splitk<2, 1, 2, 4, 4>(Ap, M, W, N, K, epi, mm, cus / 2, st);
 }
 
@@ -184,8 +178,15 @@ inline hipError_t mm_planes_staged(const int8_t* Ap, int M, const int8_t* W, int
     if (M <= 16) return mm2_staged_launch<1, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 32) return mm2_staged_launch<2, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 64) return mm2_staged_launch<2, 1, 2, 2, 4, 128>(Ap, M, W, N, K, epi, st);
-    if (mm_wide_tiles(M, N, K, mm->cus)) return mm2_staged_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, mm_group());
-    return mm2_staged_launch<2, 2, 4, 2, 3, 64>(Ap, M, W, N, K, epi, st);
+    if (K % 128 == 0) {
+        switch (mm2_wide_pick(M, N, mm->cus)) {
+        case kMm2Wide256: return mm2_staged_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2Wide192: return mm2_staged_launch<3, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2Wide128: return mm2_staged_launch<2, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        default: return mm2_staged_launch<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        }
+    }
+    return mm2_staged_launch<2, 2, 4, 2, 3, 64>(Ap, M, W, N, K, epi, st, kMmGroup);
 }
 
 // Tile and K split, from a sweep of the W8A16 shapes on MI355X: 64-row tiles

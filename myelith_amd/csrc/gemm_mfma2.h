@@ -63,28 +63,28 @@ struct Mm2 : Mm2Dims<MB, NB, WM_, WN_, STAGES, KS> {
 
 // Order of a product's output tiles over the grid.  mm_tile_index gives each
 // XCD a contiguous range of tile numbers; here tile numbers run over groups
-// of G row tiles (the row-tile count padded to a multiple of G, padding
-// tiles exit at once), the row tile fastest inside a group.  G = tiles_r is
-// the plain order (all row tiles of one weight tile, then the next weight
-// tile): the blocks an XCD runs at one time share one weight tile and read
-// as many distinct A' tiles.  A small G makes them cover G row tiles x
-// (blocks / G) weight tiles, so both operands are shared in the XCD's L2.
+// of G row tiles (the last group may have fewer), the row tile fastest inside
+// a group.  G = tiles_r is the plain order (all row tiles of one weight tile,
+// then the next weight tile): the blocks an XCD runs at one time share one
+// weight tile and read as many distinct A' tiles.  A small G makes them cover
+// G row tiles x (blocks / G) weight tiles, so both operands are shared in the
+// XCD's L2.
 struct TileOrder {
-    Divider span;  // G * tiles_n
-    Divider g;     // G
-    uint32_t tiles_r;
+    Divider span;        // G * tiles_n
+    Divider g, g_last;   // row tiles of a group, of the last group
+    uint32_t last;       // the last group
     static TileOrder of(int tiles_r, int tiles_n, int G) {
-        if (G < 1 || G > tiles_r) G = tiles_r;
-        return TileOrder{Divider::of((uint32_t)(G * tiles_n)), Divider::of((uint32_t)G), (uint32_t)tiles_r};
+        G = mm2_group_rows(tiles_r, G);
+        const int last = (tiles_r - 1) / G;
+        return TileOrder{Divider::of((uint32_t)(G * tiles_n)), Divider::of((uint32_t)G),
+                         Divider::of((uint32_t)(tiles_r - last * G)), (uint32_t)last};
     }
-    // tile numbers the grid must cover
-    int count(int tiles_n) const { return (int)(((tiles_r + g.d - 1) / g.d) * g.d) * tiles_n; }
-    __device__ inline bool decode(uint32_t t, uint32_t& tn, uint32_t& tr) const {
+    __device__ inline void decode(uint32_t t, uint32_t& tn, uint32_t& tr) const {
         uint32_t grp, in, r;
         span.divmod(t, grp, in);
-        g.divmod(in, tn, r);
+        if (grp < last) g.divmod(in, tn, r);
+        else g_last.divmod(in, tn, r);
         tr = grp * g.d + r;
-        return tr < tiles_r;
     }
 };
 
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, 
     const int t = mm_tile_index(ntiles);
     if (t < 0) return;
     uint32_t tn, tr;
-    if (!ord.decode((uint32_t)t, tn, tr)) return;
+    ord.decode((uint32_t)t, tn, tr);
     mm2_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, 0, K, (int)tr * S::BR, (int)tn * S::BN, lds, SinkEpi<Epi>{epi});
 }
 
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, 
     const int t = mm_tile_index(ntiles);
     if (t < 0) return;
     uint32_t tn, tr;
-    if (!ord.decode((uint32_t)t, tn, tr)) return;
+    ord.decode((uint32_t)t, tn, tr);
     mm2_staged_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, (int)tr * S::BR, (int)tn * S::BN, lds, epi);
 }
 
@@ -372,7 +372,7 @@ hipError_t mm2_staged_launch(const int8_t* Ap, int M, const int8_t* W, int N, in
     const int R2 = 2 * M;
     const int tiles_r = (R2 + S::BR - 1) / S::BR, tiles_n = (N + S::BN - 1) / S::BN;
     const TileOrder ord = TileOrder::of(tiles_r, tiles_n, group);
-    const int ntiles = ord.count(tiles_n);
+    const int ntiles = tiles_r * tiles_n;
     auto kern = mm2_staged_kernel<MB, NB, WM_, WN_, STAGES, KS, Epi>;
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLds);
     if (e != hipSuccess) return e;
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, 
     const int t = mm_tile_index(ntiles);
     if (t < 0) return;
     uint32_t tn, tr;
-    if (!ord.decode((uint32_t)t, tn, tr)) return;
+    ord.decode((uint32_t)t, tn, tr);
     mm2w16_tile<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, Wp, N2, K, xsum, wsum, (int)tr * S::BR, (int)tn * S::BN, lds,
                                           epi);
 }
@@ -482,7 +482,7 @@ hipError_t mm2w16_launch_cfg(const int8_t* Ap, const int32_t* xsum, int M, const
     const int R2 = 2 * M, N2 = 2 * N;
     const int tiles_r = (R2 + S::BR - 1) / S::BR, tiles_n = (N2 + S::BN - 1) / S::BN;
     const TileOrder ord = TileOrder::of(tiles_r, tiles_n, group);
-    const int ntiles = ord.count(tiles_n);
+    const int ntiles = tiles_r * tiles_n;
     auto kern = mm2w16_kernel<MB, NB, WM_, WN_, STAGES, KS, Epi>;
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLds);
     if (e != hipSuccess) return e;
@@ -637,7 +637,7 @@ hipError_t mm2_launch(const int8_t* Ap, int M, const int8_t* W, int N, int K, co
     const int R2 = 2 * M;
     const int tiles_r = (R2 + S::BR - 1) / S::BR, tiles_n = (N + S::BN - 1) / S::BN;
     const TileOrder ord = TileOrder::of(tiles_r, tiles_n, group);
-    const int ntiles = ord.count(tiles_n);
+    const int ntiles = tiles_r * tiles_n;
     auto kern = mm2_kernel<MB, NB, WM_, WN_, STAGES, KS, Epi>;
     if (S::kLds > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S::kLds);

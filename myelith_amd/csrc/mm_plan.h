@@ -40,6 +40,41 @@ struct Mm2Dims {
 // so block b's XCD is b % 8 for every tile-order computation.
 inline int mm2_grid_of(int items) { return 8 * ((items + 7) / 8); }
 
+// Tiles of products of more than 64 rows with K % 128 == 0 (plane rows x
+// weight rows, 128-byte K stages, two of them).  256 x 256 and 192 x 256 fill
+// a CU (128 and 112 KB of LDS) and share their operands best; 128 x 128 runs
+// two, 64 x 128 three blocks per CU.
+enum Mm2Wide { kMm2Wide256, kMm2Wide192, kMm2Wide128, kMm2Wide64 };
+
+// The tile by the time of the busiest CU.  A CU's queue of q tiles took, on
+// MI355X at K = 3584 (us): 256 x 256 53 q; 192 x 256 44.5 q; 128 x 128 19 for
+// one tile and 17.5 q from two on; 64 x 128 15.5 for one and 9.9 q from two on.
+// So the large tiles win where they fill whole rounds of the chip (down of the
+// 7B layout over 1500 rows: 224 tiles of 192 x 256 258 us, 168 of 256 x 256 297,
+// 672 of 128 x 128 261; q/k/v: 216 of 256 x 256 56 us, 288 of 192 x 256 84) and
+// the small ones where few tiles would leave CUs idle (200 rows of q/k/v: 252
+// of 64 x 128 17.4 us, 144 of 128 x 128 20.5, 36 of 256 x 256 48).
+inline Mm2Wide mm2_wide_pick(int M, int N, int cus) {
+    auto queue = [&](int br, int bn) {
+        const int64_t t = (int64_t)((2 * (int64_t)M + br - 1) / br) * ((N + bn - 1) / bn);
+        return (double)((t + cus - 1) / cus);
+    };
+    const double qs[4] = {queue(256, 256), queue(192, 256), queue(128, 128), queue(64, 128)};
+    const double cost[4] = {53.0 * qs[0], 44.5 * qs[1], qs[2] <= 1 ? 19.0 : 17.5 * qs[2], qs[3] <= 1 ? 15.5 : 9.9 * qs[3]};
+    int best = 0;
+    for (int i = 1; i < 4; ++i)
+        if (cost[i] < cost[best]) best = i;
+    return (Mm2Wide)best;
+}
+
+// The row tiles of a group of the grouped tile order (TileOrder): about `want`,
+// so that no group is much smaller than the others.
+inline int mm2_group_rows(int tiles_r, int want) {
+    if (want < 1 || tiles_r <= want) return tiles_r;
+    const int groups = (tiles_r + want - 1) / want;
+    return (tiles_r + groups - 1) / groups;
+}
+
 // The K split of a product over M activation rows (A' = 2M plane rows), N
 // weight rows and K (a multiple of KS): with fewer tiles than `fill` and
 // room for the M x N i64 partial sums, K is cut into ns slices of kslice

@@ -526,24 +526,25 @@ int ensure(myl_moe* m, int T) {
 }
 
 // Byte-plane tile of the grouped expert products: 0: 128 tokens x 256 weight
-// rows (16 waves, 128-byte stages), 1: 128 x 128 (8 waves, 64-byte stages),
-// 2: 64 x 128 (8 waves).  The whole 4096-token, 60-expert layer on MI355X
-// took 1.42, 1.49 and 1.58 ms with them (1.75 ms with the int16-row tiles of
-// mm_w8_grouped_kernel), so 0 when both K are multiples of 128.
-// MYL_MOE_TILE overrides the choice for sweeps.
-int moe_planes_tile(int H, int I) {
+// rows (128-byte stages), 1: 128 x 128 (64-byte stages), 2: 64 x 128 (128-byte
+// stages), all of 8 waves.  Tile 2 wastes less on experts of few tokens, tile 0
+// moves fewer operand bytes; the whole 60-expert layer on MI355X took with
+// tiles 0 / 2: 16 tokens 179 / 157 us, 400 335 / 292, 1000 (67 rows per expert)
+// 444 / 397, 3001 (200 rows) 795 / 807, 4000 951 / 1010.  Tile 1 only where a
+// K is not a multiple of 128.  MYL_MOE_TILE overrides the choice for sweeps.
+int moe_planes_tile(int H, int I, int R, int E) {
     const bool k128 = H % 128 == 0 && I % 128 == 0;
     const int v = mm_env("MYL_MOE_TILE");
-    if (v >= 0 && v <= 2) return (v == 0 && !k128) ? 1 : v;
-    return k128 ? 0 : 1;
+    if (v >= 0 && v <= 2) return !k128 ? 1 : v;
+    return !k128 ? 1 : R >= 160 * E ? 0 : 2;
 }
 int moe_tile_tokens(int tile) {
     return tile == 0 ? Mm2GroupedShape<4, 2, 2, 4, 2, 128>::kTokens
-                     : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kTokens : Mm2GroupedShape<2, 1, 2, 4, 4, 64>::kTokens;
+                     : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kTokens : Mm2GroupedShape<2, 1, 2, 4, 2, 128>::kTokens;
 }
 int moe_tile_rows(int tile) {
     return tile == 0 ? Mm2GroupedShape<4, 2, 2, 4, 2, 128>::kRows
-                     : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kRows : Mm2GroupedShape<2, 1, 2, 4, 4, 64>::kRows;
+                     : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kRows : Mm2GroupedShape<2, 1, 2, 4, 2, 128>::kRows;
 }
 template <class EpiG>
 hipError_t moe_grouped(int tile, const int8_t* Ap, const int8_t* W, size_t w_stride, int N, int K, const int* offsets,
@@ -552,7 +553,7 @@ hipError_t moe_grouped(int tile, const int8_t* Ap, const int8_t* W, size_t w_str
         return mm2_grouped_launch<4, 2, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
     if (tile == 1)
         return mm2_grouped_launch<2, 2, 4, 2, 3, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
-    return mm2_grouped_launch<2, 1, 2, 4, 4, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
+    return mm2_grouped_launch<2, 1, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
 }
 
 template <class EpiG>
@@ -565,7 +566,7 @@ hipError_t moe_grouped_staged(int tile, const int8_t* Ap, const int8_t* W, size_
     if (tile == 1)
         return mm2_grouped_staged_launch<2, 2, 4, 2, 3, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi,
                                                             st);
-    return mm2_grouped_staged_launch<2, 1, 2, 4, 4, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
+    return mm2_grouped_staged_launch<2, 1, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
 }
 
 // Work items of a grouped product over R routed rows of E experts in token
@@ -651,7 +652,7 @@ int myl_moe_forward(myl_moe* m, const int16_t* x_dev, uint32_t n_tokens, int16_t
         // byte-plane expert products, planned on the device: offsets and
         // work tables from the counts without a host round trip; the planes
         // [2R x H] and [2R x I] take the bytes of Xg and Hh
-        const int tile = moe_planes_tile(H, I);
+        const int tile = moe_planes_tile(H, I, R, E);
         const int bm = moe_tile_tokens(tile), bn = moe_tile_rows(tile);
         int bm_log = 0;
         while ((1 << bm_log) < bm) ++bm_log;

@@ -221,6 +221,35 @@ def test_mfma_large_m_byte_plane_product(backend, oracle, M, N, K):
     assert np.array_equal(y[rows], exp)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 300, 128), (129, 70, 8320), (450, 3580, 128), (1500, 3583, 128), (1501, 4599, 256)])
+def test_wide_tiles_and_requant_columns(backend, oracle, M, N, K):
+    """The tiles of more than 64 rows (64 x 128, the same split over K, 128 x 128,
+    192 x 256, 256 x 256; ragged rows and columns), with shifts in and out of
+    the range of the 32-bit requantization mixed over the columns (blocks of
+    columns inside it, so that both forms run), full-range activations
+    and weights, against the oracle's requant of the exact sums."""
+    import torch
+    case(f"wide tiles M={M} N={N} K={K}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + 5 * N + K)
+    x = torch.randint(-32768, 32768, (M, K), dtype=torch.int16, device="cuda", generator=g)
+    W = torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda", generator=g)
+    x[0], W[1] = -32768, -128
+    acc = (x.double() @ W.double().T).to(torch.int64).cpu().numpy()
+    r = rng(M * 3 + N)
+    for lo, hi in ((0, 48), (9, 20)):  # shift - 10 + 10: any of 0..47; inside 9..38
+        ws = r.integers(lo, hi, N).astype(np.uint8)
+        ws[: N // 2] = r.integers(9, 16, N // 2)
+        got = backend.linear_w8a16_dev(x, W, torch.from_numpy(ws).cuda(), 10, 10).cpu().numpy()
+        assert np.array_equal(got, oracle.requant_shift(acc, ws, 10, 10)), (lo, hi)
+    mult = r.integers(-(1 << 31), 1 << 31, N).astype(np.int32)
+    mult[:5] = [0, -1, 1 << 30, -(1 << 31), (1 << 31) - 1]
+    sh = r.integers(20, 80, N).astype(np.uint8)
+    sh[: N // 2] = r.integers(39, 60, N // 2)
+    got = backend.linear_w8a16_mult_dev(x, W, torch.from_numpy(mult).cuda(), torch.from_numpy(sh).cuda()).cpu().numpy()
+    assert np.array_equal(got, oracle.requant_mult(acc, mult, sh))
+
+
 @pytest.mark.parametrize("M", [64, 512])
 @pytest.mark.parametrize("N,K", SWEEP)
 def test_mfma_full_size_exact_sums(backend, M, N, K):

@@ -39,7 +39,7 @@ LLVM = Path("/opt/rocm/llvm/bin")
 
 # The split-K shapes of gemm_dispatch.h (mm_planes, mm_planes_fin).
 SPLIT_SHAPES = [(1, 1, 1, 4, 3, 128), (1, 1, 1, 2, 4, 128), (1, 1, 1, 4, 4, 64), (2, 1, 1, 4, 2, 128),
-                (2, 1, 1, 4, 4, 64), (1, 1, 4, 2, 3, 128), (2, 1, 2, 4, 4, 64)]
+                (2, 1, 1, 4, 4, 64), (1, 1, 4, 2, 3, 128), (2, 1, 2, 4, 4, 64), (1, 1, 2, 4, 2, 128)]
 
 DRIVER = r"""
 #include "mm_plan.h"
@@ -99,6 +99,14 @@ int main() {
     run<2, 1, 1, 4, 4, 64>("2,1,1,4,4,64");
     run<1, 1, 4, 2, 3, 128>("1,1,4,2,3,128");
     run<2, 1, 2, 4, 4, 64>("2,1,2,4,4,64");
+    run<1, 1, 2, 4, 2, 128>("1,1,2,4,2,128");
+    // groups of the tile order: the full ones and the last cover the row tiles
+    for (int tiles = 1; tiles < 300; ++tiles)
+        for (int want = 0; want < 9; ++want) {
+            const int G = mm2_group_rows(tiles, want), last = (tiles - 1) / G;
+            CHECK(G >= 1 && (want < 1 || G <= want || tiles <= want) && tiles - last * G >= 1 && tiles - last * G <= G,
+                  "group of %d row tiles, want %d: %d", tiles, want, G);
+        }
     std::printf("checked %ld bad %ld\n", checked, bad);
     return bad != 0;
 }
