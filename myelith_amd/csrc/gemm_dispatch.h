@@ -11,6 +11,7 @@
 
 #include "gemm_mfma.h"
 #include "gemm_mfma2.h"
+#include "gemm_rows.h"
 #include "gemv.h"
 #include "gemv_stream.h"
 #include "internal.h"
@@ -102,11 +103,9 @@ inline bool mm_planes_ok(int M, int K, const MmCtx* mm) {
 constexpr int kMmGroup = 4;
 
 // The product on planes Ap [2M x K] (mm_planes_ok): few rows stream the
-// weights once in 64 or 128 plane-row tiles (K split until the chip is
-// full, or half full past 32 rows).  More rows take the tile of mm2_wide_pick;
-// long sums with at most one 64 x 128 tile per CU split K (100 / 250 rows of the
-// 7B down projection: 40 / 63 us split, 74 / 80 whole; with K = 4864 the partial
-// sums cost what the split gains).  K not a multiple of 128: 256 x 128 tiles
+// weights once in 32 or 64 plane-row tiles (K split until the chip is full).
+// More than 32 rows take the tile (or split) of mm2_pick.
+// K not a multiple of 128: 256 x 128 tiles
 // with 64-byte stages (two blocks per CU) when those give every CU a tile,
 // else 128 x 128 split over K.
 template <class Epi>
@@ -123,20 +122,21 @@ inline hipError_t mm_planes(const int8_t* Ap, int M, const int8_t* W, int N, int
         return mm2_launch_splitk<1, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, mm, 2 * cus, st);
     }
     if (M <= 16) return mm2_launch_splitk<1, 1, 1, 4, 4>(Ap, M, W, N, K, epi, mm, 2 * cus, st);
-    // up to 32 / 64 tokens: 128-byte stages on 64- / 128-row plane tiles
-    // (5-20% faster than 64-byte stages on the 7B shapes)
+    // up to 32 tokens: 128-byte stages on 64-row plane tiles (5-20% faster than
+    // 64-byte stages on the 7B shapes)
     if (M <= 32 && K % 128 == 0) return mm2_launch_splitk<2, 1, 1, 4, 2, 128>(Ap, M, W, N, K, epi, mm, 2 * cus, st);
     if (M <= 32) return mm2_launch_splitk<2, 1, 1, 4, 4>(Ap, M, W, N, K, epi, mm, cus, st);
-    if (M <= 64 && K % 128 == 0) return mm2_launch_splitk<1, 1, 4, 2, 3, 128>(Ap, M, W, N, K, epi, mm, cus, st);
     if (K % 128 == 0) {
-        switch (mm2_wide_pick(M, N, cus)) {
-        case kMm2Wide256: return mm2_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
-        case kMm2Wide192: return mm2_launch<3, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
-        case kMm2Wide128: return mm2_launch<2, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
-        default: break;
+        const Mm2Pick p = mm2_pick(M, N, K, cus, mm->acc_elems);
+        if (p.split) return mm2_launch_splitk<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, mm, cus + 1, st);
+        switch (p.tile) {
+        case kMm2T256: return mm2_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T192: return mm2_launch<3, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T128: return mm2_launch<2, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T128s3: return mm2_launch<2, 1, 2, 4, 3, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T64: return mm2_launch<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        default: return mm2_launch<1, 1, 2, 2, 3, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
         }
-        if (K >= 8192) return mm2_launch_splitk<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, mm, cus + 1, st);
-        return mm2_launch<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
     }
     if (M > 64 && mm2_tiles<2, 2, 4, 2, 3>(M, N) >= cus) return mm2_launch<2, 2, 4, 2, 3>(Ap, M, W, N, K, epi, st, kMmGroup);
     return mm2_launch_splitk<2, 1, 2, 4, 4>(Ap, M, W, N, K, epi, mm, cus / 2, st);
@@ -179,11 +179,13 @@ inline hipError_t mm_planes_staged(const int8_t* Ap, int M, const int8_t* W, int
     if (M <= 32) return mm2_staged_launch<2, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 64) return mm2_staged_launch<2, 1, 2, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (K % 128 == 0) {
-        switch (mm2_wide_pick(M, N, mm->cus)) {
-        case kMm2Wide256: return mm2_staged_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
-        case kMm2Wide192: return mm2_staged_launch<3, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
-        case kMm2Wide128: return mm2_staged_launch<2, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
-        default: return mm2_staged_launch<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        switch (mm2_pick(M, N, K, mm->cus, 0).tile) {
+        case kMm2T256: return mm2_staged_launch<4, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T192: return mm2_staged_launch<3, 2, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T128: return mm2_staged_launch<2, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T128s3: return mm2_staged_launch<2, 1, 2, 4, 3, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        case kMm2T64: return mm2_staged_launch<1, 1, 2, 4, 2, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
+        default: return mm2_staged_launch<1, 1, 2, 2, 3, 128>(Ap, M, W, N, K, epi, st, kMmGroup);
         }
     }
     return mm2_staged_launch<2, 2, 4, 2, 3, 64>(Ap, M, W, N, K, epi, st, kMmGroup);
@@ -197,6 +199,14 @@ template <class Epi>
 inline hipError_t mm_i8(const int16_t* x, int M, int ldx, const int8_t* W, int N, int K, const Epi& epi,
                         const MmCtx* mm, hipStream_t st) {
     const int cus = mm ? mm->cus : 256;
+    // 2-32 rows: the weight stream (gemm_rows.h).  It reads x itself, so no
+    // planes are split first, and for most shapes no partial sums are added up
+    // (per product of the 7B layout, 8 / 32 rows: gate 20.9 -> 15.6 / 31.4 -> 22.5 us,
+    // o_proj 10.4 -> 7.0 / 15.0 -> 12.9, down 21.5 -> 18.2 / 31.7 -> 26.9).
+    if (mm && mm_env("MYL_MM_TILE") < 0) {
+        const RowsPlan pl = rows_plan(M, N, K, 1, cus, mm->acc ? mm->acc_elems : 0);
+        if (pl.S && rows_x_ok(M, ldx)) return rows_mm_i8(pl, RowsSrcX{x, ldx}, M, W, N, K, epi, mm, st);
+    }
     // The activations split once into byte planes, then the pipelined int8
     // product (gemm_mfma2.h).
     if (mm_planes_ok(M, K, mm)) {
@@ -261,12 +271,18 @@ inline hipError_t gemv_i8(const int16_t* x, int M, int ldx, const int8_t* W, int
 
 template <class Epi>
 inline hipError_t gemv_i16(const int16_t* x, int M, int ldx, const int16_t* W, int N, int K, const Epi& epi,
-                           hipStream_t st) {
+                           hipStream_t st, const MmCtx* mm = nullptr) {
     const bool fast = (K % 8 == 0) && (((uintptr_t)W & 15) == 0) && K <= 8192;
     if (!fast) {
         dim3 grid((N + 255) / 256, M);
         gemv_generic_kernel<int16_t, Epi><<<grid, 256, 0, st>>>(x, M, ldx, W, N, K, epi);
         return hipGetLastError();
+    }
+    // 2-32 rows: the weight stream (gemm_rows.h; 5 rows of the 7B head: 164 us, 350
+    // in the LDS tiles below).
+    if (M > 1 && xvec_ok(x, ldx) && mm) {
+        const RowsPlan pl = rows_plan(M, N, K, 2, mm->cus, 0);
+        if (pl.S && rows_x_ok(M, ldx)) return rows_mm_i16(pl, RowsSrcX{x, ldx}, M, W, N, K, epi, st);
     }
     // More than one activation row: the int8 matrix cores, four byte-plane products.
     if (M > 1 && xvec_ok(x, ldx) && K < 65536) {

@@ -341,10 +341,8 @@ struct EpiShift {
     }
     __device__ inline void one(int r, int m, int64_t acc) const { one_ops(r, m, acc, ops(r)); }
     using Col = PlaneRescale;
-    __device__ inline Col col(int n) const {
-        const Ops o = ops(n);
-        return Col::of((uint8_t)(o.ws + act_frac), o.of);
-    }
+    __device__ inline Col col_of(const Ops& o) const { return Col::of((uint8_t)(o.ws + act_frac), o.of); }
+    __device__ inline Col col(int n) const { return col_of(ops(n)); }
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
@@ -379,7 +377,8 @@ struct EpiMult {
     }
     __device__ inline void one(int r, int m, int64_t acc) const { one_ops(r, m, acc, ops(r)); }
     using Col = PlaneMult;
-    __device__ inline Col col(int n) const { return Col::of(mult[n], shift[n]); }
+    __device__ inline Col col_of(const Ops& o) const { return Col::of(o.mult, o.shift); }
+    __device__ inline Col col(int n) const { return col_of(ops(n)); }
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
@@ -411,7 +410,8 @@ struct EpiLogits {
     }
     __device__ inline void one(int r, int m, int64_t acc) const { one_ops(r, m, acc, ops(r)); }
     using Col = PlaneRescale;
-    __device__ inline Col col(int n) const { return Col::of((uint8_t)(row_shifts[n] + norm_frac), logit_frac); }
+    __device__ inline Col col_of(const Ops& o) const { return Col::of((uint8_t)(o.sh + norm_frac), logit_frac); }
+    __device__ inline Col col(int n) const { return col_of(ops(n)); }
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
@@ -432,7 +432,11 @@ struct EpiRaw {
     EpiRaw offset_m(int m0) const { EpiRaw e = *this; e.out += (size_t)m0 * ldo; return e; }
     __device__ inline void one(int r, int m, int64_t acc) const { out[(size_t)m * ldo + r] = acc; }
     struct Col { uint32_t fast; };
+    struct Ops {};
+    __device__ inline Ops ops(int) const { return Ops{}; }
+    __device__ inline Col col_of(const Ops&) const { return Col{1}; }
     __device__ inline Col col(int) const { return Col{1}; }
+    __device__ inline void one_ops(int n, int m, int64_t acc, const Ops&) const { one(n, m, acc); }
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }

@@ -30,7 +30,7 @@ hipError_t logits_w8(const int16_t* x, int M, int ldx, const int8_t* W, int N, i
 hipError_t logits_w16(const int16_t* x, int M, int ldx, const int16_t* W, int N, int K, const uint8_t* row_shifts,
                       uint8_t norm_frac, uint8_t logit_frac, int32_t* out, int ldo, hipStream_t st, const MmCtx* mm) {
     EpiLogits e{row_shifts, norm_frac, logit_frac, out, ldo};
-    return gemv_i16(x, M, ldx, W, N, K, e, st);
+    return gemv_i16(x, M, ldx, W, N, K, e, st, mm);
 }
 
 hipError_t dot_raw_w8(const int16_t* x, int M, int ldx, const int8_t* W, int N, int K, int64_t* out, int ldo,

@@ -40,33 +40,6 @@ struct Mm2Dims {
 // so block b's XCD is b % 8 for every tile-order computation.
 inline int mm2_grid_of(int items) { return 8 * ((items + 7) / 8); }
 
-// Tiles of products of more than 64 rows with K % 128 == 0 (plane rows x
-// weight rows, 128-byte K stages, two of them).  256 x 256 and 192 x 256 fill
-// a CU (128 and 112 KB of LDS) and share their operands best; 128 x 128 runs
-// two, 64 x 128 three blocks per CU.
-enum Mm2Wide { kMm2Wide256, kMm2Wide192, kMm2Wide128, kMm2Wide64 };
-
-// The tile by the time of the busiest CU.  A CU's queue of q tiles took, on
-// MI355X at K = 3584 (us): 256 x 256 53 q; 192 x 256 44.5 q; 128 x 128 19 for
-// one tile and 17.5 q from two on; 64 x 128 15.5 for one and 9.9 q from two on.
-// So the large tiles win where they fill whole rounds of the chip (down of the
-// 7B layout over 1500 rows: 224 tiles of 192 x 256 258 us, 168 of 256 x 256 297,
-// 672 of 128 x 128 261; q/k/v: 216 of 256 x 256 56 us, 288 of 192 x 256 84) and
-// the small ones where few tiles would leave CUs idle (200 rows of q/k/v: 252
-// of 64 x 128 17.4 us, 144 of 128 x 128 20.5, 36 of 256 x 256 48).
-inline Mm2Wide mm2_wide_pick(int M, int N, int cus) {
-    auto queue = [&](int br, int bn) {
-        const int64_t t = (int64_t)((2 * (int64_t)M + br - 1) / br) * ((N + bn - 1) / bn);
-        return (double)((t + cus - 1) / cus);
-    };
-    const double qs[4] = {queue(256, 256), queue(192, 256), queue(128, 128), queue(64, 128)};
-    const double cost[4] = {53.0 * qs[0], 44.5 * qs[1], qs[2] <= 1 ? 19.0 : 17.5 * qs[2], qs[3] <= 1 ? 15.5 : 9.9 * qs[3]};
-    int best = 0;
-    for (int i = 1; i < 4; ++i)
-        if (cost[i] < cost[best]) best = i;
-    return (Mm2Wide)best;
-}
-
 // The row tiles of a group of the grouped tile order (TileOrder): about `want`,
 // so that no group is much smaller than the others.
 inline int mm2_group_rows(int tiles_r, int want) {
@@ -103,6 +76,58 @@ inline Mm2SplitPlan mm2_split_plan(int M, int N, int K, int cus, size_t acc_elem
     p.ns = p.split ? (K + p.kslice - 1) / p.kslice : 1;
     p.nitems = p.ntiles * p.ns;
     p.grid = mm2_grid_of(p.nitems);
+    return p;
+}
+
+// Tiles of products of more than 32 rows with K % 128 == 0 (plane rows x weight
+// rows, 128-byte K stages).  256 x 256 and 192 x 256 fill a CU's LDS with two
+// stages and share their operands best; 128 x 128 and 64 x 128 with two stages
+// run two and three blocks per CU; with three stages, 128 x 128 hides the
+// memory latency of a lone block and 64 x 64 that of three small ones.
+enum Mm2Tile { kMm2T256, kMm2T192, kMm2T128, kMm2T128s3, kMm2T64, kMm2T64s3 };
+
+struct Mm2Pick {
+    Mm2Tile tile = kMm2T256;
+    bool split = false;  // K split of the 64 x 128 tiles through the accumulator
+};
+
+// The tile by the time of the busiest CU's queue of q tiles, measured on MI355X
+// with weights from HBM, us at K = 3584: 256 x 256 53 q; 192 x 256 44.5 q;
+// 128 x 128 22 alone (three stages; 28 with two), 17.6 q queued; 64 x 128 12 q
+// queued; 64 x 64 14 alone, 19 for two, then 7 q + 6.  So the large tiles win
+// where they fill whole rounds of the chip (down of the 7B layout over 1500 rows:
+// 224 tiles of 192 x 256 258 us, 168 of 256 x 256 297, 672 of 128 x 128 261) and
+// the small ones where few tiles would leave CUs idle (100 rows of o_proj: 224 of
+// 64 x 64 13.9 us, 56 of 128 x 128 20.4, 14 of 256 x 256 49).  A K split adds
+// about 5 us for the finish and its 64-bit atomics (about 180 a ns): 64 rows of
+// the 7B down projection 35 us in 10 slices, 58 whole; 300 rows x 896 x 4864 20
+// split, 17 whole.
+inline Mm2Pick mm2_pick(int M, int N, int K, int cus, size_t acc_elems) {
+    auto queue = [&](int br, int bn) {
+        const int64_t t = (int64_t)((2 * (int64_t)M + br - 1) / br) * ((N + bn - 1) / bn);
+        return (double)((t + cus - 1) / cus);
+    };
+    const double q2 = queue(128, 128), q4 = queue(64, 128), q5 = queue(64, 64);
+    const double cost[6] = {53.0 * queue(256, 256),
+                            44.5 * queue(192, 256),
+                            q2 <= 1 ? 28.0 : 17.6 * q2,
+                            q2 <= 1 ? 22.0 : 21.0 * q2,
+                            q4 <= 1 ? 25.0 : q4 <= 2 ? 28.0 : 12.0 * q4,
+                            q5 <= 1 ? 14.0 : q5 <= 2 ? 19.0 : 7.0 * q5 + 6.0};
+    int best = 0;
+    for (int i = 1; i < 6; ++i)
+        if (cost[i] < cost[best]) best = i;
+    Mm2Pick p;
+    p.tile = (Mm2Tile)best;
+    if (K >= 2048) {
+        const Mm2SplitPlan sp = mm2_split_plan<1, 1, 2, 4, 2, 128>(M, N, K, cus, acc_elems, cus + 1);
+        if (sp.split) {
+            const double qs = (double)((sp.nitems + cus - 1) / cus);
+            const double t = (double)sp.kslice / 3584.0 * (qs <= 1 ? 25.0 : qs <= 2 ? 28.0 : 12.0 * qs) + 5.0 +
+                             (double)M * N * sp.ns / 180000.0;
+            if (t < (double)K / 3584.0 * cost[best]) p.tile = kMm2T64, p.split = true;
+        }
+    }
     return p;
 }
 
@@ -158,6 +183,54 @@ inline bool frag_split_ok(int R, int K, int N, int cus, size_t acc_elems) {
     if (frag_rt(R) == 0 || R < 1 || K <= 0 || K % 64 != 0 || N <= 0 || (size_t)R * (size_t)N > acc_elems) return false;
     const FragSplit sp = frag_split_plan(K, N, cus);
     return sp.kpw != 0 && 16 * sp.ngb <= kFragWaves * 64 && frag_lds(frag_rt(R), sp.ngb, R, false) <= kFragLdsMax;
+}
+
+// ---- products of 2-32 rows on row-major weights (gemm_rows.h) ---------------
+
+constexpr int kRowsWaves = 8;
+constexpr int kRowsUnit = 2048;  // bytes of a unit: 16 weight rows x 128 bytes
+constexpr int kRowsRing = 8;     // units a wave has in flight (a power of two)
+constexpr int kRowsCpol = 2;     // the weights' cache policy: streaming
+constexpr int kRowsOpsBytes = 8; // output operands of a column, kept in LDS
+constexpr int kRowsMaxGroups = 80;  // row groups per block: their operands fit the LDS
+
+// Row groups per epilogue window and the LDS of a launch: the waves' rings, two
+// windows of plane sums (RT KiB a group), three of weight row sums, the
+// activations' sums; a launch adds its columns' operands.
+template <int RT>
+struct RowsDims {
+    static constexpr int G = RT <= 2 ? 4 : 2;
+    static constexpr size_t kLds =
+        (size_t)kRowsWaves * kRowsRing * kRowsUnit + (size_t)(2 * G * RT * 256 + 3 * G * 16 + RT * 16) * 4;
+    static_assert(kLds + 16 * kRowsMaxGroups * kRowsOpsBytes <= 160 * 1024, "LDS of a CU");
+};
+
+// S K slices of csl columns (128 weight bytes) x P parts of the row groups, at
+// most one block per CU; U columns per wave.  S == 0: not supported.
+struct RowsPlan {
+    int S = 0, P = 0, U = 0, C = 0, csl = 0, ngb = 0;
+};
+
+// The plan whose busiest block ends first.  A CU streams about 24 KB/us when all
+// do (6.2 TB/s); a K split adds the finish launch (about 4 us) and its 64-bit
+// atomics (about 90 a ns for the chip).  7B down, 13 rows: 8 slices x 32 parts
+// of 7 row groups, all CUs equally busy; the 7B head (9504 groups) needs none.
+inline RowsPlan rows_plan(int M, int N, int K, int wbytes, int cus, size_t acc_elems) {
+    RowsPlan best;
+    if (M < 2 || M > kFragMaxRows || N < 1 || N >= (1 << 22) || K % 64 != 0 || K * wbytes < 128 || K >= 65536 || cus < 1 || cus > 1024)
+        return best;
+    const int C = (K * wbytes + 127) / 128, umax = wbytes == 1 ? 4 : 8, NG = (N + 15) / 16;
+    double best_t = 0;
+    for (int S = 1; S <= std::min(C, 16) && S <= cus; ++S) {
+        if (S > 1 && (wbytes != 1 || (size_t)M * (size_t)N > acc_elems)) break;
+        const int csl = (C + S - 1) / S, U = (csl + kRowsWaves - 1) / kRowsWaves;
+        if (U > umax || (int64_t)(S - 1) * csl >= C) continue;
+        const int P = std::min(cus / S, NG), ngb = (NG + P - 1) / P;
+        if (ngb > kRowsMaxGroups || (int64_t)ngb * 16 * K * wbytes >= (1ll << 31)) continue;
+        const double t = (double)ngb * csl * kRowsUnit / 24200.0 + (S > 1 ? 4.0 + (double)M * N * S / 90000.0 : 0.0);
+        if (best.S == 0 || t < best_t) best = RowsPlan{S, P, U, C, csl, ngb}, best_t = t;
+    }
+    return best;
 }
 
 }  // namespace myl

@@ -526,48 +526,56 @@ int ensure(myl_moe* m, int T) {
 }
 
 // Byte-plane tile of the grouped expert products: 0: 128 tokens x 256 weight
-// rows (128-byte stages), 1: 128 x 128 (64-byte stages), 2: 64 x 128 (128-byte
-// stages), all of 8 waves.  Tile 2 wastes less on experts of few tokens, tile 0
-// moves fewer operand bytes; the whole 60-expert layer on MI355X took with
-// tiles 0 / 2: 16 tokens 179 / 157 us, 400 335 / 292, 1000 (67 rows per expert)
-// 444 / 397, 3001 (200 rows) 795 / 807, 4000 951 / 1010.  Tile 1 only where a
-// K is not a multiple of 128.  MYL_MOE_TILE overrides the choice for sweeps.
+// rows (two 128-byte stages), 1: 128 x 128 (64-byte stages), 2: 64 x 128 (two
+// 128-byte stages), 3: 32 x 64 (three).  Small tiles waste less on experts of
+// few tokens and keep more blocks loading, large ones move fewer operand bytes;
+// the whole 60-expert layer on MI355X, us:
+//   tokens (rows per expert)   16 (1)  100 (7)  400 (27)  1000 (67)  2400 (160)  3001 (200)
+//   tile 0                     157     261      316       426        664         795
+//   tile 2                     125     210      265       379        647         807
+//   tile 3                     114     202      283       444        878
+// Tile 1 only where a K is not a multiple of 128.  MYL_MOE_TILE overrides the
+// choice for sweeps.
 int moe_planes_tile(int H, int I, int R, int E) {
     const bool k128 = H % 128 == 0 && I % 128 == 0;
     const int v = mm_env("MYL_MOE_TILE");
-    if (v >= 0 && v <= 2) return !k128 ? 1 : v;
-    return !k128 ? 1 : R >= 160 * E ? 0 : 2;
+    if (v >= 0 && v <= 3) return !k128 ? 1 : v;
+    return !k128 ? 1 : R >= 180 * E ? 0 : R >= 14 * E ? 2 : 3;
 }
+#define MYL_MOE_TILES(F)                        \
+    switch (tile) {                             \
+    case 0: return F(4, 2, 2, 4, 2, 128);       \
+    case 1: return F(2, 2, 4, 2, 3, 64);        \
+    case 2: return F(2, 1, 2, 4, 2, 128);       \
+    default: return F(1, 1, 2, 2, 3, 128);      \
+    }
 int moe_tile_tokens(int tile) {
-    return tile == 0 ? Mm2GroupedShape<4, 2, 2, 4, 2, 128>::kTokens
-                     : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kTokens : Mm2GroupedShape<2, 1, 2, 4, 2, 128>::kTokens;
+#define MYL_MOE_TOKENS(...) Mm2GroupedShape<__VA_ARGS__>::kTokens
+    MYL_MOE_TILES(MYL_MOE_TOKENS)
 }
 int moe_tile_rows(int tile) {
-    return tile == 0 ? Mm2GroupedShape<4, 2, 2, 4, 2, 128>::kRows
-                     : tile == 1 ? Mm2GroupedShape<2, 2, 4, 2, 3, 64>::kRows : Mm2GroupedShape<2, 1, 2, 4, 2, 128>::kRows;
+#define MYL_MOE_ROWS(...) Mm2GroupedShape<__VA_ARGS__>::kRows
+    MYL_MOE_TILES(MYL_MOE_ROWS)
 }
 template <class EpiG>
 hipError_t moe_grouped(int tile, const int8_t* Ap, const int8_t* W, size_t w_stride, int N, int K, const int* offsets,
                        const MmWork* work, const int* nwork, int maxwork, const EpiG& epi, hipStream_t st) {
-    if (tile == 0)
-        return mm2_grouped_launch<4, 2, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
-    if (tile == 1)
-        return mm2_grouped_launch<2, 2, 4, 2, 3, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
-    return mm2_grouped_launch<2, 1, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
+#define MYL_MOE_PLAIN(...) (mm2_grouped_launch<__VA_ARGS__>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st))
+    MYL_MOE_TILES(MYL_MOE_PLAIN)
 }
 
 template <class EpiG>
 hipError_t moe_grouped_staged(int tile, const int8_t* Ap, const int8_t* W, size_t w_stride, int N, int K,
                               const int* offsets, const MmWork* work, const int* nwork, int maxwork, const EpiG& epi,
                               hipStream_t st) {
-    if (tile == 0)
-        return mm2_grouped_staged_launch<4, 2, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi,
-                                                             st);
-    if (tile == 1)
-        return mm2_grouped_staged_launch<2, 2, 4, 2, 3, 64>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi,
-                                                            st);
-    return mm2_grouped_staged_launch<2, 1, 2, 4, 2, 128>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st);
+#define MYL_MOE_STAGED(...) (mm2_grouped_staged_launch<__VA_ARGS__>(Ap, W, w_stride, N, K, offsets, work, nwork, maxwork, epi, st))
+    MYL_MOE_TILES(MYL_MOE_STAGED)
 }
+#undef MYL_MOE_TILES
+#undef MYL_MOE_TOKENS
+#undef MYL_MOE_ROWS
+#undef MYL_MOE_PLAIN
+#undef MYL_MOE_STAGED
 
 // Work items of a grouped product over R routed rows of E experts in token
 // tiles of bm: sum_e ceil(c_e / bm) <= floor(R / bm) + E token tiles.

@@ -48,14 +48,20 @@ struct EpiQKVRows : EpiApply<EpiQKVRows> {
     }
     __device__ inline void one(int n, int m, int64_t acc) const { out[(size_t)m * ldo + n] = value(n, acc); }
     struct Col { PlaneRescale r; uint32_t fast; int32_t b; };
-    __device__ inline Col col(int n) const {
-        const ValOps o = val_ops(n);
-        const uint8_t frac = n < nq ? q_frac : (n < nq + nkv ? k_frac : v_frac);
-        const PlaneRescale r = PlaneRescale::of((uint8_t)(o.sh + act_frac), frac);
+    struct Ops { ValOps v; uint8_t frac; };
+    __device__ inline Ops ops(int n) const {
+        return Ops{val_ops(n), n < nq ? q_frac : (n < nq + nkv ? k_frac : v_frac)};
+    }
+    __device__ inline Col col_of(const Ops& o) const {
+        const PlaneRescale r = PlaneRescale::of((uint8_t)(o.v.sh + act_frac), o.frac);
         // a bias past +-2^17 saturates the sum whatever the projection; no
         // bias is one of 0 (the second clamp then changes nothing)
-        const int32_t b = bias ? rescale32((int32_t)o.b, o.bs, frac) : 0;
+        const int32_t b = bias ? rescale32((int32_t)o.v.b, o.v.bs, o.frac) : 0;
         return Col{r, r.fast, min(max(b, -131072), 131072)};
+    }
+    __device__ inline Col col(int n) const { return col_of(ops(n)); }
+    __device__ inline void one_ops(int n, int m, int64_t acc, const Ops& o) const {
+        out[(size_t)m * ldo + n] = value_with(o.v, n, acc);
     }
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
@@ -103,11 +109,16 @@ struct EpiResidRows : EpiApply<EpiResidRows> {
     }
     __device__ inline void one(int n, int m, int64_t acc) const { (void)value(n, m, acc); }
     struct Col { PlaneRescale o; SmallRescale h, y; uint32_t fast; };
-    __device__ inline Col col(int n) const {
-        const uint8_t af = acc_frac[n];
-        const PlaneRescale o = PlaneRescale::of((uint8_t)(shifts[n] + act_frac), af);
-        const SmallRescale h = SmallRescale::of(res_frac[n], af), y = SmallRescale::of(af, out_frac[n]);
+    struct Ops { uint8_t af, sh, rf, of; };
+    __device__ inline Ops ops(int n) const { return Ops{acc_frac[n], shifts[n], res_frac[n], out_frac[n]}; }
+    __device__ inline Col col_of(const Ops& p) const {
+        const PlaneRescale o = PlaneRescale::of((uint8_t)(p.sh + act_frac), p.af);
+        const SmallRescale h = SmallRescale::of(p.rf, p.af), y = SmallRescale::of(p.af, p.of);
         return Col{o, h, y, o.fast & h.fast & y.fast};
+    }
+    __device__ inline Col col(int n) const { return col_of(ops(n)); }
+    __device__ inline void one_ops(int n, int m, int64_t acc, const Ops& p) const {
+        out[(size_t)m * ldo + n] = value_of(acc, FinOps{p.af, p.sh, p.rf, p.of, res[(size_t)m * ldo + n]});
     }
     struct Elt { int16_t r; };
     __device__ inline Elt elt(size_t i, uint32_t lo) const { return Elt{(res + i)[lo]}; }
@@ -123,14 +134,17 @@ struct EpiGURows : EpiApply<EpiGURows> {
     uint8_t act_frac, gate_frac, up_frac;
     int16_t* out; int ldo;
     EpiGURows offset_m(int m0) const { EpiGURows e = *this; e.out += (size_t)m0 * ldo; return e; }
-    __device__ inline void one(int n, int m, int64_t acc) const {
-        const uint8_t frac = (n & 1) ? up_frac : gate_frac;
-        out[(size_t)m * ldo + n] = clamp_i16_i64(rescale64(acc, (uint8_t)(shifts[n] + act_frac), frac));
+    struct Ops {
+        uint8_t sh, frac;
+    };
+    __device__ inline Ops ops(int n) const { return Ops{shifts[n], (n & 1) ? up_frac : gate_frac}; }
+    __device__ inline void one_ops(int n, int m, int64_t acc, const Ops& o) const {
+        out[(size_t)m * ldo + n] = clamp_i16_i64(rescale64(acc, (uint8_t)(o.sh + act_frac), o.frac));
     }
+    __device__ inline void one(int n, int m, int64_t acc) const { one_ops(n, m, acc, ops(n)); }
     using Col = PlaneRescale;
-    __device__ inline Col col(int n) const {
-        return Col::of((uint8_t)(shifts[n] + act_frac), (n & 1) ? up_frac : gate_frac);
-    }
+    __device__ inline Col col_of(const Ops& o) const { return Col::of((uint8_t)(o.sh + act_frac), o.frac); }
+    __device__ inline Col col(int n) const { return col_of(ops(n)); }
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }

@@ -221,10 +221,60 @@ def test_mfma_large_m_byte_plane_product(backend, oracle, M, N, K):
     assert np.array_equal(y[rows], exp)
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 300, 128), (129, 70, 8320), (450, 3580, 128), (1500, 3583, 128), (1501, 4599, 256)])
+@pytest.mark.parametrize("M,N,K", [(2, 1, 128), (3, 17, 192), (8, 130, 896), (9, 257, 3584), (16, 33, 4160), (17, 300, 448),
+                                   (32, 4097, 256), (13, 3584, 18944), (5, 152064, 128), (31, 60, 65472)])
+def test_few_row_weight_stream(backend, oracle, M, N, K):
+    """2-32 rows through the weight stream: one to four plane tiles, ragged row
+    groups, K with a half column (K % 128 == 64), whole sums and K slices, more
+    epilogue windows than one, a strided x, full-range values; exact sums, shift
+    and multiplier requant (columns in and out of the 32-bit form)."""
+    import torch
+    case(f"weight stream M={M} N={N} K={K}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + 3 * N + K)
+    x = torch.randint(-32768, 32768, (M, K + 24), dtype=torch.int16, device="cuda", generator=g)[:, 8:8 + K]
+    W = torch.randint(-128, 128, (N, K), dtype=torch.int8, device="cuda", generator=g)
+    x[0], W[0] = -32768, -128
+    acc = (x.double() @ W.double().T).to(torch.int64)
+    assert torch.equal(backend.dot_i8_i16_dev(x, W), acc)
+    assert torch.equal(backend.dot_i8_i16_dev(x, W), acc)  # the split accumulator is clear again
+    acc = acc.cpu().numpy()
+    r = rng(M * 3 + N)
+    ws = r.integers(0, 48, N).astype(np.uint8)
+    ws[: N // 2] = r.integers(9, 16, N // 2)
+    got = backend.linear_w8a16_dev(x, W, torch.from_numpy(ws).cuda(), 10, 10).cpu().numpy()
+    assert np.array_equal(got, oracle.requant_shift(acc, ws, 10, 10))
+    mult = r.integers(-(1 << 31), 1 << 31, N).astype(np.int32)
+    sh = r.integers(20, 80, N).astype(np.uint8)
+    got = backend.linear_w8a16_mult_dev(x, W, torch.from_numpy(mult).cuda(), torch.from_numpy(sh).cuda()).cpu().numpy()
+    assert np.array_equal(got, oracle.requant_mult(acc, mult, sh))
+
+
+@pytest.mark.parametrize("M,N,K", [(2, 5, 64), (8, 300, 896), (9, 70, 1024), (16, 130, 3584), (17, 33, 4096), (32, 5000, 128)])
+def test_few_row_int16_weight_stream(backend, M, N, K):
+    """The int16 head over 2-32 rows: the byte planes of both operands, against
+    float64 sums (below 2^53) rounded half to even."""
+    import torch
+    case(f"int16 weight stream M={M} N={N} K={K}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + 3 * N + K)
+    x = torch.randint(-32768, 32768, (M, K), dtype=torch.int16, device="cuda", generator=g)
+    W = torch.randint(-32768, 32768, (N, K), dtype=torch.int16, device="cuda", generator=g)
+    x[0], W[0] = -32768, -32768
+    sh = torch.randint(8, 24, (N,), dtype=torch.uint8, device="cuda", generator=g)
+    acc = (x.double() @ W.double().T).to(torch.int64)
+    s = sh.to(torch.int64) + 10 - 6
+    q = acc >> s
+    rem, half = acc - (q << s), torch.ones_like(s) << (s - 1)
+    want = torch.clamp(q + ((rem > half) | ((rem == half) & ((q & 1) == 1))).to(torch.int64), -2**31, 2**31 - 1)
+    assert torch.equal(backend.logits_dev(x, W, sh, 10, 6), want.to(torch.int32))
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 300, 128), (129, 70, 8320), (450, 3580, 128), (1500, 3583, 128), (1501, 4599, 256),
+                                   (33, 40, 256), (100, 40, 4864), (1000, 18944, 128)])
 def test_wide_tiles_and_requant_columns(backend, oracle, M, N, K):
-    """The tiles of more than 64 rows (64 x 128, the same split over K, 128 x 128,
-    192 x 256, 256 x 256; ragged rows and columns), with shifts in and out of
+    """The tiles of more than 32 rows (64 x 64, 64 x 128, the same split over K,
+    128 x 128, 192 x 256, 256 x 256; ragged rows and columns), with shifts in and out of
     the range of the 32-bit requantization mixed over the columns (blocks of
     columns inside it, so that both forms run), full-range activations
     and weights, against the oracle's requant of the exact sums."""

@@ -100,6 +100,30 @@ int main() {
     run<1, 1, 4, 2, 3, 128>("1,1,4,2,3,128");
     run<2, 1, 2, 4, 4, 64>("2,1,2,4,4,64");
     run<1, 1, 2, 4, 2, 128>("1,1,2,4,2,128");
+    // products of 2-32 rows on row-major weights: K and the row groups covered
+    // once, LDS within the CU, whatever the CU count
+    for (int wb = 1; wb <= 2; ++wb)
+        for (int cus : {1, 8, 104, 256, 304})
+            for (int M : {1, 2, 8, 9, 17, 32, 33})
+                for (int N : {1, 15, 60, 896, 4608, 18944, 152064})
+                    for (int K : {64, 128, 192, 896, 3584, 4160, 18944, 65472, 65536}) {
+                        const RowsPlan p = rows_plan(M, N, K, wb, cus, (size_t)4 << 20);
+                        if (p.S == 0) {
+                            CHECK(M < 2 || M > 32 || K * wb < 128 || K >= 65536 || (N + 15) / 16 > kRowsMaxGroups * cus ||
+                                      (wb == 2 && K > 4096) || (wb == 1 && K > 4096 && cus < 16),
+                                  "rows plan refused %d %d %d wb %d cus %d", M, N, K, wb, cus);
+                            continue;
+                        }
+                        const int NG = (N + 15) / 16;
+                        CHECK(M >= 2 && M <= 32 && p.S * p.P <= cus, "rows blocks %d x %d", p.S, p.P);
+                        CHECK(p.C * 128 >= K * wb && (p.C - 1) * 128 < K * wb, "rows columns %d", p.C);
+                        CHECK(p.S * p.csl >= p.C && (p.S - 1) * p.csl < p.C, "rows slices %d x %d of %d", p.S, p.csl, p.C);
+                        CHECK(p.U * kRowsWaves >= p.csl && p.U <= (wb == 1 ? 4 : 8), "rows columns per wave %d", p.U);
+                        CHECK(p.P <= NG && p.ngb == (NG + p.P - 1) / p.P && p.ngb <= kRowsMaxGroups, "rows groups %d", p.ngb);
+                        CHECK(p.S == 1 || (wb == 1 && (size_t)M * N <= ((size_t)4 << 20)), "rows split beyond the accumulator");
+                        CHECK((long)p.ngb * 16 * K * wb < (1l << 31), "rows descriptor");
+                    }
+    CHECK(RowsDims<1>::kLds + 16 * kRowsMaxGroups * 8 <= 160 * 1024 && RowsDims<4>::kLds + 16 * kRowsMaxGroups * 8 <= 160 * 1024, "rows lds");
     // groups of the tile order: the full ones and the last cover the row tiles
     for (int tiles = 1; tiles < 300; ++tiles)
         for (int want = 0; want < 9; ++want) {
