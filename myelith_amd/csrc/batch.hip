@@ -859,7 +859,12 @@ hipError_t forward_rows(myl_model* m, BatchState* b, int R, int lmax, int h0, in
         return e;
     if (m->spec.lm_head_int16) {
         EpiLogits el{m->lm16_shifts, m->final_norm_frac, MYL_TV_LOGIT_FRAC_BITS, logits_out, V};
-        if (HR >= 2 && H % 64 == 0 && mm && mm->planes && (size_t)2 * HR * H <= mm->planes_bytes) {
+        const RowsPlan hp = mm ? rows_plan(HR, V, H, 2, mm->cus, 0) : RowsPlan{};
+        if (hp.S) {
+            // 2-32 rows: the head's own weights stream once (24 rows of the 7B
+            // head: 216 us on prepared byte planes)
+            if ((e = rows_mm_i16(hp, RowsSrcX{b->Xn, H}, HR, m->lm16, V, H, el, st)) != hipSuccess) return e;
+        } else if (HR >= 2 && H % 64 == 0 && mm && mm->planes && (size_t)2 * HR * H <= mm->planes_bytes) {
             // byte planes of both operands, one int8 product
             if (!m->lm16_planes_ok) {
                 if (!m->lm16_planes) {

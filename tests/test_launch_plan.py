@@ -109,8 +109,10 @@ int main() {
                     for (int K : {64, 128, 192, 896, 3584, 4160, 18944, 65472, 65536}) {
                         const RowsPlan p = rows_plan(M, N, K, wb, cus, (size_t)4 << 20);
                         if (p.S == 0) {
-                            CHECK(M < 2 || M > 32 || K * wb < 128 || K >= 65536 || (N + 15) / 16 > kRowsMaxGroups * cus ||
-                                      (wb == 2 && K > 4096) || (wb == 1 && K > 4096 && cus < 16),
+                            // one slice holds 32 (int8) or 64 columns; int16 sums take no slices
+                            const int S0 = ((K * wb + 127) / 128 + (wb == 1 ? 31 : 63)) / (wb == 1 ? 32 : 64);
+                            CHECK(M < 2 || M > 32 || K * wb < 128 || K >= 65536 || S0 > cus || S0 > 16 ||
+                                      (N + 15) / 16 > kRowsMaxGroups * (cus / S0) || (S0 > 1 && (wb == 2 || (size_t)M * N > ((size_t)4 << 20))),
                                   "rows plan refused %d %d %d wb %d cus %d", M, N, K, wb, cus);
                             continue;
                         }
