@@ -120,7 +120,7 @@ struct PlaneMult {
     }
 };
 
-// rescale64 of a value |v| < 2^30 followed by a clamp to [-2^16, 2^16] or
+// rescale64 of a value |v| <= 2^30 followed by a clamp to [-2^16, 2^16] or
 // narrower, for left shifts of up to 14 and right shifts of up to 30.
 struct SmallRescale {
     uint32_t s, ls, fast;

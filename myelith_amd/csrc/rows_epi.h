@@ -153,14 +153,21 @@ struct EpiGURows : EpiApply<EpiGURows> {
     }
 };
 
+// clamp_i16(rescale64(act * u, in_frac, out_frac)): the product has 31 bits, so
+// shifts of the usual size stay in 32-bit arithmetic (SmallRescale).
+__device__ inline int16_t silu_rescale(int16_t act, int16_t u, uint8_t in_frac, uint8_t out_frac) {
+    const SmallRescale r = SmallRescale::of(in_frac, out_frac);
+    if (r.fast) return r.clamped((int32_t)act * (int32_t)u);
+    return clamp_i16_i64(rescale64((int64_t)act * (int64_t)u, in_frac, out_frac));
+}
+
 // mlp.rs:55-65 for one element: h = clamp(rescale(silu(g) * u, 8 + up_frac,
 // down_in_frac)), silu(g) from the LUT over g in the LUT's input domain.
 __device__ inline int32_t silu_mul(int16_t g, int16_t u, const int16_t* __restrict__ silu, uint32_t silu_len,
                                    uint8_t gate_frac, uint8_t up_frac, uint8_t down_in_frac) {
     const int32_t g_dom = rescale32((int32_t)g, gate_frac, MYL_TV_SILU_IN_FRAC);
     const int16_t act = lut_lookup_i16((int16_t)g_dom, silu, silu_len, (int16_t)MYL_TV_SILU_LUT_OFFSET);
-    const int64_t prod = (int64_t)act * (int64_t)u;
-    return clamp_i16_i64(rescale64(prod, (uint8_t)(MYL_TV_SILU_OUT_FRAC + up_frac), down_in_frac));
+    return silu_rescale(act, u, (uint8_t)(MYL_TV_SILU_OUT_FRAC + up_frac), down_in_frac);
 }
 
 // The gate/up product fused with the SiLU gate and the byte-plane split of

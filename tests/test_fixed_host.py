@@ -349,6 +349,7 @@ int main() {
             for (int k = 0; m.fast && k < 60; ++k) {
                 int32_t v = (int32_t)((int64_t)next() >> 34) >> (k % 30);  // |v| < 2^30
                 if (k % 4 == 1) v = (int32_t)(((int64_t)(next() % 9) - 4) << (sh > 0 && sh < 26 ? sh - 1 : 0));
+                if (k < 2) v = k ? 1 << 30 : -(1 << 30);
                 const int32_t v16 = (int32_t)(int16_t)next();
                 n += 2;
                 bad += m.clamped(v) != clamp_i16_i64(rescale64(v, (uint8_t)in, (uint8_t)out));
