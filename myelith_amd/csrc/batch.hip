@@ -924,8 +924,14 @@ int upload_rows(myl_model* m, BatchState* b, uint32_t R, const uint32_t* seq, co
     if (!rc) rc = ensure_scores(m, b, lm);
     if (rc) return rc;
     // attention tiles: each sequence's rows in position order, at most
-    // kAttnQV / G rows (and kAttnTileRows) per tile
-    const int tr = std::max(1, std::min(kAttnTileRows, kAttnQV / m->G));
+    // kAttnQV / G rows (and kAttnTileRows) per tile; halved down to 32 / G
+    // while their (tile, KV head, range) blocks leave CUs idle (a block's work
+    // is mostly per query vector and position, so few large tiles only make it
+    // longer)
+    int qvt = kAttnQV;
+    const int64_t tile_blocks = (int64_t)m->spec.kv_heads * ((lm + kAttnRange - 1) / kAttnRange);
+    while (qvt > 32 && qvt / 2 >= m->G && ((int64_t)R * m->G + qvt - 1) / qvt * tile_blocks < c->prop.multiProcessorCount) qvt /= 2;
+    const int tr = std::max(1, std::min(kAttnTileRows, qvt / m->G));
     std::vector<std::pair<uint64_t, uint32_t>> order(R);
     for (uint32_t r = 0; r < R; ++r) order[r] = {((uint64_t)seq[r] << 32) | pos[r], r};
     std::sort(order.begin(), order.end());

@@ -112,6 +112,14 @@ struct PlaneMult {
         const uint32_t t = ok ? (uint32_t)shift - 8u : 31u;
         return PlaneMult{mult, t, ok ? 1u : 0u, (int64_t)((1ull << (t - 1)) - 1u)};
     }
+    // For (int32_t)rshift_round64(sum * mult, shift), the attention scores: the
+    // low word of the result, for multipliers below 2^24 and |sum| < 2^38 (the
+    // 64-bit product does not wrap) and shifts 9..62.
+    MYL_FN PlaneMult wrapping(int64_t mult, uint8_t shift) {
+        const bool ok = shift >= 9 && shift <= 62 && mult > -(1 << 24) && mult < (1 << 24);
+        const uint32_t t = ok ? (uint32_t)shift - 8u : 1u;
+        return PlaneMult{ok ? (int32_t)mult : 0, t, ok ? 1u : 0u, (int64_t)((1ull << (t - 1)) - 1u)};
+    }
     MYL_MEM int32_t operator()(int32_t u, uint32_t r) const {
         const int64_t rm = (int64_t)(int32_t)r * mult;
         const int64_t v = (int64_t)u * mult + (int64_t)(int32_t)(rm >> 8);

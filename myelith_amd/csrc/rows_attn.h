@@ -75,7 +75,8 @@ __device__ inline int attn_sub(int MT) { return MT <= 2 ? 128 : 64; }
 
 // Row, head and position of each query vector of the block's tile.
 struct AttnQv {
-    int32_t row[kAttnQV], head[kAttnQV], pos[kAttnQV];
+    int32_t row[kAttnQV], head[kAttnQV];
+    __align__(16) int32_t pos[kAttnQV];
 };
 
 __device__ inline int attn_setup(const AttnTile* __restrict__ tiles, const int32_t* __restrict__ rows, int rows_cap,
@@ -112,8 +113,9 @@ __global__ __launch_bounds__(kAttnThreads) void rows_qk_kernel(
     constexpr int S = HD + 16;  // LDS row stride of a plane
     extern __shared__ __align__(16) int8_t lds[];
     __shared__ AttnQv qv;
-    __shared__ int32_t q_sum[kAttnQV];
-    __shared__ int32_t k_sum[256];
+    __shared__ __align__(16) int32_t q_sum[kAttnQV];  // 128 sum(q) - 16384 HD
+    __shared__ int32_t k_sum[256];                    // 128 sum(k)
+    __shared__ __align__(16) int64_t s_off[kAttnQV];  // of the vector's scores
     __shared__ int s_pmax;
     const int g = blockIdx.y, j0 = blockIdx.z * kAttnRange;
     int QV;
@@ -121,6 +123,8 @@ __global__ __launch_bounds__(kAttnThreads) void rows_qk_kernel(
     const int pmax = s_pmax;
     if (j0 > pmax) return;
     const int jend = min(j0 + kAttnRange, pmax + 1);
+    const PlaneMult pm = PlaneMult::wrapping(mult, shift);
+    if ((int)threadIdx.x < QV) s_off[threadIdx.x] = ((int64_t)qv.row[threadIdx.x] * heads + qv.head[threadIdx.x]) * lcap;
     const int MT = (QV + 31) / 32, sub = attn_sub(MT), NT = sub / 32;
     const int nt_log = sub == 128 ? 2 : 1;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -155,7 +159,7 @@ __global__ __launch_bounds__(kAttnThreads) void rows_qk_kernel(
             *reinterpret_cast<uint2*>(qh + v * S + c * 8) = h;
             *reinterpret_cast<uint2*>(ql + v * S + c * 8) = l;
             const int32_t sv = chunk_row_sum<CH>(sum8_i16(qx[i]));
-            if (c == 0 && v < QV) q_sum[v] = sv;
+            if (c == 0 && v < QV) q_sum[v] = 128 * sv - 16384 * HD;
         }
     }
     const int16_t* kg = kc + (size_t)seq * seq_stride + (size_t)g * max_pos * HD;
@@ -178,7 +182,7 @@ __global__ __launch_bounds__(kAttnThreads) void rows_qk_kernel(
             *reinterpret_cast<uint2*>(kh + p * S + c * 8) = h;
             *reinterpret_cast<uint2*>(kl + p * S + c * 8) = l;
             const int32_t sk = chunk_row_sum<CH>(sum8_i16(kx[i]));
-            if (c == 0) k_sum[p] = sk;
+            if (c == 0) k_sum[p] = 128 * sk;
         }
         __syncthreads();
         for (int task = wave; task < MT * NT; task += kAttnThreads / 64) {
@@ -201,15 +205,28 @@ __global__ __launch_bounds__(kAttnThreads) void rows_qk_kernel(
             }
             // lane: position column br; registers r: vectors 8*(r/4) + 4*(lane/32) + r%4
             const int j = js + br;
-            const int64_t kterm = 128 * (int64_t)k_sum[br] - 16384 * (int64_t)HD;
+            const int32_t kterm = k_sum[br];
+            const int vb = mt * 32 + 4 * (lane >> 5);
+            int32_t* sj = scores + j;
+            // q.k = 65536 hh + 256 mid + low, low = ll + the sums' terms: as 256 u + r
+            // (|256 hh| <= 2^29, |low| < 2^31 for HD <= 128) it scales in 32 x 32-bit
+            // products (PlaneMult); the 64-bit form took 95 us of a 1500-row prefill
+            // layer of the 7B layout.
+            if (pm.fast) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int v = mt * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                if (v < QV && j <= qv.pos[v]) {
-                    const int64_t dot = 65536 * (int64_t)hh[r] + 256 * (int64_t)mid[r] + (int64_t)ll[r] +
-                                        128 * (int64_t)q_sum[v] + kterm;
-                    scores[((size_t)qv.row[v] * heads + qv.head[v]) * lcap + j] =
-                        (int32_t)rshift_round64(wmul64(dot, mult), shift);
+                for (int r = 0; r < 16; ++r) {
+                    const int v = vb + 8 * (r >> 2) + (r & 3);
+                    const int32_t low = ll[r] + (q_sum[v] + kterm);
+                    const int32_t y = pm(256 * hh[r] + mid[r] + (low >> 8), (uint32_t)low & 255u);
+                    if (v < QV && j <= qv.pos[v]) sj[s_off[v]] = y;
+                }
+            } else {
+#pragma unroll 1
+                for (int r = 0; r < 16; ++r) {
+                    const int v = vb + 8 * (r >> 2) + (r & 3);
+                    const int64_t dot =
+                        65536 * (int64_t)hh[r] + 256 * (int64_t)mid[r] + (int64_t)ll[r] + (int64_t)q_sum[v] + (int64_t)kterm;
+                    if (v < QV && j <= qv.pos[v]) sj[s_off[v]] = (int32_t)rshift_round64(wmul64(dot, mult), shift);
                 }
             }
         }

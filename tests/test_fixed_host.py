@@ -356,6 +356,19 @@ int main() {
                 bad += (int64_t)m.of16(v16) != rescale64(v16, (uint8_t)in, (uint8_t)out);
             }
         }
+    for (int s = 0; s < 256; ++s)
+        for (int k = 0; k < 600; ++k) {
+            const int64_t mults[] = {2896, 4096, 4095, (1 << 24) - 1, -((1 << 24) - 1), 1, 0, 1 << 24, 77777};
+            const int64_t mult = mults[k % 9];
+            const PlaneMult p = PlaneMult::wrapping(mult, (uint8_t)s);
+            if (!p.fast) continue;
+            int64_t hi, low;
+            parts(k, s - 12, &hi, &low);
+            if (hi >= (1 << 29) || hi <= -(1 << 29)) hi >>= 2;  // |sum| < 2^38
+            const int32_t l32 = (int32_t)low;
+            ++n, ++fast;
+            bad += p((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u) != (int32_t)rshift_round64((hi * 256 + low) * mult, (uint8_t)s);
+        }
     const int32_t ms[] = {0, 1, -1, 3, 1 << 29, 1 << 30, (1 << 30) - 1, INT32_MAX, INT32_MIN, INT32_MIN + 1};
     for (int s = 0; s < 256; ++s)
         for (int k = 0; k < 3000; ++k) {
