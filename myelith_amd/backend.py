@@ -222,15 +222,18 @@ class RocmBackend:
 
     # ---- device forms (torch tensors on the GPU) ------------------------------
     def linear_w8a16_dev(self, x, W, w_shifts, act_frac: int, out_frac: int = 0, out_frac_pc=None, out=None):
-        import torch
         M, K = x.shape
         N = W.shape[0]
         if out is None:
+            import torch
             out = torch.empty((M, N), dtype=torch.int16, device=x.device)
-        self.check(lib().myl_linear_w8a16_dev(self._h, x.data_ptr(), M, x.stride(0), W.data_ptr(), N, K,
-                                              w_shifts.data_ptr(), act_frac, out_frac,
-                                              None if out_frac_pc is None else out_frac_pc.data_ptr(),
-                                              out.data_ptr(), out.stride(0)), "linear_w8a16_dev")
+        # small products are bound by this call: nothing is imported or wrapped
+        # that the launch does not need
+        rc = lib().myl_linear_w8a16_dev(self._h, x.data_ptr(), M, x.stride(0), W.data_ptr(), N, K, w_shifts.data_ptr(),
+                                        act_frac, out_frac, None if out_frac_pc is None else out_frac_pc.data_ptr(),
+                                        out.data_ptr(), out.stride(0))
+        if rc:
+            self.check(rc, "linear_w8a16_dev")
         return out
 
     def linear_w8a16_dev_noalloc(self, x, W, w_shifts, act_frac: int, out_frac: int = 0, out_frac_pc=None, out=None):
@@ -246,14 +249,15 @@ class RocmBackend:
         return out
 
     def linear_w8a16_mult_dev(self, x, W, mult, shift, out=None):
-        import torch
         M, K = x.shape
         N = W.shape[0]
         if out is None:
+            import torch
             out = torch.empty((M, N), dtype=torch.int16, device=x.device)
-        self.check(lib().myl_linear_w8a16_mult_dev(self._h, x.data_ptr(), M, x.stride(0), W.data_ptr(), N, K,
-                                                   mult.data_ptr(), shift.data_ptr(), out.data_ptr(), out.stride(0)),
-                   "linear_w8a16_mult_dev")
+        rc = lib().myl_linear_w8a16_mult_dev(self._h, x.data_ptr(), M, x.stride(0), W.data_ptr(), N, K, mult.data_ptr(),
+                                             shift.data_ptr(), out.data_ptr(), out.stride(0))
+        if rc:
+            self.check(rc, "linear_w8a16_mult_dev")
         return out
 
     def logits_dev(self, x, W, row_shifts, norm_frac: int, logit_frac: int, out=None):
@@ -269,13 +273,15 @@ class RocmBackend:
         return out
 
     def dot_i8_i16_dev(self, x, W, out=None):
-        import torch
         M, K = x.shape
         N = W.shape[0]
         if out is None:
+            import torch
             out = torch.empty((M, N), dtype=torch.int64, device=x.device)
-        self.check(lib().myl_dot_i8_i16_dev(self._h, x.data_ptr(), M, x.stride(0), W.data_ptr(), N, K,
-                                            out.data_ptr(), out.stride(0)), "dot_i8_i16_dev")
+        rc = lib().myl_dot_i8_i16_dev(self._h, x.data_ptr(), M, x.stride(0), W.data_ptr(), N, K, out.data_ptr(),
+                                      out.stride(0))
+        if rc:
+            self.check(rc, "dot_i8_i16_dev")
         return out
 
     def rmsnorm_dev(self, x, x_shifts, gamma, gamma_shifts, rsqrt_lut, lut_input_shift, lut_output_frac, inv_n_q20,
@@ -300,11 +306,13 @@ class RocmBackend:
         return out
 
     def argmax_dev(self, v, out=None):
-        import torch
         M, n = v.shape
         if out is None:
+            import torch
             out = torch.empty(M, dtype=torch.int64, device=v.device)
-        self.check(lib().myl_argmax_dev(self._h, v.data_ptr(), M, n, v.stride(0), out.data_ptr()), "argmax_dev")
+        rc = lib().myl_argmax_dev(self._h, v.data_ptr(), M, n, v.stride(0), out.data_ptr())
+        if rc:
+            self.check(rc, "argmax_dev")
         return out
 
     def sample_dev(self, z, states, tokens=None, new_states=None):
