@@ -664,7 +664,9 @@ hipError_t forward_rows(myl_model* m, BatchState* b, int R, int lmax, int h0, in
     // (17-64 rows: the split gate/up product with its own finish and SiLU
     // measured faster on MI355X than the unsplit fused one)
     const bool frag = planes && frag_ready(m, R, mm, st);
-    const bool fuse_silu = planes && I % 8 == 0 && (R > 64 || (R <= 16 && H % 128 == 0) || frag) &&
+    const bool fuse_silu = planes && I % 8 == 0 &&
+                           (R > 64 || (R <= 16 && H % 128 == 0) || frag ||
+                            (H % 128 == 0 && rows_short_plan(R, 2 * I, H, mm->cus).S)) &&
                            (size_t)2 * R * ((size_t)I + H) <= mm->planes_bytes;
     int8_t* const xin = mm && mm->planes ? mm->planes + (size_t)2 * R * I : nullptr;  // gate/up input planes
     const uint8_t lut_shift = MYL_TV_SCORE_FRAC_BITS - MYL_TV_EXP_INPUT_FRAC;

@@ -142,6 +142,15 @@ inline hipError_t mm_planes(const int8_t* Ap, int M, const int8_t* W, int N, int
     return mm2_launch_splitk<2, 1, 2, 4, 4>(Ap, M, W, N, K, epi, mm, cus / 2, st);
 }
 
+// Few rows over at most kRowsShortK of K on planes already written: the weight
+// stream in whole sums (gemm_rows.h), where the plane tiles would not split K
+// either and a lone tile's loads are all latency.
+constexpr int kRowsShortK = 1024;
+inline RowsPlan rows_short_plan(int M, int N, int K, int cus) {
+    if (K > kRowsShortK) return RowsPlan{};
+    return rows_plan(M, N, K, 1, cus, 0);
+}
+
 // mm_planes with a custom finish of split products (mm2_launch_splitk_fin):
 // for up to 64 rows the same tiles and splits, and *split tells whether fin
 // ran; more rows take mm_planes (no split, *split = false).
@@ -150,6 +159,8 @@ inline hipError_t mm_planes_fin(const int8_t* Ap, int M, const int8_t* W, int N,
                                 hipStream_t st, const Fin& fin, bool* split) {
     const int cus = mm->cus;
     *split = false;
+    if (const RowsPlan pl = rows_short_plan(M, N, K, cus); pl.S)
+        return rows_mm_run<1>(pl, RowsSrcPlanes{Ap, K}, M, W, N, K, RowsOutEpi<Epi>{epi}, st);
     if (M <= 16 && K % 128 == 0) {
         if (N >= 256 * cus)
             return mm2_launch_splitk_fin<1, 1, 1, 4, 3, 128>(Ap, M, W, N, K, epi, mm, 2 * cus, st, fin, split);
@@ -175,6 +186,8 @@ inline hipError_t mm_planes_staged(const int8_t* Ap, int M, const int8_t* W, int
                                    const MmCtx* mm, hipStream_t st) {
     if (M < 2 || N % 16 != 0 || K % 64 != 0) return hipErrorInvalidValue;
     if (M <= 64 && K % 128 != 0) return hipErrorInvalidValue;
+    if (const RowsPlan pl = rows_short_plan(M, N, K, mm->cus); pl.S)
+        return rows_mm_run<1>(pl, RowsSrcPlanes{Ap, K}, M, W, N, K, RowsOutPair<Epi>{epi}, st);
     if (M <= 16) return mm2_staged_launch<1, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 32) return mm2_staged_launch<2, 1, 1, 2, 4, 128>(Ap, M, W, N, K, epi, st);
     if (M <= 64) return mm2_staged_launch<2, 1, 2, 2, 4, 128>(Ap, M, W, N, K, epi, st);

@@ -69,6 +69,21 @@ struct RowsSrcX {
     }
 };
 
+// The same from byte planes [2M x K] (gemm_mfma2.h).
+struct RowsSrcPlanes {
+    const int8_t* Ap;
+    int K;
+    struct Raw { uint4 h, l; };
+    __device__ inline __amdgpu_buffer_rsrc_t rsrc(int M, int) const { return weight_rsrc(Ap, 2u * (uint32_t)M * (uint32_t)K); }
+    __device__ inline Raw load(const __amdgpu_buffer_rsrc_t& r, int m, int k, bool ok) const {
+        const uint32_t o = 2u * (uint32_t)m * (uint32_t)K + (uint32_t)k;
+        return Raw{cload16(r, ok ? o : 0x7FFFFFC0u), cload16(r, ok ? o + (uint32_t)K : 0x7FFFFFC0u)};
+    }
+    __device__ inline static v4i32_t plane(const Raw& v, bool lo, bool) {
+        return lo ? v4i32_t{(int)v.l.x, (int)v.l.y, (int)v.l.z, (int)v.l.w} : v4i32_t{(int)v.h.x, (int)v.h.y, (int)v.h.z, (int)v.h.w};
+    }
+};
+
 // Output policies.  ops(n), the operands of column n (at most 8 bytes), are
 // fetched for all the block's columns before the stream and wait in LDS: loads
 // retire in order, so one issued during the stream would wait for the whole
@@ -83,6 +98,21 @@ struct RowsOutEpi {
     __device__ inline void put(const Col& c, const Ops& o, int n, int m, int32_t hi, int32_t low) const {
         if (c.fast) e.put(e.idx(n, m), 0, hi + (low >> 8), (uint32_t)low & 255u, c, e.elt(e.idx(n, m), 0));
         else e.one_ops(n, m, 256 * (int64_t)hi + (int64_t)low, o);
+    }
+};
+// Products whose columns pair up (2i, 2i + 1 -> element i of an output row):
+// each sum reduces to an int16, the odd column's goes to the even one's lane.
+template <class Epi>
+struct RowsOutPair {
+    Epi e;
+    struct Ops { typename Epi::Op o; };
+    using Col = typename Epi::Col;
+    __device__ inline Ops ops(int n) const { return Ops{e.op(n)}; }
+    __device__ inline Col col(const Ops&) const { return Col{}; }
+    __device__ inline void put(const Col&, const Ops& o, int n, int m, int32_t hi, int32_t low) const {
+        const int32_t v = e.stage_with(o.o, n, 256 * (int64_t)hi + (int64_t)low);
+        const int32_t up = dpp_mov<dpp::kXor1>(v);
+        if ((n & 1) == 0) e.emit_one(m, n >> 1, (int16_t)v, (int16_t)up);
     }
 };
 struct RowsNoCol {};

@@ -194,6 +194,11 @@ struct EpiGUSiluPlanes {
     __device__ inline int16_t stage_with(Op sh, int n, int64_t acc) const {
         return clamp_i16_i64(rescale64(acc, (uint8_t)(sh + act_frac), (n & 1) ? up_frac : gate_frac));
     }
+    __device__ inline void emit_one(int m, int i, int16_t g, int16_t u) const {
+        const int32_t h = silu_mul(g, u, silu, silu_len, gate_frac, up_frac, down_in_frac);
+        planes[(size_t)(2 * m) * I + i] = (int8_t)(h >> 8);
+        planes[(size_t)(2 * m + 1) * I + i] = (int8_t)((h & 255) - 128);
+    }
     __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b) const {
         const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};  // (g, u) pairs
         uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
