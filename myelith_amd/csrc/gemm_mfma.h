@@ -510,11 +510,13 @@ __global__ __launch_bounds__(256) void mm_splitk_finish_kernel(unsigned long lon
                                                               Epi epi) {
     const int n = blockIdx.x * 256 + threadIdx.x;
     if (n >= N) return;
+    // the column's operands with the first sum, not behind its clearing store
+    const typename Epi::Ops ops = epi.ops(n);
     for (int m = blockIdx.y; m < M; m += gridDim.y) {
         unsigned long long* p = acc + (size_t)m * N + n;
         const int64_t v = (int64_t)*p;
         *p = 0;
-        epi.one(n, m, v);
+        epi.one_ops(n, m, v, ops);
     }
 }
 

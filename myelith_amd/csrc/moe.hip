@@ -664,7 +664,12 @@ int myl_moe_forward(myl_moe* m, const int16_t* x_dev, uint32_t n_tokens, int16_t
     hipError_t e;
     // router logits (Q8, the LM-head requant), then top-k, gates and counts
     EpiLogits el{m->r_shift, (uint8_t)MYL_MOE_X_FRAC, (uint8_t)MYL_MOE_ROUTER_FRAC, m->logits, E};
-    if ((e = gemv_i8(x_dev, T, H, m->wr, E, H, el, st, mm)) != hipSuccess) return c->hip(e, "moe router");
+    // past 32 tokens the router and the shared expert read the same planes of x
+    const bool x_planes = T > kFragMaxRows && mm_planes_ok(T, H, mm) && mm_planes_ok(T, S, mm);
+    if (x_planes && (e = split_planes(x_dev, T, H, H, mm->planes, st)) != hipSuccess) return c->hip(e, "moe planes");
+    if ((e = x_planes ? mm_planes(mm->planes, T, m->wr, E, H, el, mm, st)
+                      : gemv_i8(x_dev, T, H, m->wr, E, H, el, st, mm)) != hipSuccess)
+        return c->hip(e, "moe router");
     if ((e = hipMemsetAsync(m->counts, 0, (size_t)E * 4, st)) != hipSuccess) return c->hip(e, "moe counts");
     moe_topk_kernel<<<(T + kTopkWaves - 1) / kTopkWaves, kTopkWaves * 64, 0, st>>>(m->logits, T, E, K, m->r_bias, m->exp_lut, (uint32_t)m->exp_len,
                                                      m->ids, m->gates, m->counts);
@@ -750,17 +755,25 @@ int myl_moe_forward(myl_moe* m, const int16_t* x_dev, uint32_t n_tokens, int16_t
         }
     }
     // shared expert: dense products over every token.  With byte planes the
-    // gate/up product's staged epilogue applies the SiLU gate and writes the
-    // down product's planes [2T x S] (in the bytes of Hs).
+    // gate/up product's epilogue applies the SiLU gate and writes the down
+    // product's planes [2T x S] (in the bytes of Hs); up to 32 tokens both stream
+    // the weights, without a SiLU launch between (16 tokens: 99 -> 96 us).
     EpiShift eds{m->sd_s, m->out_frac, (uint8_t)MYL_MOE_DOWN_IN_FRAC, 0, m->Sh, H};
-    if (mm_planes_ok(T, H, mm) && mm_planes_ok(T, S, mm) && T > 64) {
-        int8_t* Sp = reinterpret_cast<int8_t*>(m->Hs);
-        EpiGUSiluPlanes es{m->sgu_s, (uint8_t)MYL_MOE_X_FRAC, (uint8_t)MYL_MOE_GATE_FRAC, (uint8_t)MYL_MOE_UP_FRAC,
-                           (uint8_t)MYL_MOE_DOWN_IN_FRAC, m->silu, (uint32_t)m->silu_len, Sp, S};
-        if ((e = split_planes(x_dev, T, H, H, mm->planes, st)) != hipSuccess) return c->hip(e, "shared planes");
+    int8_t* Sp = reinterpret_cast<int8_t*>(m->Hs);
+    const EpiGUSiluPlanes es{m->sgu_s, (uint8_t)MYL_MOE_X_FRAC, (uint8_t)MYL_MOE_GATE_FRAC, (uint8_t)MYL_MOE_UP_FRAC,
+                             (uint8_t)MYL_MOE_DOWN_IN_FRAC, m->silu, (uint32_t)m->silu_len, Sp, S};
+    const RowsPlan gu = mm && H % 64 == 0 ? rows_plan(T, 2 * S, H, 1, mm->cus, 0) : RowsPlan{};
+    const RowsPlan dn = gu.S && S % 64 == 0 ? rows_plan(T, H, S, 1, mm->cus, mm->acc ? mm->acc_elems : 0) : RowsPlan{};
+    if (x_planes && (T > 64 || H % 128 == 0)) {
         if ((e = mm_planes_staged(mm->planes, T, m->wgu_s, 2 * S, H, es, mm, st)) != hipSuccess)
             return c->hip(e, "shared gate/up");
         if ((e = mm_planes(Sp, T, m->wd_s, H, S, eds, mm, st)) != hipSuccess) return c->hip(e, "shared down");
+    } else if (dn.S) {
+        if ((e = rows_mm_run<1>(gu, RowsSrcX{x_dev, H}, T, m->wgu_s, 2 * S, H, RowsOutPair<EpiGUSiluPlanes>{es}, st)) !=
+            hipSuccess)
+            return c->hip(e, "shared gate/up");
+        if ((e = rows_mm_i8(dn, RowsSrcPlanes{Sp, S}, T, m->wd_s, H, S, eds, mm, st)) != hipSuccess)
+            return c->hip(e, "shared down");
     } else {
         EpiGURows egs{};
         egs.shifts = m->sgu_s; egs.act_frac = MYL_MOE_X_FRAC; egs.gate_frac = MYL_MOE_GATE_FRAC;
