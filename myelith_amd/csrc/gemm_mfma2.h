@@ -299,7 +299,8 @@ __global__ __launch_bounds__(WM_ * WN_ * 64, (Mm2Dims<MB, NB, WM_, WN_, STAGES, 
 // int16 by sink.stage and parked in LDS as a [BR/2 x BN] tile (the K
 // stages are free by then); the block then hands sink.emit(m, i0, v) the 16
 // staged values of columns 2 i0 .. 2 i0 + 15 of row m, for 8-column chunks of
-// N / 2 (N % 16 == 0), so the outputs leave in whole 8-byte pieces.
+// N / 2 (N % 16 == 0), so the outputs leave in whole 8-byte pieces.  The pairs
+// are gate and up of the SiLU gate, whose table the sink names.
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Sink>
 __device__ inline void mm2_staged_tile(const int8_t* __restrict__ Ap, int R2, const int8_t* __restrict__ W, int N, int K,
                                        int r0, int n0, int8_t* lds, const Sink& sink) {
@@ -313,6 +314,19 @@ __device__ inline void mm2_staged_tile(const int8_t* __restrict__ Ap, int R2, co
     mm2_main<MB, NB, WM_, WN_, STAGES, KS>(Ap, R2, W, N, K, 0, K, r0, n0, lds, acc, rs);
     __syncthreads();  // every wave is past its last stage read
     int16_t* tile = reinterpret_cast<int16_t*>(lds);  // [BR / 2][BN]
+    // The gate's table follows the tile in LDS when it fits in whole 1 KiB
+    // loads, which run while the sums are staged: a wave's 64 lookups hit 64
+    // lines, and a 32 KB table does not stay in the vector cache beside the
+    // stores (1500 x 37888 x 3584: 458 us, 465 with lookups through it; the MoE
+    // layer over 3001 tokens 702 and 720).
+    constexpr uint32_t kTileBytes = (uint32_t)(S::BR / 2) * S::BN * 2;
+    const uint32_t lut_bytes = sink.silu_table_len() * 2u;
+    const bool lut_lds = lut_bytes % 1024 == 0 && kTileBytes + lut_bytes <= S::kLds && ((uintptr_t)sink.silu_table() & 15) == 0;
+    int8_t* lut_l = lds + kTileBytes;
+    if (lut_lds)
+        for (uint32_t o = (uint32_t)wave * 1024u; o < lut_bytes; o += S::kThreads * 16u)
+            __builtin_amdgcn_global_load_lds((const void*)(reinterpret_cast<const int8_t*>(sink.silu_table()) + o + lane * 16),
+                                             (lds_void*)(lut_l + o), 16, 0, 0);
     // rows and columns past the matrix hold sums of clamped operands; they are
     // staged like the others and never emitted
 #pragma unroll
@@ -339,16 +353,21 @@ __device__ inline void mm2_staged_tile(const int8_t* __restrict__ Ap, int R2, co
             }
         }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the wave's part of the table
     __syncthreads();
     constexpr int kChunks = S::BN / 16;  // 8-column output chunks per tile row
     const int m0 = r0 >> 1, i00 = n0 >> 1;
-    for (int c = threadIdx.x; c < (S::BR / 2) * kChunks; c += S::kThreads) {
-        const int ml = c / kChunks, ic = c % kChunks;  // powers of two
-        const int m = m0 + ml, i0 = i00 + ic * 8;
-        if (2 * m >= R2 || 2 * i0 >= N) continue;
-        const uint4* src = reinterpret_cast<const uint4*>(tile + ml * S::BN + ic * 16);
-        sink.emit(m, i0, src[0], src[1]);
-    }
+    auto emit_all = [&](const int16_t* lut) {
+        for (int c = threadIdx.x; c < (S::BR / 2) * kChunks; c += S::kThreads) {
+            const int ml = c / kChunks, ic = c % kChunks;  // powers of two
+            const int m = m0 + ml, i0 = i00 + ic * 8;
+            if (2 * m >= R2 || 2 * i0 >= N) continue;
+            const uint4* src = reinterpret_cast<const uint4*>(tile + ml * S::BN + ic * 16);
+            sink.emit(m, i0, src[0], src[1], lut);
+        }
+    };
+    if (lut_lds) emit_all(reinterpret_cast<const int16_t*>(lut_l));
+    else emit_all(sink.silu_table());
 }
 
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class Epi>
@@ -573,7 +592,11 @@ struct SinkGroupedStaged {
     __device__ inline Col col(int n) const { return epi.col(e, n); }
     __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return epi.stage(c, u, r); }
     __device__ inline int16_t stage64(int n, int64_t v) const { return epi.stage64(e, n, v); }
-    __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b) const { epi.emit(e, row0 + m, i0, a, b); }
+    __device__ inline const int16_t* silu_table() const { return epi.silu; }
+    __device__ inline uint32_t silu_table_len() const { return epi.silu_len; }
+    __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b, const int16_t* lut) const {
+        epi.emit(e, row0 + m, i0, a, b, lut);
+    }
 };
 
 template <int MB, int NB, int WM_, int WN_, int STAGES, int KS, class EpiG>

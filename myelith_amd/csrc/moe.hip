@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256) void moe_gather_planes_kernel(const int16_t* _
     }
 }
 
-__device__ inline int16_t moe_silu_one(uint32_t gu, const int16_t* __restrict__ silu, uint32_t silu_len) {
+__device__ inline int16_t moe_silu_one(uint32_t gu, const int16_t* silu, uint32_t silu_len) {
     const int16_t g = (int16_t)(gu & 0xFFFFu), u = (int16_t)(gu >> 16);
     const int32_t g_dom = rescale32((int32_t)g, MYL_MOE_GATE_FRAC, MYL_TV_SILU_IN_FRAC);
     const int16_t act = lut_lookup_i16((int16_t)g_dom, silu, silu_len, (int16_t)MYL_TV_SILU_LUT_OFFSET);
@@ -399,12 +399,12 @@ struct EpiExpertGUSiluPlanes {
         const uint8_t frac = (n & 1) ? MYL_MOE_UP_FRAC : MYL_MOE_GATE_FRAC;
         return clamp_i16_i64(rescale64(acc, (uint8_t)(shifts[(size_t)e * n2 + n] + MYL_MOE_X_FRAC), frac));
     }
-    __device__ inline void emit(int, int row, int i0, const uint4& a, const uint4& b) const {
+    __device__ inline void emit(int, int row, int i0, const uint4& a, const uint4& b, const int16_t* lut) const {
         const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};  // (g, u) pairs
         uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const int32_t h = moe_silu_one(w[k], silu, silu_len);
+            const int32_t h = moe_silu_one(w[k], lut, silu_len);
             hi[k >> 2] |= ((uint32_t)(h >> 8) & 0xFFu) << (8 * (k & 3));
             lo[k >> 2] |= ((uint32_t)((h & 255) - 128) & 0xFFu) << (8 * (k & 3));
         }

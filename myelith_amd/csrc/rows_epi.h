@@ -163,7 +163,7 @@ __device__ inline int16_t silu_rescale(int16_t act, int16_t u, uint8_t in_frac, 
 
 // mlp.rs:55-65 for one element: h = clamp(rescale(silu(g) * u, 8 + up_frac,
 // down_in_frac)), silu(g) from the LUT over g in the LUT's input domain.
-__device__ inline int32_t silu_mul(int16_t g, int16_t u, const int16_t* __restrict__ silu, uint32_t silu_len,
+__device__ inline int32_t silu_mul(int16_t g, int16_t u, const int16_t* silu, uint32_t silu_len,
                                    uint8_t gate_frac, uint8_t up_frac, uint8_t down_in_frac) {
     const int32_t g_dom = rescale32((int32_t)g, gate_frac, MYL_TV_SILU_IN_FRAC);
     const int16_t act = lut_lookup_i16((int16_t)g_dom, silu, silu_len, (int16_t)MYL_TV_SILU_LUT_OFFSET);
@@ -199,12 +199,16 @@ struct EpiGUSiluPlanes {
         planes[(size_t)(2 * m) * I + i] = (int8_t)(h >> 8);
         planes[(size_t)(2 * m + 1) * I + i] = (int8_t)((h & 255) - 128);
     }
-    __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b) const {
+    __device__ inline const int16_t* silu_table() const { return silu; }
+    __device__ inline uint32_t silu_table_len() const { return silu_len; }
+    __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b) const { emit(m, i0, a, b, silu); }
+    // lut: the gate's table, here or in LDS
+    __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b, const int16_t* lut) const {
         const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};  // (g, u) pairs
         uint32_t hi[2] = {0, 0}, lo[2] = {0, 0};
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const int32_t h = silu_mul((int16_t)(w[k] & 0xFFFFu), (int16_t)(w[k] >> 16), silu, silu_len, gate_frac,
+            const int32_t h = silu_mul((int16_t)(w[k] & 0xFFFFu), (int16_t)(w[k] >> 16), lut, silu_len, gate_frac,
                                        up_frac, down_in_frac);
             hi[k >> 2] |= ((uint32_t)(h >> 8) & 0xFFu) << (8 * (k & 3));
             lo[k >> 2] |= ((uint32_t)((h & 255) - 128) & 0xFFu) << (8 * (k & 3));
