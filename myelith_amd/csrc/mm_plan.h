@@ -211,6 +211,12 @@ struct RowsPlan {
     int S = 0, P = 0, U = 0, C = 0, csl = 0, ngb = 0;
 };
 
+// With one column per wave and four plane tiles, a unit's LDS adds (17 a wave)
+// outlast its load; long row ranges then go to the plane tiles (151936 x 896 over
+// 24 / 32 rows: 41.3 / 43.2 us here, 37.5 / 41.3 there; 32001 x 896: 15.0 / 15.4
+// and 15.9 / 16.5).
+inline bool rows_short_sums(int M, int U, int ngb, int wbytes) { return wbytes == 1 && M > 16 && U == 1 && ngb > 16; }
+
 // The plan whose busiest block ends first.  A CU streams about 24 KB/us when all
 // do (6.2 TB/s); a K split adds the finish launch (about 4 us) and its 64-bit
 // atomics (about 90 a ns for the chip).  7B down, 13 rows: 8 slices x 32 parts
@@ -226,6 +232,7 @@ inline RowsPlan rows_plan(int M, int N, int K, int wbytes, int cus, size_t acc_e
         const int csl = (C + S - 1) / S, U = (csl + kRowsWaves - 1) / kRowsWaves;
         if (U > umax || (int64_t)(S - 1) * csl >= C) continue;
         const int P = std::min(cus / S, NG), ngb = (NG + P - 1) / P;
+        if (rows_short_sums(M, U, ngb, wbytes)) continue;
         if (ngb > kRowsMaxGroups || (int64_t)ngb * 16 * K * wbytes >= (1ll << 31)) continue;
         const double t = (double)ngb * csl * kRowsUnit / 24200.0 + (S > 1 ? 4.0 + (double)M * N * S / 90000.0 : 0.0);
         if (best.S == 0 || t < best_t) best = RowsPlan{S, P, U, C, csl, ngb}, best_t = t;

@@ -50,6 +50,29 @@ def test_small_moe_all_tokens(backend, T, widths):
         assert np.array_equal(y[t], om.token(xh[t], ro["ids"][t], ro["gates"][t])), t
 
 
+@pytest.mark.parametrize("widths", [(256, 128, 256), (192, 128, 320)])
+@pytest.mark.parametrize("T", [2, 9, 32, 33, 64, 130])
+def test_small_moe_around_the_stream(backend, T, widths):
+    """Token counts on both sides of the weight stream's range (the shared expert
+    with its SiLU fused up to 32 tokens, planes split once past that) and of the
+    expert tiles, with widths that are and are not multiples of 128; a call with
+    other buffers in between."""
+    from myelith_amd.moe import moe_spec
+    H, I, S = widths
+    spec = moe_spec(11, hidden=H, n_experts=8, inter=I, top_k=2, shared_inter=S)
+    case(f"moe around the stream T={T} widths={widths}")
+    gm, om = build(backend, spec, np.arange(8) * -60)
+    x = gm.synth_input(T)
+    xh = x.cpu().numpy()
+    y = gm.forward(x).cpu().numpy()
+    ro = om.route(xh)
+    compare_route(gm.route(T), ro)
+    for t in range(T):
+        assert np.array_equal(y[t], om.token(xh[t], ro["ids"][t], ro["gates"][t])), t
+    gm.forward(gm.synth_input(70))
+    assert np.array_equal(gm.forward(x).cpu().numpy(), y)
+
+
 def test_qwen15_moe_4096_tokens(backend):
     """The Qwen1.5-MoE-A2.7B-shaped layer on 4096 tokens: the whole route
     (ids, gates, counts, offsets, dispatch order) and the output of every

@@ -112,7 +112,8 @@ int main() {
                             // one slice holds 32 (int8) or 64 columns; int16 sums take no slices
                             const int S0 = ((K * wb + 127) / 128 + (wb == 1 ? 31 : 63)) / (wb == 1 ? 32 : 64);
                             CHECK(M < 2 || M > 32 || K * wb < 128 || K >= 65536 || S0 > cus || S0 > 16 ||
-                                      (N + 15) / 16 > kRowsMaxGroups * (cus / S0) || (S0 > 1 && (wb == 2 || (size_t)M * N > ((size_t)4 << 20))),
+                                      (N + 15) / 16 > kRowsMaxGroups * (cus / S0) ||
+                                      (wb == 1 && M > 16 && K <= 1024 && (N + 15) / 16 > 16 * cus) || (S0 > 1 && (wb == 2 || (size_t)M * N > ((size_t)4 << 20))),
                                   "rows plan refused %d %d %d wb %d cus %d", M, N, K, wb, cus);
                             continue;
                         }
