@@ -219,8 +219,10 @@ inline bool rows_short_sums(int M, int U, int ngb, int wbytes) { return wbytes =
 
 // The plan whose busiest block ends first.  A CU streams about 24 KB/us when all
 // do (6.2 TB/s); a K split adds the finish launch (about 4 us) and its 64-bit
-// atomics (about 90 a ns for the chip).  7B down, 13 rows: 8 slices x 32 parts
-// of 7 row groups, all CUs equally busy; the 7B head (9504 groups) needs none.
+// atomics (about 90 a ns for the chip).  7B down: 8 slices x 32 parts of 7 row
+// groups at 2-8 rows, 5 x 51 of 5 at 13-32; the 7B head (9504 groups) needs none.
+// (8 slices at 13 rows measured 19.7 us against 20.7 with 5, in one run where
+// the same plan differed by up to 2.5% between the sides: not taken.)
 inline RowsPlan rows_plan(int M, int N, int K, int wbytes, int cus, size_t acc_elems) {
     RowsPlan best;
     if (M < 2 || M > kFragMaxRows || N < 1 || N >= (1 << 22) || K % 64 != 0 || K * wbytes < 128 || K >= 65536 || cus < 1 || cus > 1024)
