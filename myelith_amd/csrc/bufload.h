@@ -33,5 +33,13 @@ __device__ inline uint2 cload8(__amdgpu_buffer_rsrc_t r, uint32_t off) {
 __device__ inline uint32_t cload4(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, kPreCpol);
 }
+// 16 bytes per lane into LDS (lane l's at p + 16 l).  The whole offset is the
+// lane's: whether a scalar offset counts in the bounds check depends on the
+// descriptor's form, so none is used here.
+typedef __attribute__((address_space(3))) void buf_lds_void;
+template <int CPOL>
+__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t r, buf_lds_void* p, uint32_t off) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, p, 16, (int)off, 0, 0, CPOL);
+}
 
 }  // namespace myl

@@ -31,8 +31,6 @@
 
 namespace myl {
 
-typedef __attribute__((address_space(3))) void rows_lds_void;
-
 // LDS reads and writes done, then the block barrier (a fence would also wait
 // for every load in flight).
 __device__ inline void rows_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -41,7 +39,7 @@ __device__ inline void rows_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_
 // wait for every such load before each of them (they might meet in LDS); here
 // they never do: the loads fill the waves' rings only.  They return nothing,
 // and rows_barrier waits for them.
-__device__ inline uint32_t rows_lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const rows_lds_void*)p; }
+__device__ inline uint32_t rows_lds_addr(const void* p) { return (uint32_t)(uintptr_t)(const buf_lds_void*)p; }
 __device__ inline void rows_add32(uint32_t a, int32_t v) { asm volatile("ds_add_u32 %0, %1" ::"v"(a), "v"(v) : "memory"); }
 __device__ inline void rows_add64(uint32_t a, int64_t v) { asm volatile("ds_add_u64 %0, %1" ::"v"(a), "v"(v) : "memory"); }
 __device__ inline void rows_set32(uint32_t a, int32_t v) { asm volatile("ds_write_b32 %0, %1" ::"v"(a), "v"(v) : "memory"); }
@@ -192,29 +190,24 @@ __global__ __launch_bounds__(kRowsWaves * 64, 2) void rows_mm_kernel(Src src, in
                 araw[u][t][j] = src.load(xr, min(RT == 1 ? (lane & 15) >> 1 : 16 * j + (lane & 15), M - 1),
                                          (cb + u) * KC + 64 * t + 16 * (lane >> 4), u < kn && (cb + u) * KC + 64 * t < K);
     __builtin_amdgcn_sched_barrier(0);
-    // The block's rows through a buffer descriptor.  A unit's LDS image is rows
-    // of 128 bytes whose 16-byte chunk c sits at slot c ^ ((row / 2) % 8) (the
-    // fragment reads of 16 rows then cover all 64 banks once): lane l of load j
-    // fetches, for row 8j + l / 8, the chunk whose slot is l % 8.  Units past
-    // the block's rows or the wave's columns take an offset past the
-    // descriptor, which reads no memory; rows past N and the bytes past K of a
-    // row's last column meet discarded outputs and zero fragments.
+    // The block's rows through a buffer descriptor, one offset per lane
+    // (rows_lane_off, rows_unit_off): the fragment reads of 16 rows then cover all
+    // 64 banks once.  Units past the block's rows or the wave's columns take an
+    // offset past the descriptor, which reads no memory; rows past N and the
+    // bytes past K of a row's last column meet discarded outputs and zero
+    // fragments.
     const int rows_b = min(16 * ngb, N - 16 * g0);
     const __amdgpu_buffer_rsrc_t wr =
         weight_rsrc(reinterpret_cast<const int8_t*>(W) + (size_t)g0 * 16 * rowb, (uint32_t)max(rows_b, 0) * rowb);
     uint32_t voff[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int row = 8 * j + (lane >> 3);
-        voff[j] = (uint32_t)row * rowb + (uint32_t)cb * 128u + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) << 4);
-    }
+    for (int j = 0; j < 2; ++j) voff[j] = rows_lane_off(j, lane, rowb, cb);
     auto issue = [&](int g, int u, int slot) {
         const bool ok = g < ngb && u < kn;
-        const uint32_t so = ok ? (uint32_t)g * 16u * rowb + (uint32_t)u * 128u : 0u;
+        const uint32_t uo = rows_unit_off(g, u, rowb);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (rows_lds_void*)(ring + slot * kRowsUnit + j * 1024), 16,
-                                                     (int)(ok ? voff[j] : 0x7FFFFFF0u), (int)so, 0, kRowsCpol);
+            load_lds16<kRowsCpol>(wr, (buf_lds_void*)(ring + slot * kRowsUnit + j * 1024), ok ? voff[j] + uo : 0x7FFFFFF0u);
     };
 #pragma unroll
     for (int d = 0; d < kRowsRing; ++d) issue(d / U, d % U, d);

@@ -211,6 +211,19 @@ struct RowsPlan {
     int S = 0, P = 0, U = 0, C = 0, csl = 0, ngb = 0;
 };
 
+// Where lane l of load j (of two) of a unit fetches its 16 bytes: the byte offset
+// within the block's rows (rowb bytes each) of row 16 g + 8 j + l / 8 and of the
+// 16-byte chunk whose LDS slot is l % 8 (chunk c of row r sits at slot
+// c ^ ((r / 2) % 8)) of column cb + u, as the lane's part and the unit's.  Their sum is
+// the load's one offset, checked against the block's bytes: rows past N (the
+// last group of N % 16 != 0) and the bytes past K of the last row's last
+// column lie past them and read no memory.
+constexpr uint32_t rows_lane_off(int j, int lane, uint32_t rowb, int cb) {
+    const int row = 8 * j + (lane >> 3);
+    return (uint32_t)row * rowb + (uint32_t)cb * 128u + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) << 4);
+}
+constexpr uint32_t rows_unit_off(int g, int u, uint32_t rowb) { return (uint32_t)g * 16u * rowb + (uint32_t)u * 128u; }
+
 // With one column per wave and four plane tiles, a unit's LDS adds (17 a wave)
 // outlast its load; long row ranges then go to the plane tiles (151936 x 896 over
 // 24 / 32 rows: 41.3 / 43.2 us here, 37.5 / 41.3 there; 32001 x 896: 15.0 / 15.4

@@ -126,6 +126,37 @@ int main() {
                         CHECK(p.S == 1 || (wb == 1 && (size_t)M * N <= ((size_t)4 << 20)), "rows split beyond the accumulator");
                         CHECK((long)p.ngb * 16 * K * wb < (1l << 31), "rows descriptor");
                     }
+    // the stream's offsets: in the block's bytes whole and once each (rows and
+    // columns of the matrix), or past them whole, where the descriptor reads nothing
+    for (int wb = 1; wb <= 2; ++wb)
+        for (int N : {1, 15, 16, 60, 100, 1000})
+            for (int K : {128, 192, 448, 896, 4160}) {
+                const RowsPlan p = rows_plan(5, N, K, wb, 16, (size_t)4 << 20);
+                if (p.S == 0) continue;
+                const uint32_t rowb = (uint32_t)K * wb;
+                const int NG = (N + 15) / 16;
+                std::vector<int> got((size_t)N * rowb / 16, 0);
+                for (int b = 0; b < p.S * p.P; ++b) {
+                    const int sl = b / p.P, g0 = (int)((long)(b % p.P) * NG / p.P), g1 = (int)((long)(b % p.P + 1) * NG / p.P);
+                    const int rows = std::min(16 * (g1 - g0), N - 16 * g0);
+                    for (int w = 0; w < kRowsWaves; ++w) {
+                        const int cb = sl * p.csl + w * p.U, kn = std::min(p.U, std::min(p.C, (sl + 1) * p.csl) - cb);
+                        for (int g = 0; g < g1 - g0; ++g)
+                            for (int u = 0; u < kn; ++u)
+                                for (int j = 0; j < 2; ++j)
+                                    for (int l = 0; l < 64; ++l) {
+                                        const uint64_t off = (uint64_t)rows_lane_off(j, l, rowb, cb) + rows_unit_off(g, u, rowb);
+                                        const uint64_t bytes = (uint64_t)rows * rowb;
+                                        CHECK(off + 16 <= bytes || (off >= bytes && off < (1ull << 31)), "rows offset %lu of %lu", off, bytes);
+                                        const int row = 16 * g + 8 * j + l / 8, c = (l % 8) ^ (row / 2 % 8);
+                                        const uint64_t col = 128ull * (cb + u) + 16 * c;
+                                        CHECK(off == row * (uint64_t)rowb + col, "rows place");
+                                        if (off < bytes && col < rowb) ++got[((size_t)(16 * g0 + row) * rowb + col) / 16];
+                                    }
+                    }
+                }
+                for (int v : got) CHECK(v == 1, "rows bytes read %d times", v);
+            }
     CHECK(RowsDims<1>::kLds + 16 * kRowsMaxGroups * 8 <= 160 * 1024 && RowsDims<4>::kLds + 16 * kRowsMaxGroups * 8 <= 160 * 1024, "rows lds");
     // groups of the tile order: the full ones and the last cover the row tiles
     for (int tiles = 1; tiles < 300; ++tiles)
