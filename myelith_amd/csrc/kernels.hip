@@ -4,6 +4,7 @@
 #include "gemm_dispatch.h"
 #include "../../include/myl_theta_v.h"
 #include "ops.h"
+#include "row_walk.h"
 #include "wave.h"
 
 namespace myl {
@@ -441,14 +442,10 @@ __device__ inline uint64_t argmax_key(int32_t v, uint32_t idx) {
 // lengths and strides), which a 16-byte global load accepts.
 typedef int32_t RowQuad __attribute__((ext_vector_type(4), aligned(4)));
 
-// The passes over whole logit rows (argmax, sampling) run one block
-// of 16 waves per row and walk it in segments of kRowSeg values per wave, the
-// block's waves side by side: four 16-byte loads per lane and segment, two
-// segments in flight, 128 KB per block, which is what one CU needs to draw
-// its share of the memory rate with few rows in flight.
-constexpr int kRowThreads = 1024;
-constexpr int kRowWaves = kRowThreads / 64;
-constexpr int kRowSeg = 1024;
+// The passes over whole logit rows (row_walk.h) walk a row with the block's
+// waves side by side: four 16-byte loads per lane and segment, two segments in
+// flight, 128 KB per block, which is what one CU needs to draw its share of the
+// memory rate with few rows in flight.
 
 // Calls full(s, v) for each whole segment s of row[0, n) that falls to this
 // wave, in ascending order (v[q][e] is value i = row_index(s, q, e), ascending
@@ -494,7 +491,7 @@ __device__ inline void row_values(const int32_t* __restrict__ row, int n, const 
             seg(s);
         },
         [&](int i0) {
-            for (int i = i0 + (int)(threadIdx.x & 63); i < n; i += 64) f(i, row[i]);
+            row_tail(i0, n, (int)(threadIdx.x & 63), [&](int i) { f(i, row[i]); });
             seg(i0 / kRowSeg);
         });
 }
@@ -596,13 +593,13 @@ __global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* 
                     }
         },
         [&](int i0) {
-            for (int i = i0 + (tid & 63); i < n; i += 64) {
+            row_tail(i0, n, tid & 63, [&](int i) {
                 const int32_t x = row[i];
                 mx = max(mx, x);
-                if (x < least) continue;
+                if (x < least) return;
                 nm = max(nm, ~x);
                 atomicAdd(&count[(uint32_t)x % kLogBins], 1u);
-            }
+            });
         });
     const int32_t lo = ~block_max_i32_dpp(nm, redm);
     const int32_t m = block_max_i32_dpp(mx, redx);  // the barriers also publish the counts
@@ -798,11 +795,11 @@ __global__ __launch_bounds__(kRowThreads) void sample_cdf_kernel(const int32_t* 
         }
         int pick = n - 1;
         const int g0 = g * gvals, g1 = (int)min((int64_t)n, (int64_t)g0 + gvals);
-        for (int i0 = g0; i0 < g1; i0 += 256) {
+        for (int k0 = 0; k0 < g1 - g0; k0 += 256) {
             int64_t w[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int i = i0 + 4 * lane + e;
+                const int i = row_group_index(g0, k0, lane) + e;
                 w[e] = i < g1 ? (int64_t)row[i] - shift : 0;
             }
             const int64_t loc = w[0] + w[1] + w[2] + w[3];
@@ -817,7 +814,7 @@ __global__ __launch_bounds__(kRowThreads) void sample_cdf_kernel(const int32_t* 
                     acc += w[e];
                     at += thr < acc ? 0 : 1;
                 }
-                pick = i0 + 4 * l + readlane_i32(at, l);
+                pick = row_group_index(g0, k0, l) + readlane_i32(at, l);
                 break;
             }
             base += (int64_t)readlane_u64((uint64_t)sc, 63);
@@ -829,7 +826,7 @@ __global__ __launch_bounds__(kRowThreads) void sample_cdf_kernel(const int32_t* 
         return;
     }
     part = 0;
-    for (int i = tid; i < n; i += kRowThreads) part += weight(row[i]);
+    row_strided(n, tid, [&](int i) { part += weight(row[i]); });
     int64_t total = 0;
     (void)block_scan_i64(part, wt, total);
     if (total <= 0) {  // uniform: an empty or non-positive total keeps the state

@@ -199,6 +199,64 @@ def test_launch_plan_under_asan_and_ubsan(plan_run):
     assert n > 100000
 
 
+ROW_DRIVER = r"""
+#include "row_walk.h"
+#include <cstdio>
+#include <climits>
+#include <vector>
+using namespace myl;
+int main() {
+    long checked = 0, bad = 0;
+    // partial last segments and strided passes: every index once, ascending per
+    // lane, none outside the row, up to the longest row an entry point takes
+    for (int64_t n64 : {1ll, 63ll, 64ll, 65ll, 1023ll, 1025ll, 5000ll, INT_MAX - 2000ll, INT_MAX - 1023ll, INT_MAX - 64ll,
+                        INT_MAX - 63ll, INT_MAX - 1ll, (long long)INT_MAX}) {
+        const int n = (int)n64, i0 = n / kRowSeg * kRowSeg;
+        std::vector<int> got(n - i0, 0);
+        for (int lane = 0; lane < 64; ++lane) {
+            int last = -1;
+            row_tail(i0, n, lane, [&](int i) {
+                ++checked;
+                if (i < i0 || i >= n || i <= last) ++bad;
+                else ++got[i - i0], last = i;
+            });
+        }
+        for (int v : got) bad += v != 1;
+        for (int tid : {0, 1, 511, kRowThreads - 1}) {
+            int64_t want = tid, bad0 = bad;
+            row_strided(n, tid, [&](int i) { bad += bad == bad0 && i != want, want += kRowThreads; });
+            bad += want < n || (want - kRowThreads >= n);
+            ++checked;
+        }
+        // a sampling group: 2^lg segments, the last one of the row
+        for (int lg = 0; lg <= 11; ++lg) {
+            const int gvals = kRowSeg << lg, g0 = (n - 1) / gvals * gvals;
+            const int g1 = (int)(n64 < (int64_t)g0 + gvals ? n64 : (int64_t)g0 + gvals);
+            for (int k0 = 0; k0 < g1 - g0; k0 += 256)
+                for (int lane : {0, 63}) ++checked, bad += row_group_index(g0, k0, lane) + 3 < g0 || row_group_index(g0, k0, lane) < g0 + k0;
+        }
+    }
+    std::printf("checked %ld bad %ld\n", checked, bad);
+    return bad != 0;
+}
+"""
+
+
+def test_row_walks_at_the_longest_rows(tmp_path):
+    """The walks of the logit-row kernels (csrc/row_walk.h) up to rows of
+    2^31 - 1 values, under UndefinedBehaviorSanitizer."""
+    if not _gxx():
+        pytest.skip("g++ absent")
+    src = tmp_path / "rows.cpp"
+    src.write_text(ROW_DRIVER)
+    exe = tmp_path / "rows"
+    subprocess.run([_gxx(), "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=all",
+                    "-I", str(CSRC), str(src), "-o", str(exe)], check=True, capture_output=True, timeout=300)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "runtime error" not in r.stderr, (r.stdout[-500:], r.stderr[-2000:])
+    assert int(re.match(r"checked (\d+) bad 0", r.stdout).group(1)) > 1000
+
+
 def _dims(plan_run) -> dict:
     out = {}
     for line in plan_run.stdout.splitlines():
