@@ -255,4 +255,43 @@ inline RowsPlan rows_plan(int M, int N, int K, int wbytes, int cus, size_t acc_e
     return best;
 }
 
+// ---- the grouped expert products (moe.hip) ----------------------------------
+
+// Byte-plane tiles (tokens x weight rows): 0: 128 x 256 (two 128-byte stages), 1:
+// 128 x 128 (64-byte stages), 2: 64 x 128 (two 128-byte stages), 3: 32 x 64 (three).
+constexpr int moe_tile_tokens(int tile) { return tile == 2 ? 64 : tile == 3 ? 32 : 128; }
+constexpr int moe_tile_rows(int tile) { return tile == 0 ? 256 : tile == 3 ? 64 : 128; }
+
+// Small tiles waste less on experts of few tokens and keep more blocks loading,
+// large ones move fewer operand bytes; the whole 60-expert layer on MI355X, us:
+//   tokens (rows per expert)   16 (1)  100 (7)  400 (27)  1000 (67)  2400 (160)  3001 (200)
+//   tile 0                     157     261      316       426        664         795
+//   tile 2                     125     210      265       379        647         807
+//   tile 3                     114     202      283       444        878
+// Tile 1 only where a K is not a multiple of 128 (k128 false).  R routed rows of E
+// experts.
+constexpr int kMoeRows2 = 14, kMoeRows0 = 180;  // rows per expert from which tiles 2 and 0 are taken
+constexpr int moe_pick_tile(bool k128, int R, int E) {
+    return !k128 ? 1 : R >= kMoeRows0 * E ? 0 : R >= kMoeRows2 * E ? 2 : 3;
+}
+
+// Work items of one grouped product over R routed rows of E experts, N weight
+// rows: sum_e ceil(c_e / tokens) <= floor(R / tokens) + E token tiles.
+constexpr int moe_max_items(int R, int E, int tile, int N) {
+    return (R / moe_tile_tokens(tile) + E) * ((N + moe_tile_rows(tile) - 1) / moe_tile_rows(tile));
+}
+// Both products' (2 I and H weight rows).
+constexpr int moe_work_items(int R, int E, int tile, int I, int H) {
+    return moe_max_items(R, E, tile, 2 * I) + moe_max_items(R, E, tile, H);
+}
+// The most that a call over up to R rows needs: fewer rows take smaller tiles
+// and can need more items, so a table sized for this is not grown again by a
+// smaller call (growing frees and allocates, which a captured call must not).
+inline int moe_work_cap(bool k128, int R, int E, int I, int H) {
+    int most = moe_work_items(R, E, moe_pick_tile(k128, R, E), I, H);
+    for (int b : {kMoeRows2 * E - 1, kMoeRows0 * E - 1})
+        if (k128 && b < R) most = std::max(most, moe_work_items(b, E, moe_pick_tile(true, b, E), I, H));
+    return most;
+}
+
 }  // namespace myl

@@ -540,22 +540,12 @@ int ensure(myl_moe* m, int T) {
     return MYL_OK;
 }
 
-// Byte-plane tile of the grouped expert products: 0: 128 tokens x 256 weight
-// rows (two 128-byte stages), 1: 128 x 128 (64-byte stages), 2: 64 x 128 (two
-// 128-byte stages), 3: 32 x 64 (three).  Small tiles waste less on experts of
-// few tokens and keep more blocks loading, large ones move fewer operand bytes;
-// the whole 60-expert layer on MI355X, us:
-//   tokens (rows per expert)   16 (1)  100 (7)  400 (27)  1000 (67)  2400 (160)  3001 (200)
-//   tile 0                     157     261      316       426        664         795
-//   tile 2                     125     210      265       379        647         807
-//   tile 3                     114     202      283       444        878
-// Tile 1 only where a K is not a multiple of 128.  MYL_MOE_TILE overrides the
-// choice for sweeps.
+// Byte-plane tile of the grouped expert products (mm_plan.h).  MYL_MOE_TILE
+// overrides the choice for sweeps.
 int moe_planes_tile(int H, int I, int R, int E) {
     const bool k128 = H % 128 == 0 && I % 128 == 0;
     const int v = mm_env("MYL_MOE_TILE");
-    if (v >= 0 && v <= 3) return !k128 ? 1 : v;
-    return !k128 ? 1 : R >= 180 * E ? 0 : R >= 14 * E ? 2 : 3;
+    return k128 && v >= 0 && v <= 3 ? v : moe_pick_tile(k128, R, E);
 }
 #define MYL_MOE_TILES(F)                        \
     switch (tile) {                             \
@@ -564,14 +554,12 @@ int moe_planes_tile(int H, int I, int R, int E) {
     case 2: return F(2, 1, 2, 4, 2, 128);       \
     default: return F(1, 1, 2, 2, 3, 128);      \
     }
-int moe_tile_tokens(int tile) {
-#define MYL_MOE_TOKENS(...) Mm2GroupedShape<__VA_ARGS__>::kTokens
-    MYL_MOE_TILES(MYL_MOE_TOKENS)
-}
-int moe_tile_rows(int tile) {
-#define MYL_MOE_ROWS(...) Mm2GroupedShape<__VA_ARGS__>::kRows
-    MYL_MOE_TILES(MYL_MOE_ROWS)
-}
+#define MYL_MOE_DIMS(T, ...) \
+    (moe_tile_tokens(T) == Mm2GroupedShape<__VA_ARGS__>::kTokens && moe_tile_rows(T) == Mm2GroupedShape<__VA_ARGS__>::kRows)
+static_assert(MYL_MOE_DIMS(0, 4, 2, 2, 4, 2, 128) && MYL_MOE_DIMS(1, 2, 2, 4, 2, 3, 64) &&
+                  MYL_MOE_DIMS(2, 2, 1, 2, 4, 2, 128) && MYL_MOE_DIMS(3, 1, 1, 2, 2, 3, 128),
+              "the plan's tile sizes");
+#undef MYL_MOE_DIMS
 template <class EpiG>
 hipError_t moe_grouped(int tile, const int8_t* Ap, const int8_t* W, size_t w_stride, int N, int K, const int* offsets,
                        const MmWork* work, const int* nwork, int maxwork, const EpiG& epi, hipStream_t st) {
@@ -587,14 +575,8 @@ hipError_t moe_grouped_staged(int tile, const int8_t* Ap, const int8_t* W, size_
     MYL_MOE_TILES(MYL_MOE_STAGED)
 }
 #undef MYL_MOE_TILES
-#undef MYL_MOE_TOKENS
-#undef MYL_MOE_ROWS
 #undef MYL_MOE_PLAIN
 #undef MYL_MOE_STAGED
-
-// Work items of a grouped product over R routed rows of E experts in token
-// tiles of bm: sum_e ceil(c_e / bm) <= floor(R / bm) + E token tiles.
-int moe_max_items(int R, int E, int bm, int nt) { return (R / bm + E) * nt; }
 
 // Work table of a grouped product: (expert, m-tile, n-tile), m fastest.
 void work_table(const std::vector<int32_t>& counts, int bm, int bn, int N, std::vector<MmWork>& out) {
@@ -685,15 +667,15 @@ int myl_moe_forward(myl_moe* m, const int16_t* x_dev, uint32_t n_tokens, int16_t
         int bm_log = 0;
         while ((1 << bm_log) < bm) ++bm_log;
         const int nt1 = (2 * I + bn - 1) / bn, nt2 = (H + bn - 1) / bn;
-        const int max1 = moe_max_items(R, E, bm, nt1), max2 = moe_max_items(R, E, bm, nt2);
+        const int max1 = moe_max_items(R, E, tile, 2 * I), max2 = moe_max_items(R, E, tile, H);
         if (max1 + max2 > m->work_cap) {
+            const int cap = std::max(max1 + max2, moe_work_cap(H % 128 == 0 && I % 128 == 0, R, E, I, H));
             (void)hipStreamSynchronize(st);
             if (m->work) (void)hipFree(m->work);
             m->work = nullptr;
             m->work_cap = 0;
-            if (hipMalloc(&m->work, (size_t)(max1 + max2) * sizeof(MmWork)) != hipSuccess)
-                return c->fail(MYL_E_NOMEM, "moe work");
-            m->work_cap = max1 + max2;
+            if (hipMalloc(&m->work, (size_t)cap * sizeof(MmWork)) != hipSuccess) return c->fail(MYL_E_NOMEM, "moe work");
+            m->work_cap = cap;
         }
         moe_plan_kernel<<<1, kPlanThreads, 0, st>>>(m->counts, E, bm_log, bn, nt1, nt2, max1, m->offsets, m->work, m->nwork);
         moe_dispatch_kernel<<<E, 256, 0, st>>>(m->ids, T, K, m->offsets, m->list_tok, m->slotpos);

@@ -158,6 +158,23 @@ int main() {
                 for (int v : got) CHECK(v == 1, "rows bytes read %d times", v);
             }
     CHECK(RowsDims<1>::kLds + 16 * kRowsMaxGroups * 8 <= 160 * 1024 && RowsDims<4>::kLds + 16 * kRowsMaxGroups * 8 <= 160 * 1024, "rows lds");
+    // the expert products' work table: one sized for R rows holds every call of
+    // fewer rows, whatever their tile
+    for (int E : {1, 8, 60, 256})
+        for (int I : {128, 192, 1408})
+            for (int H : {256, 448, 2048}) {
+                const bool k128 = H % 128 == 0 && I % 128 == 0;
+                int most = 0;
+                for (int R = 1; R < 200 * E + 500; R += R < 16 * E + 64 ? 1 : 37) {
+                    const int tile = moe_pick_tile(k128, R, E), items = moe_work_items(R, E, tile, I, H);
+                    CHECK(tile >= 0 && tile <= 3 && (k128 || tile == 1), "moe tile %d", tile);
+                    most = std::max(most, items);
+                    CHECK(moe_work_cap(k128, R, E, I, H) >= most, "moe table E %d I %d H %d R %d: %d < %d", E, I, H, R,
+                          moe_work_cap(k128, R, E, I, H), most);
+                }
+            }
+    CHECK(moe_work_items(64, 60, moe_pick_tile(true, 64, 60), 1408, 2048) >
+              moe_work_items(16384, 60, moe_pick_tile(true, 16384, 60), 1408, 2048), "small tiles need more items");
     // groups of the tile order: the full ones and the last cover the row tiles
     for (int tiles = 1; tiles < 300; ++tiles)
         for (int want = 0; want < 9; ++want) {
