@@ -100,15 +100,17 @@ struct PlaneRescale {
     }
 };
 
-// rshift_round128((256 u + r) * mult, shift) for shifts 39..70: the product is
-// 256 V + (r mult & 255) with V = u mult + (r mult >> 8), |V| < 2^62, and the
-// result fits 32 bits.
+// rshift_round128((256 u + r) * mult, shift) for shifts 9..70: the product is
+// 256 V + (r mult & 255) with V = u mult + (r mult >> 8), |V| < 2^62, so the
+// result is one 64-bit shift of V by t = shift - 8 with the low byte as the
+// sticky bits (wide).  It fits 32 bits from shift 39 on only; every caller of
+// the smaller shifts clamps it (clamped).
 struct PlaneMult {
     int32_t mult;
     uint32_t t, fast;
     int64_t base;
     MYL_FN PlaneMult of(int32_t mult, uint8_t shift) {
-        const bool ok = shift >= 39 && shift <= 70;
+        const bool ok = shift >= 9 && shift <= 70;
         const uint32_t t = ok ? (uint32_t)shift - 8u : 31u;
         return PlaneMult{mult, t, ok ? 1u : 0u, (int64_t)((1ull << (t - 1)) - 1u)};
     }
@@ -120,12 +122,16 @@ struct PlaneMult {
         const uint32_t t = ok ? (uint32_t)shift - 8u : 1u;
         return PlaneMult{ok ? (int32_t)mult : 0, t, ok ? 1u : 0u, (int64_t)((1ull << (t - 1)) - 1u)};
     }
-    MYL_MEM int32_t operator()(int32_t u, uint32_t r) const {
+    MYL_MEM int64_t wide(int32_t u, uint32_t r) const {
         const int64_t rm = (int64_t)(int32_t)r * mult;
         const int64_t v = (int64_t)u * mult + (int64_t)(int32_t)(rm >> 8);
         const uint32_t c = ((uint32_t)(v >> t) & 1u) | ((uint32_t)rm & 255u);
-        return (int32_t)((v + base + (int64_t)(c < 1u ? c : 1u)) >> t);
+        return (v + base + (int64_t)(c < 1u ? c : 1u)) >> t;
     }
+    // the low word
+    MYL_MEM int32_t operator()(int32_t u, uint32_t r) const { return (int32_t)wide(u, r); }
+    // clamp_i16 of the result
+    MYL_MEM int16_t clamped(int32_t u, uint32_t r) const { return clamp_i16_i64(wide(u, r)); }
 };
 
 // rescale64 of a value |v| <= 2^30 followed by a clamp to [-2^16, 2^16] or

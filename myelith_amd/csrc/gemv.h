@@ -383,7 +383,7 @@ struct EpiMult {
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
     __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const {
-        (out + i)[lo] = clamp_i16(c(u, r));
+        (out + i)[lo] = c.clamped(u, r);
     }
     template <int R, int MT>
     __device__ inline void apply(int row0, int N, int M, int lane, const int64_t (&tot)[R][MT]) const {

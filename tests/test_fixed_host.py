@@ -374,12 +374,18 @@ int main() {
         for (int k = 0; k < 3000; ++k) {
             const int32_t mult = k % 3 ? (int32_t)next() : ms[(k / 3) % 10];
             const PlaneMult p = PlaneMult::of(mult, (uint8_t)s);
+            if (p.fast != (s >= 9 && s <= 70)) ++bad;  // the published sweep's shifts are 20..40
             if (!p.fast) continue;
             int64_t hi, low;
             parts(k, s - (k % 7 ? 29 : 30), &hi, &low);
             const int32_t l32 = (int32_t)low;
             ++n, ++fast;
-            bad += clamp_i16(p((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u)) != mult_general(hi * 256 + low, mult, (uint8_t)s);
+            bad += p.clamped((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u) != mult_general(hi * 256 + low, mult, (uint8_t)s);
+            // sums of a few units times small multipliers: results inside the clamp at the small shifts
+            const int64_t sum = (int64_t)(next() % (1u << (k % 20 + 1))) - (1 << (k % 20)), sm_ = mult >> (31 - k % 24);
+            const PlaneMult q = PlaneMult::of((int32_t)sm_, (uint8_t)s);
+            ++n;
+            bad += q.clamped((int32_t)(sum >> 8), (uint32_t)sum & 255u) != mult_general(sum, (int32_t)sm_, (uint8_t)s);
         }
     printf("checked %ld (plane sums %ld), mismatches %ld\n", n, fast, bad);
     return bad != 0 || fast < 100000;
