@@ -390,6 +390,9 @@ struct SinkEpi {
     using Col = typename Epi::Col;
     using Elt = typename Epi::Elt;
     __device__ inline Col col(int n) const { return e.col(n); }
+    __device__ inline auto ops(int n) const { return e.ops(n); }
+    template <class Ops>
+    __device__ inline void put64(int n, int m, int64_t v, const Ops& o) const { e.one_ops(n, m, v, o); }
     __device__ inline Elt elt(size_t i, uint32_t lo) const { return e.elt(i, lo); }
     __device__ inline size_t idx(int n, int m) const { return e.idx(n, m); }
     __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt& x) const { e.put(i, lo, u, r, c, x); }
@@ -403,6 +406,8 @@ struct SinkAtomic {
     struct Col { uint32_t fast; };
     struct Elt {};
     __device__ inline Col col(int) const { return Col{1}; }
+    __device__ inline Elt ops(int) const { return Elt{}; }
+    __device__ inline void put64(int n, int m, int64_t v, const Elt&) const { (*this)(n, m, v); }
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldn + n; }
     __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col&, const Elt&) const {
@@ -483,6 +488,9 @@ struct SinkGrouped {
     using Col = typename EpiG::Col;
     using Elt = EpiNoElt;
     __device__ inline Col col(int n) const { return epi.col(e, n); }
+    __device__ inline auto ops(int n) const { return epi.ops(e, n); }
+    template <class Ops>
+    __device__ inline void put64(int n, int m, int64_t v, const Ops& o) const { epi.one_ops(n, row0 + m, v, o); }
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return epi.idx(n, row0 + m); }
     __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const { epi.put(i, lo, u, r, c); }

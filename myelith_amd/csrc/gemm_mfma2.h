@@ -240,20 +240,22 @@ __device__ inline void mm2_emit(const v16i32_t (&acc)[MB][NB], const int32_t (&r
 }
 
 // The same from 64-bit sums (a column's shift or K outside the 32-bit range),
-// one register pair at a time.
+// one register pair at a time.  The column's operands are loaded once: behind
+// the stores, which may alias them, they cost a memory round trip per value.
 template <int MB, int NB, class Sink>
 __device__ inline void mm2_emit64(const v16i32_t (&acc)[MB][NB], const int32_t (&rs)[NB], int R2, int N, int arow0,
                                   int nw0, int lane, const Sink& sink) {
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
         const int n = nw0 + j * 32 + (lane & 31);
+        const auto ops = sink.ops(min(n, N - 1));
 #pragma unroll
         for (int i = 0; i < MB; ++i) {
-#pragma unroll 1
+#pragma unroll 2
             for (int r = 0; r < 16; r += 2) {
                 const int64_t v = (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128;
                 const int m = ((arow0 + i * 32 + mm2_row(r)) >> 1) + 2 * (lane >> 5);
-                if (2 * m < R2 && n < N) sink(n, m, v);
+                if (2 * m < R2 && n < N) sink.put64(n, m, v, ops);
             }
         }
     }

@@ -419,10 +419,12 @@ struct EpiExpertDown {
     const uint8_t* out_frac;  // [H]
     int H;
     int16_t* out;             // [rows x H]
-    __device__ inline void one(int e, int n, int row, int64_t acc) const {
-        out[(size_t)row * H + n] = clamp_i16_i64(
-            rescale64(acc, (uint8_t)(shifts[(size_t)e * H + n] + MYL_MOE_DOWN_IN_FRAC), out_frac[n]));
+    struct Ops { uint8_t sh, of; };
+    __device__ inline Ops ops(int e, int n) const { return Ops{shifts[(size_t)e * H + n], out_frac[n]}; }
+    __device__ inline void one_ops(int n, int row, int64_t acc, const Ops& o) const {
+        out[(size_t)row * H + n] = clamp_i16_i64(rescale64(acc, (uint8_t)(o.sh + MYL_MOE_DOWN_IN_FRAC), o.of));
     }
+    __device__ inline void one(int e, int n, int row, int64_t acc) const { one_ops(n, row, acc, ops(e, n)); }
     using Col = PlaneRescale;
     __device__ inline Col col(int e, int n) const {
         return Col::of((uint8_t)(shifts[(size_t)e * H + n] + MYL_MOE_DOWN_IN_FRAC), out_frac[n]);
