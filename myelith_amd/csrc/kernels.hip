@@ -449,8 +449,8 @@ typedef int32_t RowQuad __attribute__((ext_vector_type(4), aligned(4)));
 
 // Calls full(s, v) for each whole segment s of row[0, n) that falls to this
 // wave, in ascending order (v[q][e] is value i = row_index(s, q, e), ascending
-// in q and e), then tail(i0) on the wave whose turn the partial last segment
-// [i0, n) is.
+// in q and e), then tail(i0) on every wave for the partial last segment [i0, n),
+// whose values the block's threads share (row_tail).
 __device__ inline int row_index(int s, int q, int e) {
     return s * kRowSeg + q * 256 + (int)(threadIdx.x & 63) * 4 + e;
 }
@@ -473,12 +473,12 @@ __device__ inline void row_segments(const int32_t* __restrict__ row, int n, cons
         RowQuad a[4];
         load(a, s);
         full(s, a);
-        s += kRowWaves;
     }
-    if (s == nfull && s * kRowSeg < n) tail(s * kRowSeg);
+    if (nfull * kRowSeg < n) tail(nfull * kRowSeg);
 }
 
-// The same with f(i, v) for every value and seg(s) after each segment.
+// The same with f(i, v) for every value and seg(s) after each segment (on each
+// wave that had values of it).
 template <class F, class Seg>
 __device__ inline void row_values(const int32_t* __restrict__ row, int n, const F& f, const Seg& seg) {
     row_segments(
@@ -491,8 +491,8 @@ __device__ inline void row_values(const int32_t* __restrict__ row, int n, const 
             seg(s);
         },
         [&](int i0) {
-            row_tail(i0, n, (int)(threadIdx.x & 63), [&](int i) { f(i, row[i]); });
-            seg(i0 / kRowSeg);
+            row_tail(i0, n, (int)threadIdx.x, kRowThreads, [&](int i) { f(i, row[i]); });
+            if ((int)(threadIdx.x & ~63u) < n - i0) seg(i0 / kRowSeg);
         });
 }
 
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* 
                     }
         },
         [&](int i0) {
-            row_tail(i0, n, tid & 63, [&](int i) {
+            row_tail(i0, n, tid, kRowThreads, [&](int i) {
                 const int32_t x = row[i];
                 mx = max(mx, x);
                 if (x < least) return;

@@ -15,10 +15,13 @@ constexpr int kRowThreads = 1024;
 constexpr int kRowWaves = kRowThreads / 64;
 constexpr int kRowSeg = 1024;
 
-// f(i) for lane `lane`'s values of the partial last segment [i0, n).
+// f(i) for thread tid's values of the partial last segment [i0, n), spread over
+// all of the block's threads: at most one each for a block of kRowThreads, so
+// the segment costs one memory latency (one wave alone takes up to 16, which is
+// all the time of a row of less than one segment).
 template <class F>
-constexpr void row_tail(int i0, int n, int lane, const F& f) {
-    for (int k = lane; k < n - i0; k += 64) f(i0 + k);
+constexpr void row_tail(int i0, int n, int tid, int threads, const F& f) {
+    for (int k = tid; k < n - i0; k += threads) f(i0 + k);
 }
 
 // f(i) for every kRowThreads-th value from tid on.

@@ -225,20 +225,23 @@ using namespace myl;
 int main() {
     long checked = 0, bad = 0;
     // partial last segments and strided passes: every index once, ascending per
-    // lane, none outside the row, up to the longest row an entry point takes
+    // thread, none outside the row, up to the longest row an entry point takes
     for (int64_t n64 : {1ll, 63ll, 64ll, 65ll, 1023ll, 1025ll, 5000ll, INT_MAX - 2000ll, INT_MAX - 1023ll, INT_MAX - 64ll,
                         INT_MAX - 63ll, INT_MAX - 1ll, (long long)INT_MAX}) {
         const int n = (int)n64, i0 = n / kRowSeg * kRowSeg;
-        std::vector<int> got(n - i0, 0);
-        for (int lane = 0; lane < 64; ++lane) {
-            int last = -1;
-            row_tail(i0, n, lane, [&](int i) {
-                ++checked;
-                if (i < i0 || i >= n || i <= last) ++bad;
-                else ++got[i - i0], last = i;
-            });
+        for (int threads : {kRowThreads, 256}) {
+            std::vector<int> got(n - i0, 0);
+            for (int tid = 0; tid < threads; ++tid) {
+                int last = -1, took = 0;
+                row_tail(i0, n, tid, threads, [&](int i) {
+                    ++checked, ++took;
+                    if (i < i0 || i >= n || i <= last) ++bad;
+                    else ++got[i - i0], last = i;
+                });
+                bad += took > kRowSeg / threads;  // the segment is shared by the whole block
+            }
+            for (int v : got) bad += v != 1;
         }
-        for (int v : got) bad += v != 1;
         for (int tid : {0, 1, 511, kRowThreads - 1}) {
             int64_t want = tid, bad0 = bad;
             row_strided(n, tid, [&](int i) { bad += bad == bad0 && i != want, want += kRowThreads; });
