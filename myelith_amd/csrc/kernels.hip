@@ -496,30 +496,44 @@ __device__ inline void row_values(const int32_t* __restrict__ row, int n, const 
         });
 }
 
+// f(i, v) for every value of a short row, ascending per thread.
+template <class F>
+__device__ inline void row_short(const int32_t* __restrict__ row, int n, const F& f) {
+    row_quads(
+        n, (int)threadIdx.x,
+        [&](int i) {
+            const RowQuad v = *reinterpret_cast<const RowQuad*>(row + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f(i + e, v[e]);
+        },
+        [&](int i) { f(i, row[i]); });
+}
+
 // Bound by reading the row: 600 x 152064 values in 61 us (6.0 TB/s), 24 in 7.8
 // us; 256 threads with one load in flight each and 64-bit keys throughout took
 // 280 and 73 us.  A thread keeps its first maximum (ascending i, so strictly
 // greater wins); keys order the threads'.
-__global__ __launch_bounds__(kRowThreads) void argmax_kernel(const int32_t* __restrict__ v, int n, int ldv,
-                                                            int64_t* __restrict__ out) {
-    __shared__ uint64_t red[kRowWaves];
+template <bool SHORT>
+__global__ __launch_bounds__(SHORT ? kRowShortThreads : kRowThreads) void argmax_kernel(const int32_t* __restrict__ v, int n,
+                                                                                       int ldv, int64_t* __restrict__ out) {
+    constexpr int kWaves = (SHORT ? kRowShortThreads : kRowThreads) / 64;
+    __shared__ uint64_t red[kWaves];
     const int32_t* row = v + (size_t)blockIdx.x * ldv;
     int32_t best = INT32_MIN;
     int at = -1;
-    row_values(
-        row, n,
-        [&](int i, int32_t x) {
-            const bool up = x > best || at < 0;
-            best = up ? x : best;
-            at = up ? i : at;
-        },
-        [](int) {});
+    auto take = [&](int i, int32_t x) {
+        const bool up = x > best || at < 0;
+        best = up ? x : best;
+        at = up ? i : at;
+    };
+    if constexpr (SHORT) row_short(row, n, take);
+    else row_values(row, n, take, [](int) {});
     const uint64_t key = wave_max_u64(at < 0 ? 0 : argmax_key(best, (uint32_t)at));
     const int lane = threadIdx.x & 63;
     if (lane == 0) red[threadIdx.x >> 6] = key;
     __syncthreads();
     if (threadIdx.x >= 64) return;
-    const uint64_t m = wave_max_u64(lane < kRowWaves ? red[lane] : 0);
+    const uint64_t m = wave_max_u64(lane < kWaves ? red[lane] : 0);
     if (lane == 0) out[blockIdx.x] = (int64_t)(0xFFFFFFFFu - (uint32_t)(m & 0xFFFFFFFFu));
 }
 
@@ -542,6 +556,17 @@ __global__ __launch_bounds__(kRowThreads) void argmax_kernel(const int32_t* __re
 // Constant rows, rows wider than the ring and half-masked rows take 76, 150 and
 // 83 us (186, 200 and 293 before).
 constexpr int kLogBins = 8192;
+
+// One value's term of S, `below` under the maximum; the result from S.
+__device__ inline int64_t logsoftmax_term(uint64_t below, const int16_t* lut, uint32_t lut_len) {
+    const uint64_t d = below << (MYL_TV_EXP_INPUT_FRAC - MYL_TV_LOGIT_FRAC_BITS);
+    return d < lut_len ? (int64_t)lut[d] : 0;
+}
+__device__ inline int64_t logsoftmax_at(const int32_t* row, int n, int64_t target, int32_t m, int64_t S) {
+    if (target < 0 || target >= n) return 0;
+    return ((int64_t)row[target] - (int64_t)m) * 1024 - ln_q16_of_sum(S < 1 ? 1u : (uint64_t)S);
+}
+
 __global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* __restrict__ z, int n, int ldz,
                                                                 const int16_t* __restrict__ lut, uint32_t lut_len,
                                                                 const int64_t* __restrict__ targets,
@@ -604,10 +629,7 @@ __global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* 
     const int32_t lo = ~block_max_i32_dpp(nm, redm);
     const int32_t m = block_max_i32_dpp(mx, redx);  // the barriers also publish the counts
     constexpr uint32_t sh = MYL_TV_EXP_INPUT_FRAC - MYL_TV_LOGIT_FRAC_BITS;
-    auto term = [&](uint64_t below) -> int64_t {
-        const uint64_t d = below << sh;
-        return d < lut_len ? (int64_t)lut[d] : 0;
-    };
+    auto term = [&](uint64_t below) { return logsoftmax_term(below, lut, lut_len); };
     int64_t s = 0;
     if ((int64_t)m - (int64_t)lo < kLogBins && lut_len <= ((uint32_t)kLogBins << sh)) {
         for (uint32_t k = tid; k < (uint32_t)kLogBins && ((uint64_t)k << sh) < lut_len; k += kRowThreads)
@@ -630,23 +652,60 @@ __global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* 
     __syncthreads();
     if (tid >= 64) return;
     const int64_t S = wave_sum_i64(tid < kRowWaves ? red64[tid] : 0);
-    if (tid == 0) {
-        const int64_t t = targets[blockIdx.x];
-        int64_t lp = 0;
-        if (t >= 0 && t < n)
-            lp = ((int64_t)row[t] - (int64_t)m) * 1024 - ln_q16_of_sum(S < 1 ? 1u : (uint64_t)S);
-        out[blockIdx.x] = lp;
-    }
+    if (tid == 0) out[blockIdx.x] = logsoftmax_at(row, n, targets[blockIdx.x], m, S);
+}
+
+// The same for short rows: the row is read twice, the second time from the
+// cache, which costs less than clearing and summing the counters.  Past
+// kLogTabRow values, the table's first entries (32 logit units) wait in LDS: 2000
+// rows of 1000 / 8192 values 7.2 / 24.6 us (8.1 with the table for the first; 26.1
+// for the second with the table copied before the row is read).
+constexpr int kLogTab = 2048, kLogTabRow = 1024;
+__global__ __launch_bounds__(kRowShortThreads) void logsoftmax_short_kernel(const int32_t* __restrict__ z, int n, int ldz,
+                                                                           const int16_t* __restrict__ lut, uint32_t lut_len,
+                                                                           const int64_t* __restrict__ targets,
+                                                                           int64_t* __restrict__ out) {
+    constexpr int kWaves = kRowShortThreads / 64;
+    __shared__ int32_t redx[kWaves];
+    __shared__ int64_t red64[kWaves];
+    __shared__ int16_t tab[kLogTab];
+    const int32_t* row = z + (size_t)blockIdx.x * ldz;
+    const int tid = threadIdx.x;
+    const uint64_t nt = n > kLogTabRow ? kLogTab : 0;
+    constexpr int kTabEach = kLogTab / kRowShortThreads;
+    int16_t own[kTabEach];  // the thread's entries, on their way while the row is read
+    if (nt)
+#pragma unroll
+        for (int j = 0; j < kTabEach; ++j) own[j] = (int16_t)logsoftmax_term((uint64_t)(j * kRowShortThreads + tid), lut, lut_len);
+    int32_t mx = INT32_MIN;
+    row_short(row, n, [&](int, int32_t x) { mx = max(mx, x); });
+    if (nt)
+#pragma unroll
+        for (int j = 0; j < kTabEach; ++j) tab[j * kRowShortThreads + tid] = own[j];
+    const int32_t m = block_max_i32_dpp(mx, redx);  // its barrier also publishes the table
+    int64_t s = 0;
+    row_short(row, n, [&](int, int32_t x) {
+        const uint64_t below = (uint64_t)((int64_t)m - (int64_t)x);
+        s += below < nt ? (int64_t)tab[below] : logsoftmax_term(below, lut, lut_len);
+    });
+    s = wave_sum_i64(s);
+    if ((tid & 63) == 0) red64[tid >> 6] = s;
+    __syncthreads();
+    if (tid >= 64) return;
+    const int64_t S = wave_sum_i64(tid < kWaves ? red64[tid] : 0);
+    if (tid == 0) out[blockIdx.x] = logsoftmax_at(row, n, targets[blockIdx.x], m, S);
 }
 
 hipError_t logsoftmax(const int32_t* z, int M, int n, int ldz, const int16_t* lut, int lut_len, const int64_t* targets,
                       int64_t* out, hipStream_t st) {
-    logsoftmax_kernel<<<M, kRowThreads, 0, st>>>(z, n, ldz, lut, (uint32_t)lut_len, targets, out);
+    if (row_short_logsoftmax(M, n)) logsoftmax_short_kernel<<<M, kRowShortThreads, 0, st>>>(z, n, ldz, lut, (uint32_t)lut_len, targets, out);
+    else logsoftmax_kernel<<<M, kRowThreads, 0, st>>>(z, n, ldz, lut, (uint32_t)lut_len, targets, out);
     return hipGetLastError();
 }
 
 hipError_t argmax(const int32_t* v, int M, int n, int ldv, int64_t* out, hipStream_t st) {
-    argmax_kernel<<<M, kRowThreads, 0, st>>>(v, n, ldv, out);
+    if (row_short_argmax(M, n)) argmax_kernel<true><<<M, kRowShortThreads, 0, st>>>(v, n, ldv, out);
+    else argmax_kernel<false><<<M, kRowThreads, 0, st>>>(v, n, ldv, out);
     return hipGetLastError();
 }
 

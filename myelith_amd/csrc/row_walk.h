@@ -15,6 +15,28 @@ constexpr int kRowThreads = 1024;
 constexpr int kRowWaves = kRowThreads / 64;
 constexpr int kRowSeg = 1024;
 
+// Short rows (argmax, log-softmax) take blocks of kRowShortThreads threads
+// instead, which step over them by four values a thread: with more rows than
+// CUs, blocks of 16 waves wait for each other (and the log-softmax's counters cost
+// more than a second read of the row); with fewer, the 16 waves' loads in
+// flight win earlier.  us on MI355X, short / long block, rows x values:
+//   argmax       1 x 1000 2.2 / 2.2    1 x 2048 2.3 / 2.2    2000 x 1000 3.3 / 7.7   2000 x 8192 11.2 / 13.9
+//   log-softmax  1 x 4096 5.5 / 5.6    1 x 6000 6.4 / 5.8    600 x 8192 8.9 / 12.9   2000 x 1000 7.2 / 25.1
+constexpr int kRowFew = 256;  // one row per CU
+constexpr int kRowShort = 8192, kRowShortArgmax = 1024, kRowShortLogsoftmax = 4096;
+constexpr bool row_short_argmax(int M, int n) { return n <= (M > kRowFew ? kRowShort : kRowShortArgmax); }
+constexpr bool row_short_logsoftmax(int M, int n) { return n <= (M > kRowFew ? kRowShort : kRowShortLogsoftmax); }
+constexpr int kRowShortThreads = 256;
+
+// quad(i) for each whole four values of a short row that fall to thread tid (i
+// their first index), then one(i) for at most one of the last n % 4.
+template <class Quad, class One>
+constexpr void row_quads(int n, int tid, const Quad& quad, const One& one) {
+#pragma unroll 4
+    for (int i = 4 * tid; i < (n & ~3); i += 4 * kRowShortThreads) quad(i);
+    if (tid < (n & 3)) one((n & ~3) + tid);
+}
+
 // f(i) for thread tid's values of the partial last segment [i0, n), spread over
 // all of the block's threads: at most one each for a block of kRowThreads, so
 // the segment costs one memory latency (one wave alone takes up to 16, which is

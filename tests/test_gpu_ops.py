@@ -533,7 +533,7 @@ def test_sample_dev_rows(backend, oracle):
         assert (int(tok[m]), int(ns[m])) == oracle.sample_integer_cdf(z[m], int(states[m])), m
 
 
-@pytest.mark.parametrize("n", [1, 255, 1023, 1024, 1025, 16384, 16385, 33793, 1 << 20, (1 << 20) + 1, (1 << 21) + 4097])
+@pytest.mark.parametrize("n", [1, 3, 255, 1023, 1024, 1025, 16384, 16385, 33793, 1 << 20, (1 << 20) + 1, (1 << 21) + 4097])
 def test_row_choice_edges(backend, oracle, n):
     """argmax and the sampler at the edges of their row walk (1024 values per
     wave segment, 16 waves, two segments in flight; past 2^20 values the
@@ -558,6 +558,34 @@ def test_row_choice_edges(backend, oracle, n):
         for m in range(M):
             want = oracle.sample_integer_cdf(np.ascontiguousarray(z[m]), state)
             assert (int(tok[m]), int(ns.view(np.uint64)[m])) == want, (n, m, state)
+
+
+@pytest.mark.parametrize("M,n", [(257, 1), (257, 6), (300, 1027), (300, 8191), (300, 8192), (300, 8193), (4, 4096), (4, 4097)])
+def test_many_short_rows(backend, oracle, M, n):
+    """argmax and the log-softmax at the edges of the small blocks (more than 256
+    rows of up to 8192 values; few rows of up to 1024 and 4096), rows at odd
+    addresses: ties, a first and a last maximum, the least value, values past the
+    table's LDS part; against the oracle."""
+    import torch
+    from myelith_amd.luts import exp_lut
+    case(f"short rows M={M} n={n}")
+    r = rng(M + n)
+    ld = n + 1
+    buf = r.integers(-700, 700, M * ld + 1).astype(np.int32)
+    z = np.lib.stride_tricks.as_strided(buf[1:], (M, n), (4 * ld, 4))
+    z[0, n // 2:] = 699
+    z[1, n - 1] = 2**31 - 1
+    z[2] = -2**31
+    z[3, 0] = 9000
+    z[4:: 7] *= 9
+    zd = torch.as_strided(torch.from_numpy(buf).cuda(), (M, n), (ld, 1), 1)
+    rows = [np.ascontiguousarray(v) for v in z]
+    assert list(backend.argmax_dev(zd).cpu().numpy()) == [oracle.argmax_int(v) for v in rows]
+    t = r.integers(-1, n, M).astype(np.int64)
+    t[:4] = [0, n - 1, n // 2, 0]
+    for lut in (exp_lut(), r.integers(-300, 300, 40001).astype(np.int16), exp_lut()[:5]):
+        got = backend.logsoftmax_dev(zd, lut, t).cpu().numpy()
+        assert list(got) == [oracle.logsoftmax_at(v, lut, int(k)) if k >= 0 else 0 for v, k in zip(rows, t)]
 
 
 def test_device_forms_batch_rows(backend, oracle, luts64):

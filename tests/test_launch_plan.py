@@ -226,7 +226,10 @@ int main() {
     long checked = 0, bad = 0;
     // partial last segments and strided passes: every index once, ascending per
     // thread, none outside the row, up to the longest row an entry point takes
-    for (int64_t n64 : {1ll, 63ll, 64ll, 65ll, 1023ll, 1025ll, 5000ll, INT_MAX - 2000ll, INT_MAX - 1023ll, INT_MAX - 64ll,
+    // many short rows take small blocks, few or long ones blocks of 16 waves
+    bad += !row_short_argmax(2000, 1000) || !row_short_logsoftmax(2000, 64) || !row_short_argmax(1, 1000);
+    bad += row_short_argmax(1, 152064) || row_short_logsoftmax(600, 152064) || row_short_logsoftmax(24, 8192);
+    for (int64_t n64 : {1ll, 3ll, 63ll, 64ll, 65ll, 1023ll, 1025ll, 5000ll, 8191ll, 8192ll, INT_MAX - 2000ll, INT_MAX - 1023ll, INT_MAX - 64ll,
                         INT_MAX - 63ll, INT_MAX - 1ll, (long long)INT_MAX}) {
         const int n = (int)n64, i0 = n / kRowSeg * kRowSeg;
         for (int threads : {kRowThreads, 256}) {
@@ -241,6 +244,15 @@ int main() {
                 bad += took > kRowSeg / threads;  // the segment is shared by the whole block
             }
             for (int v : got) bad += v != 1;
+        }
+        if (n <= kRowShort) {  // the walk of a short row
+            std::vector<int> seen(n, 0);
+            for (int tid = 0; tid < kRowShortThreads; ++tid) {
+                int last = -1;
+                auto take = [&](int i) { ++checked, bad += i <= last || i < 0 || i >= n || seen[i]++, last = i; };
+                row_quads(n, tid, [&](int i) { for (int e = 0; e < 4; ++e) take(i + e); }, take);
+            }
+            for (int v : seen) bad += v != 1;
         }
         for (int tid : {0, 1, 511, kRowThreads - 1}) {
             int64_t want = tid, bad0 = bad;
