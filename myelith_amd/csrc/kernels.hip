@@ -929,8 +929,64 @@ __global__ __launch_bounds__(kRowThreads) void sample_cdf_kernel(const int32_t* 
     if (tid == 0) tokens[blockIdx.x] = pick;
 }
 
+// The same for rows of at most kRowShortThreads x EACH values, which stay in registers: one
+// read, one scan over the block (wrapped weights included).  With the groups, a
+// short row is mostly their two wave scans one after the other and the 16 waves'
+// segment sums.  24 rows of 1000 / 4096 values: 5.0 / 6.8 us, 8.1 / 8.2 with the
+// groups; 2000 rows of 1000: 11.6 and 20.6 (16 waves of four values a lane took
+// 40 at 2000 x 2048: all of them work out the threshold's remainder).
+template <int EACH>
+__global__ __launch_bounds__(kRowShortThreads) void sample_short_kernel(const int32_t* __restrict__ z, int n, int ldz,
+                                                                       const uint64_t* __restrict__ states,
+                                                                       int64_t* __restrict__ tokens,
+                                                                       uint64_t* __restrict__ new_states) {
+    __shared__ int32_t redm[kRowShortThreads / 64], redc[kRowShortThreads / 64];
+    __shared__ int64_t wt[kRowShortThreads / 64];
+    const int32_t* row = z + (size_t)blockIdx.x * ldz;
+    const int tid = threadIdx.x, i0 = EACH * tid;
+    uint64_t state = states[blockIdx.x];
+    int32_t v[EACH], nm = INT32_MIN;
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) v[e] = row[min(i0 + e, n - 1)];  // past the row: the last value again
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) nm = max(nm, ~v[e]);
+    const int32_t m = ~block_max_i32_dpp(nm, redm);
+    int64_t w[EACH], loc = 0;
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) {
+        w[e] = i0 + e < n ? (int64_t)(int32_t)((uint32_t)v[e] - (uint32_t)m + 1u) : 0;
+        loc += w[e];
+    }
+    int64_t total = 0;
+    int64_t acc = block_scan_i64(loc, wt, total);
+    if (total <= 0) {  // uniform: a non-positive total keeps the state
+        if (tid == 0) {
+            tokens[blockIdx.x] = 0;
+            new_states[blockIdx.x] = state;
+        }
+        return;
+    }
+    const int64_t thr = (int64_t)umod64(splitmix64_next(state), (uint64_t)total);
+    int cand = INT32_MAX;
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) {
+        acc += w[e];
+        if (i0 + e < n && thr < acc && cand == INT32_MAX) cand = i0 + e;
+    }
+    const int first = ~block_max_i32_dpp(~cand, redc);
+    if (tid == 0) {
+        tokens[blockIdx.x] = first == INT32_MAX ? n - 1 : first;
+        new_states[blockIdx.x] = state;
+    }
+}
+
 hipError_t sample_cdf(const int32_t* z, int M, int n, int ldz, const uint64_t* states, int64_t* tokens,
                       uint64_t* new_states, hipStream_t st) {
+    if (n <= kRowShortThreads * 16) {
+        if (n <= kRowShortThreads * 4) sample_short_kernel<4><<<M, kRowShortThreads, 0, st>>>(z, n, ldz, states, tokens, new_states);
+        else sample_short_kernel<16><<<M, kRowShortThreads, 0, st>>>(z, n, ldz, states, tokens, new_states);
+        return hipGetLastError();
+    }
     // 2^lg segments per group, so that the row's groups fit the block's LDS sums
     int lg = 0;
     while (((int64_t)kSampleGroups * kRowSeg << lg) < n) ++lg;
