@@ -548,14 +548,18 @@ __global__ __launch_bounds__(SHORT ? kRowShortThreads : kRowThreads) void argmax
 // second pass had an LDS table lookup), with the maximum and the least value
 // counted.  Values kLogBins (128 logit units) or more below the largest of
 // 1024 sampled ones are past the table whatever the maximum is and are not
-// counted (masked tokens, say), and a segment of equal values is one add.
+// counted (masked tokens, say); a value that fills a segment, or half of it, is
+// counted in registers.
 // When the counted values lie less than kLogBins apart every counter stands
 // for one value and S = sum over k of count[m - k] * lut[k << 2]; other rows,
 // and tables longer than the ring, sum the table over a second pass.
 // 600 x 152064 values in 80 us (4.6 TB/s); two passes of 256 threads took 385.
-// Constant rows, rows wider than the ring and half-masked rows take 76, 150 and
-// 83 us (186, 200 and 293 before).
+// Constant rows, rows wider than the ring, rows half masked with the least value
+// and rows with all but 1% at one value in the ring take 78,
+// 140, 83 and 92 us (189, 188, 346 and 193 with two passes; the last 402 with an add
+// per value).
 constexpr int kLogBins = 8192;
+constexpr int kLogSame = 32;  // lanes of a wave with one value from which it is counted in registers
 
 // One value's term of S, `below` under the maximum; the result from S.
 __device__ inline int64_t logsoftmax_term(uint64_t below, const int16_t* lut, uint32_t lut_len) {
@@ -593,11 +597,36 @@ __global__ __launch_bounds__(kRowThreads) void logsoftmax_kernel(const int32_t* 
                     smax = max(smax, v[q][e]);
                 }
             mx = max(mx, smax);
-            const int32_t first = __builtin_amdgcn_readfirstlane(smin);
-            if (__all(smin == first && smax == first)) {
-                if (first < least) return;
-                nm = max(nm, ~first);
-                if ((tid & 63) == 0) atomicAdd(&count[(uint32_t)first % kLogBins], (uint32_t)kRowSeg);
+            // A value that many lanes hold is counted in registers, and a second
+            // one with it: the lanes' adds to one counter come one after another.
+            const int32_t some = __builtin_amdgcn_readfirstlane(v[0][0]), low = __builtin_amdgcn_readfirstlane(smin),
+                          high = __builtin_amdgcn_readfirstlane(smax);
+            auto many = [&](int32_t x, int32_t y) {
+                return (int)(y >= least) & (int)(__builtin_popcountll(__ballot(x == y)) >= kLogSame);
+            };
+            const int many_some = many(v[0][0], some), many_low = many(smin, low), many_high = many(smax, high);
+            if (many_some | many_low | many_high) {  // uniform
+                if (__all(smin == smax && smin == some)) {
+                    nm = max(nm, ~some);
+                    if ((tid & 63) == 0) atomicAdd(&count[(uint32_t)some % kLogBins], (uint32_t)kRowSeg);
+                    return;
+                }
+                const int32_t a = many_some ? some : many_low ? low : high, b = high != a ? high : low;
+                int32_t c = 0;  // of a | of b << 16
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const int32_t x = v[q][e];
+                        nm = x >= least ? max(nm, ~x) : nm;
+                        c += x == a ? 1 : (x == b ? 0x10000 : 0);
+                        if (x != a && x != b && x >= least) atomicAdd(&count[(uint32_t)x % kLogBins], 1u);
+                    }
+                c = wave_sum_i32(c);
+                if ((tid & 63) == 0) {
+                    atomicAdd(&count[(uint32_t)a % kLogBins], (uint32_t)c & 0xFFFFu);
+                    if (b >= least) atomicAdd(&count[(uint32_t)b % kLogBins], (uint32_t)c >> 16);
+                }
                 return;
             }
             if (__all(smin >= least)) {

@@ -371,7 +371,7 @@ def test_logsoftmax_dev(backend, oracle):
 
 
 @pytest.mark.parametrize("n", [1, 1023, 1025, 4096, 4097, 16385, 40003])
-@pytest.mark.parametrize("spread", [0, 700, 8191, 8192, 2**31])
+@pytest.mark.parametrize("spread", [0, 1, 2, 3, 700, 8191, 8192, 2**31])
 def test_logsoftmax_row_spreads(backend, oracle, n, spread):
     """The counted pass (maximum - minimum below 8192) up to its edge and the
     second pass beyond it, at the edges of the row walk, rows at odd addresses;
