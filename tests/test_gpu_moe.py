@@ -73,6 +73,24 @@ def test_small_moe_around_the_stream(backend, T, widths):
     assert np.array_equal(gm.forward(x).cpu().numpy(), y)
 
 
+@pytest.mark.parametrize("T,S", [(70, 5632), (131, 5632), (203, 5632), (515, 5632), (90, 18944)])
+def test_moe_shared_expert_tiles(backend, T, S):
+    """The shared expert's fused gate/up product on its tiles of more than 64 rows:
+    128 x 128 of three stages, 64 x 128, 128 x 128 of two, 256 x 256 and 192 x 256
+    (the CPU plan test holds which shape takes which), ragged token counts."""
+    from myelith_amd.moe import moe_spec
+    spec = moe_spec(13, hidden=128, n_experts=4, inter=128, top_k=2, shared_inter=S)
+    case(f"moe shared expert T={T} S={S}")
+    gm, om = build(backend, spec, np.arange(4) * -60)
+    x = gm.synth_input(T)
+    xh = x.cpu().numpy()
+    y = gm.forward(x).cpu().numpy()
+    ro = om.route(xh)
+    compare_route(gm.route(T), ro)
+    for t in range(T):
+        assert np.array_equal(y[t], om.token(xh[t], ro["ids"][t], ro["gates"][t])), t
+
+
 def test_qwen15_moe_4096_tokens(backend):
     """The Qwen1.5-MoE-A2.7B-shaped layer on 4096 tokens: the whole route
     (ids, gates, counts, offsets, dispatch order) and the output of every

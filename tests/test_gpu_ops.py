@@ -271,11 +271,12 @@ def test_few_row_int16_weight_stream(backend, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(65, 300, 128), (129, 70, 8320), (450, 3580, 128), (1500, 3583, 128), (1501, 4599, 256),
-                                   (33, 40, 256), (100, 40, 4864), (1000, 18944, 128)])
+                                   (33, 40, 256), (100, 40, 4864), (1000, 18944, 128), (131, 11263, 128), (203, 11263, 128)])
 def test_wide_tiles_and_requant_columns(backend, oracle, M, N, K):
-    """The tiles of more than 32 rows (64 x 64, 64 x 128, the same split over K,
-    128 x 128, 192 x 256, 256 x 256; ragged rows and columns), with shifts in and out of
-    the range of the 32-bit requantization mixed over the columns (blocks of
+    """The tiles of more than 32 rows (64 x 64, 64 x 128 whole and split over K,
+    128 x 128 of two and of three stages, 192 x 256, 256 x 256; ragged rows and
+    columns; the CPU plan test holds which shape takes which), with shifts in and
+    out of the range of the 32-bit requantization mixed over the columns (blocks of
     columns inside it, so that both forms run), full-range activations
     and weights, against the oracle's requant of the exact sums."""
     import torch
@@ -294,10 +295,12 @@ def test_wide_tiles_and_requant_columns(backend, oracle, M, N, K):
         assert np.array_equal(got, oracle.requant_shift(acc, ws, 10, 10)), (lo, hi)
     mult = r.integers(-(1 << 31), 1 << 31, N).astype(np.int32)
     mult[:5] = [0, -1, 1 << 30, -(1 << 31), (1 << 31) - 1]
-    sh = r.integers(20, 80, N).astype(np.uint8)
-    sh[: N // 2] = r.integers(39, 60, N // 2)
-    got = backend.linear_w8a16_mult_dev(x, W, torch.from_numpy(mult).cuda(), torch.from_numpy(sh).cuda()).cpu().numpy()
-    assert np.array_equal(got, oracle.requant_mult(acc, mult, sh))
+    for lo, hi, lo2, hi2 in ((20, 80, 39, 60), (0, 100, 9, 71)):  # the second half of the columns, the first
+        sh = r.integers(lo, hi, N).astype(np.uint8)
+        sh[: N // 2] = r.integers(lo2, hi2, N // 2)
+        got = backend.linear_w8a16_mult_dev(x, W, torch.from_numpy(mult).cuda(), torch.from_numpy(sh).cuda()).cpu().numpy()
+        assert np.array_equal(got, oracle.requant_mult(acc, mult, sh)), (lo, hi)
+        mult[N // 4:] >>= 20  # results inside the clamp at the small shifts too
 
 
 @pytest.mark.parametrize("M", [64, 512])

@@ -175,6 +175,20 @@ int main() {
             }
     CHECK(moe_work_items(64, 60, moe_pick_tile(true, 64, 60), 1408, 2048) >
               moe_work_items(16384, 60, moe_pick_tile(true, 16384, 60), 1408, 2048), "small tiles need more items");
+    // the tiles that the GPU tests of the products of more than 32 rows mean to run
+    // (acc: room for partial sums, none in the gate/up product with the SiLU gate)
+    struct Want { int M, N, K; bool acc; Mm2Tile tile; bool split; };
+    for (const Want& w : {Want{65, 300, 128, true, kMm2T64s3, false}, Want{33, 40, 256, true, kMm2T64s3, false},
+                          Want{129, 70, 8320, true, kMm2T64, true}, Want{100, 40, 4864, true, kMm2T64, true},
+                          Want{131, 11263, 128, true, kMm2T64, false}, Want{203, 11263, 128, true, kMm2T128, false},
+                          Want{450, 3580, 128, true, kMm2T128s3, false}, Want{1500, 3583, 128, true, kMm2T192, false},
+                          Want{1501, 4599, 256, true, kMm2T256, false}, Want{1000, 18944, 128, true, kMm2T256, false},
+                          Want{70, 11264, 128, false, kMm2T128s3, false}, Want{131, 11264, 128, false, kMm2T64, false},
+                          Want{203, 11264, 128, false, kMm2T128, false}, Want{515, 11264, 128, false, kMm2T256, false},
+                          Want{90, 37888, 128, false, kMm2T192, false}}) {
+        const Mm2Pick p = mm2_pick(w.M, w.N, w.K, 256, w.acc ? (size_t)4 << 20 : 0);
+        CHECK(p.tile == w.tile && p.split == w.split, "tile of %d x %d x %d: %d %d", w.M, w.N, w.K, (int)p.tile, (int)p.split);
+    }
     // groups of the tile order: the full ones and the last cover the row tiles
     for (int tiles = 1; tiles < 300; ++tiles)
         for (int want = 0; want < 9; ++want) {
