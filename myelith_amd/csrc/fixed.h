@@ -133,6 +133,12 @@ struct PlaneMult {
     // clamp_i16 of the result
     MYL_MEM int16_t clamped(int32_t u, uint32_t r) const { return clamp_i16_i64(wide(u, r)); }
 };
+// The same where the shift is at least kPlaneMultNarrow: the low word is the result.
+constexpr uint32_t kPlaneMultNarrow = 39;
+struct PlaneMultNarrow {
+    PlaneMult c;
+    MYL_MEM int16_t clamped(int32_t u, uint32_t r) const { return clamp_i16(c(u, r)); }
+};
 
 // rescale64 of a value |v| <= 2^30 followed by a clamp to [-2^16, 2^16] or
 // narrower, for left shifts of up to 14 and right shifts of up to 30.

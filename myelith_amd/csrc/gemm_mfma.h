@@ -395,7 +395,8 @@ struct SinkEpi {
     __device__ inline void put64(int n, int m, int64_t v, const Ops& o) const { e.one_ops(n, m, v, o); }
     __device__ inline Elt elt(size_t i, uint32_t lo) const { return e.elt(i, lo); }
     __device__ inline size_t idx(int n, int m) const { return e.idx(n, m); }
-    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt& x) const { e.put(i, lo, u, r, c, x); }
+    template <class C>
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const C& c, const Elt& x) const { e.put(i, lo, u, r, c, x); }
 };
 struct SinkAtomic {
     unsigned long long* acc;

@@ -382,7 +382,8 @@ struct EpiMult {
     using Elt = EpiNoElt;
     __device__ inline Elt elt(size_t, uint32_t) const { return Elt{}; }
     __device__ inline size_t idx(int n, int m) const { return (size_t)m * ldo + n; }
-    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const Col& c, const Elt&) const {
+    template <class C>  // PlaneMult or PlaneMultNarrow
+    __device__ inline void put(size_t i, uint32_t lo, int32_t u, uint32_t r, const C& c, const Elt&) const {
         (out + i)[lo] = c.clamped(u, r);
     }
     template <int R, int MT>

@@ -381,11 +381,22 @@ int main() {
             const int32_t l32 = (int32_t)low;
             ++n, ++fast;
             bad += p.clamped((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u) != mult_general(hi * 256 + low, mult, (uint8_t)s);
+            if (s >= (int)kPlaneMultNarrow)
+                bad += PlaneMultNarrow{p}.clamped((int32_t)hi + (l32 >> 8), (uint32_t)l32 & 255u) != mult_general(hi * 256 + low, mult, (uint8_t)s);
             // sums of a few units times small multipliers: results inside the clamp at the small shifts
             const int64_t sum = (int64_t)(next() % (1u << (k % 20 + 1))) - (1 << (k % 20)), sm_ = mult >> (31 - k % 24);
             const PlaneMult q = PlaneMult::of((int32_t)sm_, (uint8_t)s);
             ++n;
             bad += q.clamped((int32_t)(sum >> 8), (uint32_t)sum & 255u) != mult_general(sum, (int32_t)sm_, (uint8_t)s);
+            if (mult) {  // products around the clamp
+                const myl_i128 edge = (myl_i128)1 << (s + 14 + k % 3 < 69 ? s + 14 + k % 3 : 68);
+                int64_t x = (int64_t)(edge / mult) + (int64_t)(next() % 65) - 32;
+                if (k & 4) x = -x;
+                if (x < ((int64_t)1 << 38) && x > -((int64_t)1 << 38)) {
+                    ++n;
+                    bad += p.clamped((int32_t)(x >> 8), (uint32_t)x & 255u) != mult_general(x, mult, (uint8_t)s);
+                }
+            }
         }
     printf("checked %ld (plane sums %ld), mismatches %ld\n", n, fast, bad);
     return bad != 0 || fast < 100000;
