@@ -660,9 +660,11 @@ hipError_t forward_rows(myl_model* m, BatchState* b, int R, int lmax, int h0, in
     const bool planes = mm_planes_ok(R, H, mm) && mm_planes_ok(R, I, mm) && mm_planes_ok(R, nq, mm) &&
                         rmsnorm_planes_ok(H) && xvec_ok(b->X, H);
     // the gate/up product applies the SiLU and writes the down product's
-    // planes itself (staged epilogue) when its tiles need no K split
-    // (17-64 rows: the split gate/up product with its own finish and SiLU
-    // measured faster on MI355X than the unsplit fused one)
+    // planes itself where its sums are whole: past 64 rows in the tiles' staged
+    // epilogue, up to 16 rows in that of the small tiles, on fragment-major
+    // weights, and for 2-32 rows over short K (0.5B: 896) in the weight stream.
+    // Elsewhere at 17-64 rows the split gate/up product with its own finish and
+    // SiLU measured faster on MI355X than the unsplit fused one.
     const bool frag = planes && frag_ready(m, R, mm, st);
     const bool fuse_silu = planes && I % 8 == 0 &&
                            (R > 64 || (R <= 16 && H % 128 == 0) || frag ||

@@ -15,10 +15,11 @@
 // rows of A' and BN = 32*NB*WN weight rows; K advances KS = 64 or 128 bytes
 // per stage through STAGES LDS buffers filled by direct global-to-LDS loads
 // (global_load_lds_dwordx4: each wave instruction writes 1 KiB = 1024/KS rows
-// x KS bytes), issued STAGES-1 stages ahead and awaited with an explicit
-// vmcnt.  128-byte stages read whole cache lines of every row per load
-// instruction and halve the barriers per K; they pay off for grids of many
-// large tiles.  The KS/16 chunks of LDS row r sit at slot
+// x KS bytes): all STAGES buffers are filled before the loop, each is refilled
+// as soon as the barrier that frees it is past, and a stage is awaited with an
+// explicit vmcnt.  128-byte stages read whole cache lines of every row per load
+// instruction and halve the barriers per K; 64-byte ones are kept for a K that
+// is no multiple of 128.  The KS/16 chunks of LDS row r sit at slot
 // chunk ^ ((r / (256/KS)) % (KS/16)), so the 16-byte fragment reads of 16
 // consecutive rows cover all 64 banks once.  K must be a multiple of KS; rows
 // past the matrix clamp to its last row (their outputs are discarded), so
@@ -263,9 +264,8 @@ __device__ inline void mm2_emit64(const v16i32_t (&acc)[MB][NB], const int32_t (
 }
 
 // A multiplier sink whose columns' results fit 32 bits before their clamp: a wave
-// of such columns skips the 64-bit clamp (4001 x 18944 x 3584: 576 us,
-// 583 where the ragged last row tiles alone kept it, 595 and 586 with and without it
-// in another run).
+// of such columns skips the 64-bit clamp (4001 x 18944 x 3584, shifts 41-43: 586 us,
+// 595 with it; in another run 576, and 583 with it in the ragged last tiles alone).
 template <class Sink>
 struct SinkNarrow {
     const Sink& s;
