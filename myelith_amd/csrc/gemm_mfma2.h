@@ -356,8 +356,12 @@ __device__ inline void mm2_staged_tile(const int8_t* __restrict__ Ap, int R2, co
         for (uint32_t o = (uint32_t)wave * 1024u; o < lut_bytes; o += S::kThreads * 16u)
             __builtin_amdgcn_global_load_lds((const void*)(reinterpret_cast<const int8_t*>(sink.silu_table()) + o + lane * 16),
                                              (lds_void*)(lut_l + o), 16, 0, 0);
-    // rows and columns past the matrix hold sums of clamped operands; they are
-    // staged like the others and never emitted
+    // rows and columns past the matrix hold sums of clamped operands; in the
+    // accumulator tiles that reach into it they are staged like the others and
+    // never emitted.  Columns outside the 32-bit range (a hidden size of 448: shifts
+    // of 8) take 64-bit sums; with their operand loaded again for each value and
+    // every tile staged, one token of a 448-wide expert layer took 13.8 us here,
+    // 9.4 before the 32-bit steps.
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
         rs[j] += __shfl_xor(rs[j], 32);
@@ -366,19 +370,25 @@ __device__ inline void mm2_staged_tile(const int8_t* __restrict__ Ap, int R2, co
         const bool fast = K < kPlaneSumK && __all((int)col.fast);
         const int32_t rs128 = (int32_t)((uint32_t)rs[j] << 7);
         int16_t* tj = tile + (wm * MB * 16 + 2 * (lane >> 5)) * S::BN + nl;
+        if (fast) {
 #pragma unroll
-        for (int i = 0; i < MB; ++i) {
-            if (fast) {
+            for (int i = 0; i < MB; ++i) {
+                if (r0 + (wm * MB + i) * 32 >= R2) break;  // uniform
 #pragma unroll
                 for (int r = 0; r < 16; r += 2) {
                     const int32_t low = acc[i][j][r + 1] + rs128;
                     tj[((i * 32 + mm2_row(r)) >> 1) * S::BN] = sink.stage(col, acc[i][j][r] + (low >> 8), (uint32_t)low & 255u);
                 }
-            } else {
-#pragma unroll 1
+            }
+        } else {
+            const auto op = sink.op(n);
+#pragma unroll
+            for (int i = 0; i < MB; ++i) {
+                if (r0 + (wm * MB + i) * 32 >= R2) break;
+#pragma unroll 2
                 for (int r = 0; r < 16; r += 2)
                     tj[((i * 32 + mm2_row(r)) >> 1) * S::BN] =
-                        sink.stage64(n, (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128);
+                        sink.stage64(op, n, (int64_t)acc[i][j][r] * 256 + (int64_t)acc[i][j][r + 1] + (int64_t)rs[j] * 128);
             }
         }
     }
@@ -620,7 +630,9 @@ struct SinkGroupedStaged {
     using Col = typename EpiG::Col;
     __device__ inline Col col(int n) const { return epi.col(e, n); }
     __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return epi.stage(c, u, r); }
-    __device__ inline int16_t stage64(int n, int64_t v) const { return epi.stage64(e, n, v); }
+    __device__ inline auto op(int n) const { return epi.op(e, n); }
+    template <class Op>
+    __device__ inline int16_t stage64(const Op& o, int n, int64_t v) const { return epi.stage64(o, n, v); }
     __device__ inline const int16_t* silu_table() const { return epi.silu; }
     __device__ inline uint32_t silu_table_len() const { return epi.silu_len; }
     __device__ inline void emit(int m, int i0, const uint4& a, const uint4& b, const int16_t* lut) const {

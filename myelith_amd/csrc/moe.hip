@@ -395,9 +395,9 @@ struct EpiExpertGUSiluPlanes {
         return Col::of((uint8_t)(shifts[(size_t)e * n2 + n] + MYL_MOE_X_FRAC), (n & 1) ? MYL_MOE_UP_FRAC : MYL_MOE_GATE_FRAC);
     }
     __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return clamp_i16(c(u, r)); }
-    __device__ inline int16_t stage64(int e, int n, int64_t acc) const {
-        const uint8_t frac = (n & 1) ? MYL_MOE_UP_FRAC : MYL_MOE_GATE_FRAC;
-        return clamp_i16_i64(rescale64(acc, (uint8_t)(shifts[(size_t)e * n2 + n] + MYL_MOE_X_FRAC), frac));
+    __device__ inline uint8_t op(int e, int n) const { return shifts[(size_t)e * n2 + n]; }
+    __device__ inline int16_t stage64(uint8_t sh, int n, int64_t acc) const {
+        return clamp_i16_i64(rescale64(acc, (uint8_t)(sh + MYL_MOE_X_FRAC), (n & 1) ? MYL_MOE_UP_FRAC : MYL_MOE_GATE_FRAC));
     }
     __device__ inline void emit(int, int row, int i0, const uint4& a, const uint4& b, const int16_t* lut) const {
         const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};  // (g, u) pairs

@@ -187,13 +187,13 @@ struct EpiGUSiluPlanes {
         return Col::of((uint8_t)(shifts[n] + act_frac), (n & 1) ? up_frac : gate_frac);
     }
     __device__ inline int16_t stage(const Col& c, int32_t u, uint32_t r) const { return clamp_i16(c(u, r)); }
-    __device__ inline int16_t stage64(int n, int64_t acc) const { return stage_with(op(n), n, acc); }
     // in two steps: the row's operand, fetched ahead of the sum
     using Op = uint8_t;
     __device__ inline Op op(int n) const { return shifts[n]; }
     __device__ inline int16_t stage_with(Op sh, int n, int64_t acc) const {
         return clamp_i16_i64(rescale64(acc, (uint8_t)(sh + act_frac), (n & 1) ? up_frac : gate_frac));
     }
+    __device__ inline int16_t stage64(Op sh, int n, int64_t acc) const { return stage_with(sh, n, acc); }
     __device__ inline void emit_one(int m, int i, int16_t g, int16_t u) const {
         const int32_t h = silu_mul(g, u, silu, silu_len, gate_frac, up_frac, down_in_frac);
         planes[(size_t)(2 * m) * I + i] = (int8_t)(h >> 8);
